@@ -181,7 +181,8 @@ int vxg_graph_stats(vxg_sim* s, int* captures, int* replays);
    block-to-XCD mapping of kernel 0 = fused mixed step, 1 = FP64 link kernel, 2 = FP64 voxel
    kernel, 3 = fused FP64 step are chosen by timing each candidate on the first 24 steps of every model size;
    results do not depend on the choice.  vxg_launch_config reports it (settled = 1 once
-   chosen). */
+   chosen).  A model small enough for the form of a step kernel that splits link directions over
+   waves runs that form from its first step, with nothing to choose (settled = 1). */
 int vxg_autotune(vxg_sim* s, int enable);
 int vxg_launch_config(vxg_sim* s, int kernel, int* block, int* xcd_mapping, int* settled);
 /* Pins kernel's launch configuration (block 64/128/256, xcd_mapping 0/1) as if the autotuner

@@ -257,7 +257,7 @@ API int vxg_set_launch_config(vxg_sim* h, int kernel, int block, int xcd) {
     Sim::Tuner& t = s->tuner[kernel];
     t.reset(s->nv());
     t.chosen = vx::LaunchCfg{block, xcd};
-    t.settled = true;
+    t.settled = t.pinned = true;
     return 1;
 }
 API int vxg_profile_read(vxg_sim* h, double* ms, int* launches, int cap) {

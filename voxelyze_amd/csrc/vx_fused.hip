@@ -68,57 +68,86 @@ __device__ __forceinline__ double axis_size(const VoxMat& m, int axis) {
     return axis == 0 ? m.sizeX : axis == 1 ? m.sizeY : m.sizeZ;
 }
 
-/* one link of voxel i (direction dir, neighbour o) as CVX_Link::updateForces
-   (VX_Link.cpp:149-217): its end vector on voxel i added to the direction-ordered sums,
-   written to the force slot on the last step; the negative end (Neg) owns the link state.
-   Poisson: some material has Poisson's ratio != 0 (the transverse info is read and kept) */
-template <bool ForcesOnly, bool Neg, bool Poisson>
-__device__ __forceinline__ void link_end(const FusedPtrs& s, int i, int o, int dir, int rob, float prevDt, float tnow,
-                                         float tempI, const dvec& pos0, const dquat& q0, dvec& sf, dvec& sm) {
+/* the step's output link state: past the caches, or through them where the next step's reads of
+   the same workgroup find it there (a model whose state the L2s hold) */
+template <bool Cached, class T>
+__device__ __forceinline__ void put(T* p, T v) {
+    if (Cached) *p = v;
+    else st_nt(p, v);
+}
+
+/* what one end of a link reads: the neighbour's pose and material, the link's material and state */
+struct LinkIn {
+    int meta, mo;
+    dvec po;
+    dquat qo;
+    double rest;
+    LinkPrev old;
+};
+/* the loads of one link of voxel i (direction dir, neighbour o), those that wait for nothing but
+   the slot first */
+template <bool Neg, bool Poisson>
+__device__ __forceinline__ void link_load(const FusedPtrs& s, int i, int o, int dir, LinkIn& in) {
     const int nv = s.nv, nl = s.nl;
     const double* __restrict__ vd = s.vdIn;
+    const int slot = (dir >> 1) * nv + (Neg ? i : o);
+    in.meta = s.lmeta[slot];
+    in.old.flags = s.lflIn[slot];
+    in.old.pos2 = dv(s.ldIn[LP2X * nl + slot], s.ldIn[LP2Y * nl + slot], s.ldIn[LP2Z * nl + slot]);
+    in.old.a1 = dv(s.ldIn[LA1X * nl + slot], s.ldIn[LA1Y * nl + slot], s.ldIn[LA1Z * nl + slot]);
+    in.old.a2 = dv(s.ldIn[LA2X * nl + slot], s.ldIn[LA2Y * nl + slot], s.ldIn[LA2Z * nl + slot]);
+    in.old.maxStrain = s.lfIn[LMAXSTRAIN * nl + slot];
+    in.old.strainOffset = s.lfIn[LOFFSET * nl + slot];
+    if (Poisson) {
+        in.old.tArea = s.lfIn[LTAREA * nl + slot];
+        in.old.tss = s.lfIn[LTSS * nl + slot];
+    }
+    in.rest = s.ldIn[LREST * nl + slot];
+    in.mo = s.vmat[o];
+    in.po = dv(vd[VPX * nv + o], vd[VPY * nv + o], vd[VPZ * nv + o]);
+    in.qo = dq(vd[VQW * nv + o], vd[VQX * nv + o], vd[VQY * nv + o], vd[VQZ * nv + o]);
+}
+
+/* one link of voxel i (direction dir, neighbour o, material mi) as CVX_Link::updateForces
+   (VX_Link.cpp:149-217): its end vectors on voxel i (force f, moment mm), written to the force
+   slot on the last step; the negative end (Neg) owns the link state.
+   Poisson: some material has Poisson's ratio != 0 (the transverse info is read and kept) */
+template <bool ForcesOnly, bool Neg, bool Poisson, bool Cached>
+__device__ __forceinline__ void link_end(const FusedPtrs& s, LinkIn& in, int i, int o, int mi, int dir, int rob,
+                                         float prevDt, float tnow, float tempI, const dvec& pos0, const dquat& q0,
+                                         dvec& f, dvec& mm) {
+    const int nv = s.nv, nl = s.nl;
     const int axis = dir >> 1;
     const int n = Neg ? i : o, p = Neg ? o : i;
     const int slot = axis * nv + n;
-    const LinkMat m = s.lmats[s.lmeta[slot]];
-    const dvec po = dv(vd[VPX * nv + o], vd[VPY * nv + o], vd[VPZ * nv + o]);
-    const dquat qo = dq(vd[VQW * nv + o], vd[VQX * nv + o], vd[VQY * nv + o], vd[VQZ * nv + o]);
-    double rest;
+    const LinkMat m = s.lmats[in.meta];
+    const VoxMat& mn = s.vmats[Neg ? mi : in.mo];
+    const VoxMat& mp = s.vmats[Neg ? in.mo : mi];
+    const dvec po = in.po;
+    const dquat qo = in.qo;
+    double rest = in.rest;
     if (s.vphase) { /* updateRestLength (VX_Link.cpp:137-140) at this step's temperatures */
         const float tempO = actuation_temperature(s.actBase, s.actAmp, s.actFreq, tnow, s.vphase[o]);
-        const VoxMat& mn = s.vmats[s.vmat[n]];
-        const VoxMat& mp = s.vmats[s.vmat[p]];
         rest = 0.5 * (base_size(axis_size(mn, axis), Neg ? tempI : tempO, mn.alphaCTE) +
                       base_size(axis_size(mp, axis), Neg ? tempO : tempI, mp.alphaCTE));
-    } else {
-        rest = s.ldIn[LREST * nl + slot];
     }
-    LinkPrev old;
-    old.pos2 = dv(s.ldIn[LP2X * nl + slot], s.ldIn[LP2Y * nl + slot], s.ldIn[LP2Z * nl + slot]);
-    old.a1 = dv(s.ldIn[LA1X * nl + slot], s.ldIn[LA1Y * nl + slot], s.ldIn[LA1Z * nl + slot]);
-    old.a2 = dv(s.ldIn[LA2X * nl + slot], s.ldIn[LA2Y * nl + slot], s.ldIn[LA2Z * nl + slot]);
-    old.flags = s.lflIn[slot];
-    old.maxStrain = s.lfIn[LMAXSTRAIN * nl + slot];
-    old.strainOffset = s.lfIn[LOFFSET * nl + slot];
+    LinkPrev old = in.old;
     if (Poisson) { /* volume effects (VX_Link.cpp:160) */
-        old.tArea = s.lfIn[LTAREA * nl + slot];
-        old.tss = s.lfIn[LTSS * nl + slot];
-        link_transverse(m, s.vmats[s.vmat[n]], s.vmats[s.vmat[p]], s.vps, nv, n, p, axis, &old.tArea, &old.tss);
+        link_transverse(m, mn, mp, s.vps, nv, n, p, axis, &old.tArea, &old.tss);
     } else {
         old.tArea = m.transverseArea;
         old.tss = 0.0f;
     }
     float dmN = 0.0f, dmP = 0.0f;
     if (old.flags & LF_LVV) { /* dampingMultiplier (VX_Voxel.h:130) of both voxels */
-        dmN = s.vmats[s.vmat[n]].dampNum / prevDt;
-        dmP = s.vmats[s.vmat[p]].dampNum / prevDt;
+        dmN = mn.dampNum / prevDt;
+        dmP = mp.dampNum / prevDt;
     }
     LinkEval e;
     link_eval_fp64<Poisson>(m, s.curveStrain + m.curveOff, s.curveStress + m.curveOff, axis, Neg ? pos0 : po,
                    Neg ? q0 : qo, Neg ? po : pos0, Neg ? qo : q0, rest, old, dmN, dmP, &e);
-    const dvec f = Neg ? e.fN : e.fP, mm = Neg ? e.mN : e.mP;
-    sf.x += f.x; sf.y += f.y; sf.z += f.z;
-    sm.x += mm.x; sm.y += mm.y; sm.z += mm.z;
+    f = Neg ? e.fN : e.fP;
+    mm = Neg ? e.mN : e.mP;
     if (s.storeForces) {
         double* slotF = s.vf + vf_index(dir, 0, nv, i);
         slotF[0] = f.x; slotF[1] = f.y; slotF[2] = f.z;
@@ -126,23 +155,23 @@ __device__ __forceinline__ void link_end(const FusedPtrs& s, int i, int o, int d
     }
     if (!ForcesOnly && Neg) {
         double* ld = s.ldOut;
-        st_nt(&ld[LP2X * nl + slot], e.pos2.x); st_nt(&ld[LP2Y * nl + slot], e.pos2.y);
-        st_nt(&ld[LP2Z * nl + slot], e.pos2.z);
-        st_nt(&ld[LA1X * nl + slot], e.a1v.x); st_nt(&ld[LA1Y * nl + slot], e.a1v.y);
-        st_nt(&ld[LA1Z * nl + slot], e.a1v.z);
-        st_nt(&ld[LA2X * nl + slot], e.a2v.x); st_nt(&ld[LA2Y * nl + slot], e.a2v.y);
-        st_nt(&ld[LA2Z * nl + slot], e.a2v.z);
-        if (!s.restConst) st_nt(&ld[LREST * nl + slot], rest);
+        put<Cached>(&ld[LP2X * nl + slot], e.pos2.x); put<Cached>(&ld[LP2Y * nl + slot], e.pos2.y);
+        put<Cached>(&ld[LP2Z * nl + slot], e.pos2.z);
+        put<Cached>(&ld[LA1X * nl + slot], e.a1v.x); put<Cached>(&ld[LA1Y * nl + slot], e.a1v.y);
+        put<Cached>(&ld[LA1Z * nl + slot], e.a1v.z);
+        put<Cached>(&ld[LA2X * nl + slot], e.a2v.x); put<Cached>(&ld[LA2Y * nl + slot], e.a2v.y);
+        put<Cached>(&ld[LA2Z * nl + slot], e.a2v.z);
+        if (!s.restConst) put<Cached>(&ld[LREST * nl + slot], rest);
         float* lf = s.lfOut;
-        st_nt(&lf[LSTRAIN * nl + slot], e.strain);
-        st_nt(&lf[LMAXSTRAIN * nl + slot], e.maxStrain);
-        if (!s.offsetConst) st_nt(&lf[LOFFSET * nl + slot], e.strainOffset);
-        st_nt(&lf[LSTRESS * nl + slot], e.stress);
+        put<Cached>(&lf[LSTRAIN * nl + slot], e.strain);
+        put<Cached>(&lf[LMAXSTRAIN * nl + slot], e.maxStrain);
+        if (!s.offsetConst) put<Cached>(&lf[LOFFSET * nl + slot], e.strainOffset);
+        put<Cached>(&lf[LSTRESS * nl + slot], e.stress);
         if (Poisson) {
             lf[LTAREA * nl + slot] = old.tArea;
             lf[LTSS * nl + slot] = old.tss;
         }
-        st_nt(&s.lflOut[slot], e.flags);
+        put<Cached>(&s.lflOut[slot], e.flags);
         if (e.strain > 100) {
             atomicMin(&s.rdiv[rob], s.k);
             atomicOr(&s.ctl[0], 1);
@@ -165,6 +194,30 @@ __device__ __forceinline__ void link_end(const FusedPtrs& s, int i, int o, int d
 #define VX_MATS_LDS 1
 #endif
 constexpr int kLdsVoxMats = 32, kLdsLinkMats = 64;
+__device__ __forceinline__ void stage_materials(const FusedPtrs& s, VoxMat* svm, LinkMat* slm) {
+    const int nv32 = s.nvmats * (int)(sizeof(VoxMat) / 4), nl32 = s.nlmats * (int)(sizeof(LinkMat) / 4);
+    for (int t = threadIdx.x; t < nv32; t += blockDim.x) ((uint32_t*)svm)[t] = ((const uint32_t*)s.vmats)[t];
+    for (int t = threadIdx.x; t < nl32; t += blockDim.x) ((uint32_t*)slm)[t] = ((const uint32_t*)s.lmats)[t];
+    __syncthreads();
+}
+
+/* contacts in partner order (VX_Voxel.cpp:250-253), each pair's force from voxel i's side as the
+   split step's contact kernel forms it */
+__device__ __forceinline__ void subtract_contacts(const FusedPtrs& s, const VoxMat& m, int i, float tempI, float tnow,
+                                                  dvec& t) {
+    if (!s.colCnt) return;
+    const int nv = s.nv;
+    const int cnt = s.colCnt[i], off = s.colOff[i];
+    if (cnt == 0) return;
+    const ContactSelf me = contact_self(m, s.vdIn, nv, i, tempI);
+    for (int c = 0; c < cnt; c++) {
+        const int j = s.partners[off + c];
+        const float tj = s.vphase ? actuation_temperature(s.actBase, s.actAmp, s.actFreq, tnow, s.vphase[j])
+                                  : s.vtemp[j];
+        const fvec f = contact_pair_force(me, s.vmats[s.vmat[j]], s.vdIn, nv, j, tj);
+        t.x -= f.x; t.y -= f.y; t.z -= f.z;
+    }
+}
 
 /* Driven: instances for contact-batch steps (the watch-list test on the positions written) and
    prescribed-displacement ramps; the others carry neither, and none of their registers. */
@@ -174,12 +227,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(VX_FUS
     if (MatsLds) {
         __shared__ VoxMat svm[kLdsVoxMats];
         __shared__ LinkMat slm[kLdsLinkMats];
-        {
-            const int nv32 = s0.nvmats * (int)(sizeof(VoxMat) / 4), nl32 = s0.nlmats * (int)(sizeof(LinkMat) / 4);
-            for (int t = threadIdx.x; t < nv32; t += blockDim.x) ((uint32_t*)svm)[t] = ((const uint32_t*)s0.vmats)[t];
-            for (int t = threadIdx.x; t < nl32; t += blockDim.x) ((uint32_t*)slm)[t] = ((const uint32_t*)s0.lmats)[t];
-        }
-        __syncthreads();
+        stage_materials(s0, svm, slm);
         s.vmats = svm;
         s.lmats = slm;
     }
@@ -232,8 +280,17 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(VX_FUS
             continue;
         }
         /* the two ends as separate instances, each computing only its own end vectors */
-        if ((dir & 1) == 0) link_end<ForcesOnly, true, Poisson>(s, i, o, dir, rob, prevDt, tnow, tempI, pos0, q0, sf, sm);
-        else link_end<ForcesOnly, false, Poisson>(s, i, o, dir, rob, prevDt, tnow, tempI, pos0, q0, sf, sm);
+        dvec f, mm;
+        LinkIn in;
+        if ((dir & 1) == 0) {
+            link_load<true, Poisson>(s, i, o, dir, in);
+            link_end<ForcesOnly, true, Poisson, false>(s, in, i, o, mi, dir, rob, prevDt, tnow, tempI, pos0, q0, f, mm);
+        } else {
+            link_load<false, Poisson>(s, i, o, dir, in);
+            link_end<ForcesOnly, false, Poisson, false>(s, in, i, o, mi, dir, rob, prevDt, tnow, tempI, pos0, q0, f, mm);
+        }
+        sf.x += f.x; sf.y += f.y; sf.z += f.z;
+        sm.x += mm.x; sm.y += mm.y; sm.z += mm.z;
     }
     if (ForcesOnly) return;
     /* the voxel's index through an opaque copy: its addresses are formed here, after the link
@@ -258,24 +315,171 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(VX_FUS
     dvec pos = pos0, lin = dv(ld_nt(&vd[VLX * nv + iv]), ld_nt(&vd[VLY * nv + iv]), ld_nt(&vd[VLZ * nv + iv]));
     dvec ang = dv(ld_nt(&vd[VAX * nv + iv]), ld_nt(&vd[VAY * nv + iv]), ld_nt(&vd[VAZ * nv + iv]));
     dquat q = q0;
-    voxel_step_fp64(m, ex, s.vijk, nv, iv, dt, tempI, sf, sm, pos, lin, ang, q, flags, [&](dvec& t) {
-        /* contacts in partner order (VX_Voxel.cpp:250-253), each pair's force from this
-           voxel's side as the split step's contact kernel forms it */
-        if (!s.colCnt) return;
-        const int cnt = s.colCnt[iv], off = s.colOff[iv];
-        if (cnt == 0) return;
-        const ContactSelf me = contact_self(m, vd, nv, iv, tempI);
-        for (int c = 0; c < cnt; c++) {
-            const int j = s.partners[off + c];
-            const float tj = s.vphase ? actuation_temperature(s.actBase, s.actAmp, s.actFreq, tnow, s.vphase[j])
-                                      : s.vtemp[j];
-            const fvec f = contact_pair_force(me, s.vmats[s.vmat[j]], vd, nv, j, tj);
-            t.x -= f.x; t.y -= f.y; t.z -= f.z;
-        }
-    });
+    voxel_step_fp64(m, ex, s.vijk, nv, iv, dt, tempI, sf, sm, pos, lin, ang, q, flags,
+                    [&](dvec& t) { subtract_contacts(s, m, iv, tempI, tnow, t); });
     store_voxel(s.vdOut, nv, iv, pos, lin, ang, q);
     st_nt(&s.vflOut[iv], flags & ~(uint32_t)VF_PS_VALID); /* poissonsStrainInvalid = true (VX_Voxel.cpp:231) */
     if (Driven && s.haltTest) halt_if_stale(s.halt, s.k + 1, s.colLast, s.recalcSq, s.vflIn, nv, iv, pos.x, pos.y, pos.z);
+}
+
+/* The same step for models that do not fill the chip: a workgroup takes 64 voxels and splits
+   their link directions over its waves, PerWave directions to a wave, so a voxel's <= 6 links run
+   side by side instead of one after the other; the end vectors meet in LDS (18 KB), where wave 0
+   sums the forces in direction order and integrates the translations while wave 1 does the same
+   with the moments and rotations.  Each link end is evaluated by link_end on the same inputs and
+   the sums keep their order (an absent link adds +0.0), so the bits are k_step_fp64's.
+
+   What bounds it: the chain of dependent loads and FP64 operations of one link (2.7 us of the 5 us
+   a workgroup lives; 2.5 us more pass between two launches), which k_step_fp64 walks through six
+   times over.  us per step of a two-material lattice, k_step_fp64 at its best launch shape -> here:
+   290 voxels 14.7 -> 6.6; 7,169 15.5 -> 6.7; 15,784 15.9 -> 7.3 (PerWave 1: six waves with 185
+   VGPRs, two a SIMD, everything a lane reads asked for up front);
+   17,676 16.9 -> 10.1; 45,352 19.4 -> 13.8; 112,451 29.9 -> 26.8; 235,932 59.9 -> 48.8 (PerWave 2:
+   three waves at three a SIMD; PerWave 1 takes 12.2 at 24,286 voxels where PerWave 2 takes 10.4,
+   since a second workgroup of six waves no longer finds room beside the first).
+   The blocks map to the XCDs in contiguous ranges and the stores go through the caches, so that
+   the next step finds a tile's state, and most of its neighbours', in the same L2 (45,352 voxels:
+   15.9 linear and non-temporal, 15.0 contiguous, 13.8 contiguous and cached). */
+constexpr int kEndsTile = 64;
+constexpr int kEndsWideMax = 256 * kEndsTile; /* one workgroup of six waves a CU */
+template <int PerWave, bool Poisson, bool MatsLds, bool Driven>
+__global__ void __launch_bounds__(6 / PerWave * kEndsTile) __attribute__((amdgpu_waves_per_eu(PerWave == 1 ? 2 : 3, 8))) k_step_fp64_ends(FusedPtrs s0) {
+    FusedPtrs s = s0;
+    const int nv = s.nv;
+    if (s.halt && s.halt[0] <= s.k) return; /* the whole grid: a halt recorded by this step is k + 1 */
+    const int lane = threadIdx.x & (kEndsTile - 1);
+    const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x / kEndsTile);
+    const int at = xcd_block() * kEndsTile + lane;
+    const double* __restrict__ vd = s.vdIn;
+    __shared__ double ends[6][6][kEndsTile];
+    __shared__ VoxMat svm[MatsLds ? kLdsVoxMats : 1];
+    __shared__ LinkMat slm[MatsLds ? kLdsLinkMats : 1];
+    const int c0 = 3 * wave; /* wave 0 integrates the translations, wave 1 the rotations */
+    int i = at, rob = 0, mi = 0, o = -1, ei = -1, d = 0;
+    float dt = 0.0f, tnow = 0.0f, tempI = 0.0f;
+    uint32_t flags = 0;
+    dvec pos0, mom = dv(0.0, 0.0, 0.0);
+    dquat q0;
+    bool live;
+    if (PerWave == 1) {
+        /* what a lane reads is asked for at once, before the material tables' barrier and the
+           test of its robot (a lane past the end reads the last voxel's) */
+        i = at < nv ? at : nv - 1;
+        o = s.vnbr[wave * nv + i];
+        rob = s.vrobot[i];
+        mi = s.vmat[i];
+        pos0 = dv(vd[VPX * nv + i], vd[VPY * nv + i], vd[VPZ * nv + i]);
+        q0 = dq(vd[VQW * nv + i], vd[VQX * nv + i], vd[VQY * nv + i], vd[VQZ * nv + i]);
+        tempI = s.vtemp[i];
+        if (wave < 2) {
+            mom = dv(vd[(VLX + c0) * nv + i], vd[(VLY + c0) * nv + i], vd[(VLZ + c0) * nv + i]);
+            ei = s.vext[i];
+            flags = s.vflIn[i];
+        }
+    }
+    if (MatsLds) {
+        stage_materials(s0, svm, slm);
+        s.vmats = svm;
+        s.lmats = slm;
+    }
+    if (PerWave == 1) {
+        d = s.rdiv[rob];
+        dt = s.rdt[rob];
+        tnow = s.rtimeIn[rob];
+        live = at < nv && d >= s.k;
+    } else {
+        live = at < nv;
+        if (live) {
+            rob = s.vrobot[i];
+            d = s.rdiv[rob];
+            live = d >= s.k;
+        }
+    }
+    if (at < nv && !live && wave == 0) {
+        frozen_fp64(s, i, rob, d);
+        if (Driven && s.haltTest)
+            halt_if_stale(s.halt, s.k + 1, s.colLast, s.recalcSq, s.vflIn, nv, i, s.vdOut[VPX * nv + i],
+                          s.vdOut[VPY * nv + i], s.vdOut[VPZ * nv + i]);
+    }
+    if (live) {
+        if (PerWave > 1) {
+            mi = s.vmat[i];
+            pos0 = dv(vd[VPX * nv + i], vd[VPY * nv + i], vd[VPZ * nv + i]);
+            q0 = dq(vd[VQW * nv + i], vd[VQX * nv + i], vd[VQY * nv + i], vd[VQZ * nv + i]);
+            tempI = s.vtemp[i];
+            dt = s.rdt[rob];
+            tnow = s.rtimeIn[rob];
+        }
+        const float prevDt = s.k == 0 ? s.rprev[rob] : dt;
+        if (s.vphase) {
+            tempI = actuation_temperature(s.actBase, s.actAmp, s.actFreq, tnow, s.vphase[i]);
+            if (wave == 0) s.vtemp[i] = tempI;
+        }
+#pragma unroll 1
+        for (int dir = PerWave * wave; dir < PerWave * (wave + 1); dir++) {
+            if (PerWave > 1) o = s.vnbr[dir * nv + i];
+            dvec f = dv(0.0, 0.0, 0.0), mm = dv(0.0, 0.0, 0.0);
+            if (o >= 0) {
+                LinkIn in;
+                if ((dir & 1) == 0) {
+                    link_load<true, Poisson>(s, i, o, dir, in);
+                    link_end<false, true, Poisson, true>(s, in, i, o, mi, dir, rob, prevDt, tnow, tempI, pos0, q0, f, mm);
+                } else {
+                    link_load<false, Poisson>(s, i, o, dir, in);
+                    link_end<false, false, Poisson, true>(s, in, i, o, mi, dir, rob, prevDt, tnow, tempI, pos0, q0, f, mm);
+                }
+            } else if (s.storeForces) {
+                for (int c = 0; c < 6; c++) s.vf[vf_index(dir, c, nv, i)] = 0.0;
+            }
+            ends[dir][0][lane] = f.x; ends[dir][1][lane] = f.y; ends[dir][2][lane] = f.z;
+            ends[dir][3][lane] = mm.x; ends[dir][4][lane] = mm.y; ends[dir][5][lane] = mm.z;
+        }
+    }
+    __syncthreads();
+    if (wave > 1 || !live) return;
+    if (PerWave > 1) {
+        mom = dv(vd[(VLX + c0) * nv + i], vd[(VLY + c0) * nv + i], vd[(VLZ + c0) * nv + i]);
+        ei = s.vext[i];
+        flags = s.vflIn[i];
+    }
+
+    /* CVX_Voxel::timeStep (VX_Voxel.cpp:162-232): translation in wave 0, rotation in wave 1 */
+    const VoxMat m = s.vmats[mi];
+    const ExtRec* ex = ei >= 0 ? &s.exts[ei] : nullptr;
+    const bool pinned = ex && (ex->dof & 0x3F) == 0x3F;
+    dvec sum = dv(0.0, 0.0, 0.0);
+    for (int e = 0; e < 6; e++) {
+        sum.x += ends[e][c0][lane]; sum.y += ends[e][c0 + 1][lane]; sum.z += ends[e][c0 + 2][lane];
+    }
+    double* __restrict__ out = s.vdOut;
+    if (wave == 1) {
+        if (pinned) return;
+        dvec ang = mom;
+        dquat q = q0;
+        voxel_rotate_fp64(m, ex, dt, sum, ang, q);
+        if (ex) voxel_fix_rotation(ex, ang, q);
+        out[VAX * nv + i] = ang.x; out[VAY * nv + i] = ang.y; out[VAZ * nv + i] = ang.z;
+        out[VQW * nv + i] = q.w; out[VQX * nv + i] = q.x; out[VQY * nv + i] = q.y; out[VQZ * nv + i] = q.z;
+        return;
+    }
+    if (i == 0 || s.vrobot[i - 1] != rob) s.rtimeOut[rob] = tnow + dt; /* currentTime += dt */
+    if (Driven) apply_ramp(s.exts, s.ramps, ei, tnow);
+    if (pinned) {
+        voxel_pinned(m, ex, s.vijk, nv, i, out);
+        s.vflOut[i] = flags;
+        if (Driven && s.haltTest)
+            halt_if_stale(s.halt, s.k + 1, s.colLast, s.recalcSq, s.vflIn, nv, i, out[VPX * nv + i], out[VPY * nv + i],
+                          out[VPZ * nv + i]);
+        return;
+    }
+    dvec pos = pos0, lin = mom;
+    voxel_translate_fp64(m, ex, dt, tempI, sum, q0, pos, lin, flags,
+                         [&](dvec& t) { subtract_contacts(s, m, i, tempI, tnow, t); });
+    if (ex) voxel_fix_translation(m, ex, s.vijk, nv, i, pos, lin);
+    out[VPX * nv + i] = pos.x; out[VPY * nv + i] = pos.y; out[VPZ * nv + i] = pos.z;
+    out[VLX * nv + i] = lin.x; out[VLY * nv + i] = lin.y; out[VLZ * nv + i] = lin.z;
+    s.vflOut[i] = flags & ~(uint32_t)VF_PS_VALID; /* poissonsStrainInvalid = true (VX_Voxel.cpp:231) */
+    if (Driven && s.haltTest) halt_if_stale(s.halt, s.k + 1, s.colLast, s.recalcSq, s.vflIn, nv, i, pos.x, pos.y, pos.z);
 }
 
 /* after a launch: previousDt of every voxel whose robot completed at least one step */
@@ -324,6 +528,28 @@ void launch_step_fp64(const FusedPtrs& s, int block, bool forcesOnly, hipStream_
         else { VX_STEP64(false, false); }
     }
 #undef VX_STEP64
+}
+void launch_step_fp64_ends(const FusedPtrs& s, hipStream_t st) {
+    if (s.nv <= 0) return;
+    const int perWave = s.nv <= kEndsWideMax ? 1 : 2;
+    const dim3 grid((unsigned)((s.nv + kEndsTile - 1) / kEndsTile)), block(6 / perWave * kEndsTile);
+    const bool lds = VX_MATS_LDS && s.nvmats <= kLdsVoxMats && s.nlmats <= kLdsLinkMats;
+    const bool driven = s.haltTest || s.ramps;
+#define VX_ENDS64(W, P, L)                                                                                \
+    if (driven) hipLaunchKernelGGL((k_step_fp64_ends<W, P, L, true>), grid, block, 0, st, s);            \
+    else hipLaunchKernelGGL((k_step_fp64_ends<W, P, L, false>), grid, block, 0, st, s)
+#define VX_ENDS64_W(W)                                                                                    \
+    if (s.poisson) {                                                                                      \
+        if (lds) { VX_ENDS64(W, true, true); }                                                            \
+        else { VX_ENDS64(W, true, false); }                                                               \
+    } else {                                                                                              \
+        if (lds) { VX_ENDS64(W, false, true); }                                                           \
+        else { VX_ENDS64(W, false, false); }                                                              \
+    }
+    if (perWave == 1) { VX_ENDS64_W(1) }
+    else { VX_ENDS64_W(2) }
+#undef VX_ENDS64_W
+#undef VX_ENDS64
 }
 void launch_fused_prevdt(const int* vrobot, const int* rdiv, const float* rdt, float* vprevdt, int nv, hipStream_t st) {
     if (nv > 0)

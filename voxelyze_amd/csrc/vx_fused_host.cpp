@@ -12,6 +12,7 @@
 namespace vx {
 
 void launch_step_fp64(const FusedPtrs& s, int block, bool forcesOnly, hipStream_t st);
+void launch_step_fp64_ends(const FusedPtrs& s, hipStream_t st);
 void launch_fused_prevdt(const int* vrobot, const int* rdiv, const float* rdt, float* vprevdt, int nv, hipStream_t st);
 void launch_fused_restore(double* vd, const double* vdPrev, uint32_t* vfl, const uint32_t* vflPrev, float* vtemp,
                           const float* vtempPrev, float* rtime, const float* rtimePrev, int nv, int first, int count,
@@ -114,7 +115,8 @@ bool Sim::stepFp64Fused(int nsteps) {
         a.rtimeIn = dp.rtime;
         a.rtimeOut = (float*)brtimeAlt.p;
     };
-    const bool tune = tuning(3);
+    const bool ends = endsPath(3, kEndsMaxFp64);
+    const bool tune = !ends && tuning(3);
     const bool timed = profiling || tune;
     const bool graph = useGraphs && !collisions && !timed && nsteps > 1 && nsteps <= kGraphMaxStepsFused;
     const LaunchCfg chosen = tuner[3].chosen;
@@ -139,7 +141,7 @@ bool Sim::stepFp64Fused(int nsteps) {
         FusedPtrs k0 = fp;
         bind(k0);
         k0.xcd = chosen.xcd;
-        key = graph_key(&k0, sizeof k0, 4, nsteps, ((actOn ? 1 : 0) | (chosen.block << 1)) ^ rampKey());
+        key = graph_key(&k0, sizeof k0, ends ? 5 : 4, nsteps, ((actOn ? 1 : 0) | (chosen.block << 1)) ^ rampKey());
         bool replayed = false;
         if (!graphLaunch(key, &replayed)) return false;
         if (replayed) { /* the host side of the ping-pong, as the recorded launch left it */
@@ -204,7 +206,8 @@ bool Sim::stepFp64Fused(int nsteps) {
         fp.xcd = cfg.xcd;
         launch_poisson_fp64(dp, k, stream); /* the Poisson strains this step's links read */
         if (timed) (void)hipEventRecord(events[2 * k], stream);
-        launch_step_fp64(fp, cfg.block, false, stream);
+        if (ends) launch_step_fp64_ends(fp, stream);
+        else launch_step_fp64(fp, cfg.block, false, stream);
         if (timed) (void)hipEventRecord(events[2 * k + 1], stream);
         swapFp64Buffers();
         launched++;

@@ -1362,7 +1362,7 @@ static const int kTuneSamples = 2;
 void Sim::Tuner::reset(int n) {
     nv = n;
     steps = 0;
-    settled = false;
+    settled = pinned = false;
     chosen = kCands[0];
     for (int c = 0; c < 6; c++) { best[c] = 1e30f; count[c] = 0; }
 }
@@ -1388,6 +1388,13 @@ bool Sim::tuning(int t) {
     if (!autotune) return false;
     if (tuner[t].nv != nv()) tuner[t].reset(nv());
     return !tuner[t].settled;
+}
+
+bool Sim::endsPath(int t, int maxVoxels) {
+    if (tuner[t].nv != nv()) tuner[t].reset(nv());
+    if (tuner[t].pinned || nv() > maxVoxels) return false;
+    tuner[t].settled = true; /* nothing to choose */
+    return true;
 }
 
 /* ------------------------------------------------------------ step graphs */

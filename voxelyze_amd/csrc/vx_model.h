@@ -242,6 +242,7 @@ struct Sim {
         int count[6];
         LaunchCfg chosen{256, 0};
         bool settled = false;
+        bool pinned = false; /* set by vxg_set_launch_config for this model size */
         Tuner() { reset(-1); }
         void reset(int n);
         LaunchCfg next(int* cand);
@@ -250,6 +251,13 @@ struct Sim {
     Tuner tuner[4]; /* 0 fused mixed step, 1 FP64 link kernel, 2 FP64 voxel kernel, 3 fused FP64 step */
     bool autotune = true;
     bool tuning(int t);
+    /* step kernel t with its link directions split over waves (vx_fused.hip): models of at most
+       maxVoxels, unless a launch configuration was pinned.  The FP64 step up to 294,912 voxels,
+       where the two copies of the state outgrow the 256 MB Infinity Cache and the kernel with the
+       fewest bytes in flight per voxel wins (us per step, k_step_fp64 against k_step_fp64_ends:
+       282,309 voxels 68.2 / 63.4, 332,769 voxels 77.5 / 82.2, 943,896 voxels 226 / 251). */
+    bool endsPath(int t, int maxVoxels);
+    static constexpr int kEndsMaxFp64 = 294912;
     /* kernel timing */
     bool profiling = false;
     std::vector<hipEvent_t> events;

@@ -247,14 +247,13 @@ __device__ __forceinline__ float floor_penetration(const VoxMat& m, float temp, 
     return (float)(bsa / 2 - m.nomSize / 2 - pz);
 }
 
-/* CVX_Voxel::timeStep from the link force and moment sums on (VX_Voxel.cpp:174-232, force()
-   and moment() after their direction-ordered sums, VX_Voxel.cpp:234-271, floorForce
-   :274-298), in place on the state; contacts(t) subtracts the contact forces in partner
-   order (VX_Voxel.cpp:250-253). */
+/* The translation of CVX_Voxel::timeStep from the link force sum on (VX_Voxel.cpp:174-196, force()
+   after its direction-ordered sum, VX_Voxel.cpp:234-256, floorForce :274-298), in place on the
+   state; contacts(t) subtracts the contact forces in partner order (VX_Voxel.cpp:250-253). */
 template <class Contacts>
-__device__ __forceinline__ void voxel_step_fp64(const VoxMat& m, const ExtRec* ex, const int* __restrict__ vijk, int nv,
-                                                int i, float dt, float temp, dvec sumF, dvec sumM, dvec& pos,
-                                                dvec& lin, dvec& ang, dquat& q, uint32_t& flags, Contacts contacts) {
+__device__ __forceinline__ void voxel_translate_fp64(const VoxMat& m, const ExtRec* ex, float dt, float temp, dvec sumF,
+                                                     const dquat& q, dvec& pos, dvec& lin, uint32_t& flags,
+                                                     Contacts contacts) {
     dvec t = qrot(q, sumF);
     if (ex) { t.x += ex->fx; t.y += ex->fy; t.z += ex->fz; }
     {
@@ -307,7 +306,11 @@ __device__ __forceinline__ void voxel_step_fp64(const VoxMat& m, const ExtRec* e
         flags &= ~VF_STATIC;
     }
     pos.x += tr.x; pos.y += tr.y; pos.z += tr.z;
+}
 
+/* its rotation from the link moment sum on (VX_Voxel.cpp:198-208, moment() :258-271) */
+__device__ __forceinline__ void voxel_rotate_fp64(const VoxMat& m, const ExtRec* ex, float dt, dvec sumM, dvec& ang,
+                                                  dquat& q) {
     dvec mo = qrot(q, sumM);
     if (ex) { mo.x += ex->mx; mo.y += ex->my; mo.z += ex->mz; }
     {
@@ -317,26 +320,43 @@ __device__ __forceinline__ void voxel_step_fp64(const VoxMat& m, const ExtRec* e
     ang.x += dt * mo.x; ang.y += dt * mo.y; ang.z += dt * mo.z;
     const float dti = dt * m.momentInertiaInverse;
     q = qmul(qfromrv(dv(dti * ang.x, dti * ang.y, dti * ang.z)), q);
+}
 
-    if (ex) {
-        /* partial dof fixes (VX_Voxel.cpp:210-228) */
-        const double sz = m.nomSize;
-        const int dof = ex->dof;
-        if (dof & 1) { pos.x = vijk[i] * sz + ex->tx; lin.x = 0.0; }
-        if (dof & 2) { pos.y = vijk[nv + i] * sz + ex->ty; lin.y = 0.0; }
-        if (dof & 4) { pos.z = vijk[2 * nv + i] * sz + ex->tz; lin.z = 0.0; }
-        if (dof & 56) {
-            if ((dof & 56) == 56) {
-                q = dq(ex->qw, ex->qx, ex->qy, ex->qz);
-                ang = dv(0.0, 0.0, 0.0);
-            } else {
-                dvec rv = qtorv(q);
-                if (dof & 8) { rv.x = 0.0; ang.x = 0.0; }
-                if (dof & 16) { rv.y = 0.0; ang.y = 0.0; }
-                if (dof & 32) { rv.z = 0.0; ang.z = 0.0; }
-                q = qfromrv(rv);
-            }
+/* partial dof fixes (VX_Voxel.cpp:210-228): the fixed coordinates, and the fixed rotation axes */
+__device__ __forceinline__ void voxel_fix_translation(const VoxMat& m, const ExtRec* ex, const int* __restrict__ vijk,
+                                                      int nv, int i, dvec& pos, dvec& lin) {
+    const double sz = m.nomSize;
+    const int dof = ex->dof;
+    if (dof & 1) { pos.x = vijk[i] * sz + ex->tx; lin.x = 0.0; }
+    if (dof & 2) { pos.y = vijk[nv + i] * sz + ex->ty; lin.y = 0.0; }
+    if (dof & 4) { pos.z = vijk[2 * nv + i] * sz + ex->tz; lin.z = 0.0; }
+}
+__device__ __forceinline__ void voxel_fix_rotation(const ExtRec* ex, dvec& ang, dquat& q) {
+    const int dof = ex->dof;
+    if (dof & 56) {
+        if ((dof & 56) == 56) {
+            q = dq(ex->qw, ex->qx, ex->qy, ex->qz);
+            ang = dv(0.0, 0.0, 0.0);
+        } else {
+            dvec rv = qtorv(q);
+            if (dof & 8) { rv.x = 0.0; ang.x = 0.0; }
+            if (dof & 16) { rv.y = 0.0; ang.y = 0.0; }
+            if (dof & 32) { rv.z = 0.0; ang.z = 0.0; }
+            q = qfromrv(rv);
         }
+    }
+}
+
+/* CVX_Voxel::timeStep from the link force and moment sums on (VX_Voxel.cpp:174-232) */
+template <class Contacts>
+__device__ __forceinline__ void voxel_step_fp64(const VoxMat& m, const ExtRec* ex, const int* __restrict__ vijk, int nv,
+                                                int i, float dt, float temp, dvec sumF, dvec sumM, dvec& pos,
+                                                dvec& lin, dvec& ang, dquat& q, uint32_t& flags, Contacts contacts) {
+    voxel_translate_fp64(m, ex, dt, temp, sumF, q, pos, lin, flags, contacts);
+    voxel_rotate_fp64(m, ex, dt, sumM, ang, q);
+    if (ex) {
+        voxel_fix_translation(m, ex, vijk, nv, i, pos, lin);
+        voxel_fix_rotation(ex, ang, q);
     }
 }
 
