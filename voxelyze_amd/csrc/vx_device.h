@@ -325,7 +325,9 @@ struct FusedPtrs {
     const int* vmat;
     const int* vext;
     const int* vijk;
-    float* vtemp;             /* in place: under actuation each lane writes its own */
+    float* vtempIn;           /* temperatures of this step; under actuation a step writes the next */
+    float* vtempOut;          /* step's into vtempOut unless it is the launch's last (tempNext 0) */
+    int tempNext;
     const VoxMat* vmats;
     const LinkMat* lmats;
     const float* curveStrain;

@@ -25,8 +25,11 @@
  * End forces (what CVX_Link::force() returns) are written to the split step's force slots
  * on the launch's last step only.
  *
- * Actuation: each lane sets its own temperature for the step (as k_actuate_fp64 does) and
- * evaluates its neighbours' temperatures itself for the links' rest lengths and contacts.
+ * Actuation: temperatures are double-buffered like the state.  A launch starts with k_fused_temps
+ * (as k_actuate_fp64 sets them), and every step but the last writes its voxels' temperatures at the
+ * robot's time after it, which the next step's rest lengths and contacts read: one correctly
+ * rounded sine per voxel and step instead of one for each link end as well (a population of 48
+ * robots, 74,400 voxels: 21.5 -> 18.1 ms for 200 steps).
  */
 #include "vx_contact_force.h"
 #include "vx_device.h"
@@ -41,6 +44,10 @@ namespace vx {
 __device__ void frozen_fp64(const FusedPtrs& s, int i, int rob, int d) {
     const int nv = s.nv, nl = s.nl;
     const bool idle = d < 0;
+    if (s.vphase) { /* both halves keep the temperatures of the last step that counted */
+        if (idle) s.vtempOut[i] = s.vtempIn[i];
+        else if (s.k == d + 1) s.vtempIn[i] = s.vtempOut[i];
+    }
     if (idle || ((s.k - d) & 1) == 0) {
         for (int c = 0; c < VD_COUNT; c++) s.vdOut[c * nv + i] = s.vdIn[c * nv + i];
         s.vflOut[i] = s.vflIn[i];
@@ -79,6 +86,7 @@ __device__ __forceinline__ void put(T* p, T v) {
 /* what one end of a link reads: the neighbour's pose and material, the link's material and state */
 struct LinkIn {
     int meta, mo;
+    float to; /* the neighbour's temperature (read under actuation) */
     dvec po;
     dquat qo;
     double rest;
@@ -104,6 +112,7 @@ __device__ __forceinline__ void link_load(const FusedPtrs& s, int i, int o, int 
     }
     in.rest = s.ldIn[LREST * nl + slot];
     in.mo = s.vmat[o];
+    if (s.vphase) in.to = s.vtempIn[o];
     in.po = dv(vd[VPX * nv + o], vd[VPY * nv + o], vd[VPZ * nv + o]);
     in.qo = dq(vd[VQW * nv + o], vd[VQX * nv + o], vd[VQY * nv + o], vd[VQZ * nv + o]);
 }
@@ -114,7 +123,7 @@ __device__ __forceinline__ void link_load(const FusedPtrs& s, int i, int o, int 
    Poisson: some material has Poisson's ratio != 0 (the transverse info is read and kept) */
 template <bool ForcesOnly, bool Neg, bool Poisson, bool Cached>
 __device__ __forceinline__ void link_end(const FusedPtrs& s, LinkIn& in, int i, int o, int mi, int dir, int rob,
-                                         float prevDt, float tnow, float tempI, const dvec& pos0, const dquat& q0,
+                                         float prevDt, float tempI, const dvec& pos0, const dquat& q0,
                                          dvec& f, dvec& mm) {
     const int nv = s.nv, nl = s.nl;
     const int axis = dir >> 1;
@@ -127,7 +136,7 @@ __device__ __forceinline__ void link_end(const FusedPtrs& s, LinkIn& in, int i, 
     const dquat qo = in.qo;
     double rest = in.rest;
     if (s.vphase) { /* updateRestLength (VX_Link.cpp:137-140) at this step's temperatures */
-        const float tempO = actuation_temperature(s.actBase, s.actAmp, s.actFreq, tnow, s.vphase[o]);
+        const float tempO = in.to;
         rest = 0.5 * (base_size(axis_size(mn, axis), Neg ? tempI : tempO, mn.alphaCTE) +
                       base_size(axis_size(mp, axis), Neg ? tempO : tempI, mp.alphaCTE));
     }
@@ -201,10 +210,15 @@ __device__ __forceinline__ void stage_materials(const FusedPtrs& s, VoxMat* svm,
     __syncthreads();
 }
 
+/* voxel i's temperature for the next step, at its robot's time after this one */
+__device__ __forceinline__ void next_temperature(const FusedPtrs& s, int i, int rob, float dt) {
+    if (s.vphase && s.tempNext)
+        s.vtempOut[i] = actuation_temperature(s.actBase, s.actAmp, s.actFreq, s.rtimeIn[rob] + dt, s.vphase[i]);
+}
+
 /* contacts in partner order (VX_Voxel.cpp:250-253), each pair's force from voxel i's side as the
    split step's contact kernel forms it */
-__device__ __forceinline__ void subtract_contacts(const FusedPtrs& s, const VoxMat& m, int i, float tempI, float tnow,
-                                                  dvec& t) {
+__device__ __forceinline__ void subtract_contacts(const FusedPtrs& s, const VoxMat& m, int i, float tempI, dvec& t) {
     if (!s.colCnt) return;
     const int nv = s.nv;
     const int cnt = s.colCnt[i], off = s.colOff[i];
@@ -212,9 +226,7 @@ __device__ __forceinline__ void subtract_contacts(const FusedPtrs& s, const VoxM
     const ContactSelf me = contact_self(m, s.vdIn, nv, i, tempI);
     for (int c = 0; c < cnt; c++) {
         const int j = s.partners[off + c];
-        const float tj = s.vphase ? actuation_temperature(s.actBase, s.actAmp, s.actFreq, tnow, s.vphase[j])
-                                  : s.vtemp[j];
-        const fvec f = contact_pair_force(me, s.vmats[s.vmat[j]], s.vdIn, nv, j, tj);
+        const fvec f = contact_pair_force(me, s.vmats[s.vmat[j]], s.vdIn, nv, j, s.vtempIn[j]);
         t.x -= f.x; t.y -= f.y; t.z -= f.z;
     }
 }
@@ -251,6 +263,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(VX_FUS
             return;
         }
         prevDt = s.k == 0 ? s.rprev[rob] : dt;
+        next_temperature(s, i, rob, dt);
         if (i == 0 || s.vrobot[i - 1] != rob) s.rtimeOut[rob] = s.rtimeIn[rob] + dt; /* currentTime += dt */
         /* here, before the link loop, where few registers are live; read back further down */
         if (Driven) apply_ramp(s.exts, s.ramps, s.vext[i], s.rtimeIn[rob]);
@@ -259,14 +272,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(VX_FUS
     const dvec pos0 = dv(vd[VPX * nv + i], vd[VPY * nv + i], vd[VPZ * nv + i]);
     const dquat q0 = dq(vd[VQW * nv + i], vd[VQX * nv + i], vd[VQY * nv + i], vd[VQZ * nv + i]);
     const int mi = s.vmat[i];
-    const float tnow = s.rtimeIn[rob];
-    float tempI;
-    if (s.vphase) {
-        tempI = actuation_temperature(s.actBase, s.actAmp, s.actFreq, tnow, s.vphase[i]);
-        if (!ForcesOnly) s.vtemp[i] = tempI;
-    } else {
-        tempI = s.vtemp[i];
-    }
+    const float tempI = s.vtempIn[i];
 
     /* force() and moment() (VX_Voxel.cpp:234-271): the end vectors of the links in direction
        order 0..5, each link evaluated as CVX_Link::updateForces (VX_Link.cpp:149-217) */
@@ -284,10 +290,10 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(VX_FUS
         LinkIn in;
         if ((dir & 1) == 0) {
             link_load<true, Poisson>(s, i, o, dir, in);
-            link_end<ForcesOnly, true, Poisson, false>(s, in, i, o, mi, dir, rob, prevDt, tnow, tempI, pos0, q0, f, mm);
+            link_end<ForcesOnly, true, Poisson, false>(s, in, i, o, mi, dir, rob, prevDt, tempI, pos0, q0, f, mm);
         } else {
             link_load<false, Poisson>(s, i, o, dir, in);
-            link_end<ForcesOnly, false, Poisson, false>(s, in, i, o, mi, dir, rob, prevDt, tnow, tempI, pos0, q0, f, mm);
+            link_end<ForcesOnly, false, Poisson, false>(s, in, i, o, mi, dir, rob, prevDt, tempI, pos0, q0, f, mm);
         }
         sf.x += f.x; sf.y += f.y; sf.z += f.z;
         sm.x += mm.x; sm.y += mm.y; sm.z += mm.z;
@@ -316,7 +322,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(VX_FUS
     dvec ang = dv(ld_nt(&vd[VAX * nv + iv]), ld_nt(&vd[VAY * nv + iv]), ld_nt(&vd[VAZ * nv + iv]));
     dquat q = q0;
     voxel_step_fp64(m, ex, s.vijk, nv, iv, dt, tempI, sf, sm, pos, lin, ang, q, flags,
-                    [&](dvec& t) { subtract_contacts(s, m, iv, tempI, tnow, t); });
+                    [&](dvec& t) { subtract_contacts(s, m, iv, tempI, t); });
     store_voxel(s.vdOut, nv, iv, pos, lin, ang, q);
     st_nt(&s.vflOut[iv], flags & ~(uint32_t)VF_PS_VALID); /* poissonsStrainInvalid = true (VX_Voxel.cpp:231) */
     if (Driven && s.haltTest) halt_if_stale(s.halt, s.k + 1, s.colLast, s.recalcSq, s.vflIn, nv, iv, pos.x, pos.y, pos.z);
@@ -370,7 +376,7 @@ __global__ void __launch_bounds__(6 / PerWave * kEndsTile) __attribute__((amdgpu
         mi = s.vmat[i];
         pos0 = dv(vd[VPX * nv + i], vd[VPY * nv + i], vd[VPZ * nv + i]);
         q0 = dq(vd[VQW * nv + i], vd[VQX * nv + i], vd[VQY * nv + i], vd[VQZ * nv + i]);
-        tempI = s.vtemp[i];
+        tempI = s.vtempIn[i];
         if (wave < 2) {
             mom = dv(vd[(VLX + c0) * nv + i], vd[(VLY + c0) * nv + i], vd[(VLZ + c0) * nv + i]);
             ei = s.vext[i];
@@ -406,15 +412,11 @@ __global__ void __launch_bounds__(6 / PerWave * kEndsTile) __attribute__((amdgpu
             mi = s.vmat[i];
             pos0 = dv(vd[VPX * nv + i], vd[VPY * nv + i], vd[VPZ * nv + i]);
             q0 = dq(vd[VQW * nv + i], vd[VQX * nv + i], vd[VQY * nv + i], vd[VQZ * nv + i]);
-            tempI = s.vtemp[i];
+            tempI = s.vtempIn[i];
             dt = s.rdt[rob];
             tnow = s.rtimeIn[rob];
         }
         const float prevDt = s.k == 0 ? s.rprev[rob] : dt;
-        if (s.vphase) {
-            tempI = actuation_temperature(s.actBase, s.actAmp, s.actFreq, tnow, s.vphase[i]);
-            if (wave == 0) s.vtemp[i] = tempI;
-        }
 #pragma unroll 1
         for (int dir = PerWave * wave; dir < PerWave * (wave + 1); dir++) {
             if (PerWave > 1) o = s.vnbr[dir * nv + i];
@@ -423,10 +425,10 @@ __global__ void __launch_bounds__(6 / PerWave * kEndsTile) __attribute__((amdgpu
                 LinkIn in;
                 if ((dir & 1) == 0) {
                     link_load<true, Poisson>(s, i, o, dir, in);
-                    link_end<false, true, Poisson, true>(s, in, i, o, mi, dir, rob, prevDt, tnow, tempI, pos0, q0, f, mm);
+                    link_end<false, true, Poisson, true>(s, in, i, o, mi, dir, rob, prevDt, tempI, pos0, q0, f, mm);
                 } else {
                     link_load<false, Poisson>(s, i, o, dir, in);
-                    link_end<false, false, Poisson, true>(s, in, i, o, mi, dir, rob, prevDt, tnow, tempI, pos0, q0, f, mm);
+                    link_end<false, false, Poisson, true>(s, in, i, o, mi, dir, rob, prevDt, tempI, pos0, q0, f, mm);
                 }
             } else if (s.storeForces) {
                 for (int c = 0; c < 6; c++) s.vf[vf_index(dir, c, nv, i)] = 0.0;
@@ -436,7 +438,9 @@ __global__ void __launch_bounds__(6 / PerWave * kEndsTile) __attribute__((amdgpu
         }
     }
     __syncthreads();
-    if (wave > 1 || !live) return;
+    if (!live) return;
+    if (wave == 2) next_temperature(s, i, rob, dt);
+    if (wave > 1) return;
     if (PerWave > 1) {
         mom = dv(vd[(VLX + c0) * nv + i], vd[(VLY + c0) * nv + i], vd[(VLZ + c0) * nv + i]);
         ei = s.vext[i];
@@ -474,12 +478,25 @@ __global__ void __launch_bounds__(6 / PerWave * kEndsTile) __attribute__((amdgpu
     }
     dvec pos = pos0, lin = mom;
     voxel_translate_fp64(m, ex, dt, tempI, sum, q0, pos, lin, flags,
-                         [&](dvec& t) { subtract_contacts(s, m, i, tempI, tnow, t); });
+                         [&](dvec& t) { subtract_contacts(s, m, i, tempI, t); });
     if (ex) voxel_fix_translation(m, ex, s.vijk, nv, i, pos, lin);
     out[VPX * nv + i] = pos.x; out[VPY * nv + i] = pos.y; out[VPZ * nv + i] = pos.z;
     out[VLX * nv + i] = lin.x; out[VLY * nv + i] = lin.y; out[VLZ * nv + i] = lin.z;
     s.vflOut[i] = flags & ~(uint32_t)VF_PS_VALID; /* poissonsStrainInvalid = true (VX_Voxel.cpp:231) */
     if (Driven && s.haltTest) halt_if_stale(s.halt, s.k + 1, s.colLast, s.recalcSq, s.vflIn, nv, i, pos.x, pos.y, pos.z);
+}
+
+/* temperatures at each robot's current time, before the first step of an actuated launch (robots
+   that do not step keep theirs, which the other half holds if `moved`) */
+__global__ void __launch_bounds__(256) k_fused_temps(FusedPtrs s, int moved) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= s.nv) return;
+    const int rob = s.vrobot[i];
+    if (s.rdiv[rob] < 0) {
+        if (moved) s.vtempIn[i] = s.vtempOut[i];
+        return;
+    }
+    s.vtempIn[i] = actuation_temperature(s.actBase, s.actAmp, s.actFreq, s.rtimeIn[rob], s.vphase[i]);
 }
 
 /* after a launch: previousDt of every voxel whose robot completed at least one step */
@@ -550,6 +567,10 @@ void launch_step_fp64_ends(const FusedPtrs& s, hipStream_t st) {
     else { VX_ENDS64_W(2) }
 #undef VX_ENDS64_W
 #undef VX_ENDS64
+}
+void launch_fused_temps(const FusedPtrs& s, bool moved, hipStream_t st) {
+    if (s.nv > 0)
+        hipLaunchKernelGGL(k_fused_temps, dim3((unsigned)((s.nv + 255) / 256)), dim3(256), 0, st, s, moved ? 1 : 0);
 }
 void launch_fused_prevdt(const int* vrobot, const int* rdiv, const float* rdt, float* vprevdt, int nv, hipStream_t st) {
     if (nv > 0)

@@ -13,6 +13,7 @@ namespace vx {
 
 void launch_step_fp64(const FusedPtrs& s, int block, bool forcesOnly, hipStream_t st);
 void launch_step_fp64_ends(const FusedPtrs& s, hipStream_t st);
+void launch_fused_temps(const FusedPtrs& s, bool moved, hipStream_t st);
 void launch_fused_prevdt(const int* vrobot, const int* rdiv, const float* rdt, float* vprevdt, int nv, hipStream_t st);
 void launch_fused_restore(double* vd, const double* vdPrev, uint32_t* vfl, const uint32_t* vflPrev, float* vtemp,
                           const float* vtempPrev, float* rtime, const float* rtimePrev, int nv, int first, int count,
@@ -31,13 +32,19 @@ uint64_t graph_key(const void* args, size_t n, int path, int nsteps, int flags);
 /* the "out" half of the voxel and link state, and the saved link state of diverged robots */
 bool Sim::fusedFp64Buffers() {
     const size_t vc = (size_t)std::max(nv(), 1), sc = 3 * vc;
-    if (!bvdAlt.ensure((size_t)VD_COUNT * vc * 8) || !bvflAlt.ensure(vc * 4) || !bldAlt.ensure((size_t)LDEV_COUNT * sc * 8) ||
+    if (!bvdAlt.ensure((size_t)VD_COUNT * vc * 8) || !bvflAlt.ensure(vc * 4) || !bvtempAlt.ensure(vc * 4) || !bldAlt.ensure((size_t)LDEV_COUNT * sc * 8) ||
         !blfAlt.ensure((size_t)LF_COUNT * sc * 4) || !blflAlt.ensure(sc * 4) || !bldSide.ensure((size_t)LDEV_COUNT * sc * 8) ||
         !blfSide.ensure((size_t)LF_COUNT * sc * 4) || !blflSide.ensure(sc * 4)) {
         err = "device allocation failed";
         return false;
     }
     return true;
+}
+
+void Sim::swapTemps() {
+    std::swap(bvtemp.p, bvtempAlt.p);
+    std::swap(bvtemp.bytes, bvtempAlt.bytes);
+    dp.vtemp = (float*)bvtemp.p;
 }
 
 /* the step's output state becomes the current one */
@@ -48,6 +55,7 @@ void Sim::swapFp64Buffers() {
     };
     sw(bvd, bvdAlt);
     sw(bvflags, bvflAlt);
+    if (actOn) swapTemps(); /* the next step's temperatures (fusedFp64Finish) */
     sw(brtime, brtimeAlt);
     sw(bld, bldAlt);
     sw(blf, blfAlt);
@@ -80,7 +88,6 @@ bool Sim::stepFp64Fused(int nsteps) {
     fp.vmat = dp.vmat;
     fp.vext = dp.vext;
     fp.vijk = dp.vijk;
-    fp.vtemp = dp.vtemp;
     fp.vmats = dp.vmats;
     fp.lmats = dp.lmats;
     fp.nvmats = (int)vmats.size();
@@ -106,6 +113,8 @@ bool Sim::stepFp64Fused(int nsteps) {
         a.vdOut = (double*)bvdAlt.p;
         a.vflIn = dp.vflags;
         a.vflOut = (uint32_t*)bvflAlt.p;
+        a.vtempIn = dp.vtemp;
+        a.vtempOut = (float*)bvtempAlt.p;
         a.ldIn = dp.ld;
         a.ldOut = (double*)bldAlt.p;
         a.lfIn = dp.lf;
@@ -136,6 +145,14 @@ bool Sim::stepFp64Fused(int nsteps) {
     bool allLinear = true;
     for (const auto& m : lmats) allLinear = allLinear && m->linear;
     fp.offsetConst = allLinear && nsteps >= 4 && nv() > 0 ? 1 : 0;
+    if (actOn) {
+        /* temperatures at the robots' current times, in the half that goes with the state's, so
+           that launches of one length and parity replay one graph */
+        const bool moved = (bvtemp.p > bvtempAlt.p) != (bvd.p > bvdAlt.p);
+        if (moved) swapTemps();
+        bind(fp);
+        launch_fused_temps(fp, moved, stream);
+    }
     uint64_t key = 0;
     if (graph) {
         FusedPtrs k0 = fp;
@@ -202,6 +219,7 @@ bool Sim::stepFp64Fused(int nsteps) {
         fp.colLast = collisions ? cp.last : nullptr;
         fp.recalcSq = cp.recalcSq;
         fp.storeForces = (k == nsteps - 1 || lastStep) ? 1 : 0;
+        fp.tempNext = k < nsteps - 1 && !lastStep ? 1 : 0;
         const LaunchCfg cfg = tune ? tuner[3].next(&cand[k]) : chosen;
         fp.xcd = cfg.xcd;
         launch_poisson_fp64(dp, k, stream); /* the Poisson strains this step's links read */
@@ -250,6 +268,7 @@ bool Sim::stepFp64Fused(int nsteps) {
    earlier gets the end forces of its diverging step recomputed from its saved link state. */
 bool Sim::fusedFp64Finish(int launched) {
     const int n = nv(), R = nRobots();
+    if (actOn && launched > 0) swapTemps(); /* back to the temperatures of the last step */
     launch_fused_prevdt(dp.vrobot, dp.rdiv, dp.rdt, dp.vprevdt, n, stream);
     HIPCHK(hipGetLastError());
     /* the divergence record and the clocks in one copy: when no robot diverged they are also
@@ -286,7 +305,7 @@ bool Sim::fusedFp64Finish(int launched) {
         fp.vmat = dp.vmat;
         fp.vext = dp.vext;
         fp.vijk = dp.vijk;
-        fp.vtemp = dp.vtemp;
+        fp.vtempIn = dp.vtemp;
         fp.vmats = dp.vmats;
         fp.lmats = dp.lmats;
         fp.curveStrain = dp.curveStrain;

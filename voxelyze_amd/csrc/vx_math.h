@@ -206,13 +206,36 @@ VX_HD void dd_sincos(double x, dd* sn, dd* cs) {
     else { *sn = dd_neg(c); *cs = s; }
 }
 
+/* sin of a double in double-double: dd_sincos's operations for the one series that x's quadrant
+   needs, its coefficients selected per lane (lanes of a wave lie in all quadrants, and both series
+   are 800 operations) */
+VX_HD dd dd_sin(double x) {
+    double kq = rint(x * (1.0 / VX_PIO2_HI));
+    dd p = two_prod(kq, VX_PIO2_HI);
+    dd r = dd_sub(dd_make(x, 0.0), p);
+    r = dd_sub(r, dd_mul_d(dd_make(VX_PIO2_MD, VX_PIO2_LO), kq));
+    dd y = dd_mul(r, r);
+    const int q = ((int)kq) & 3;
+    const bool odd = q & 1; /* the cosine series */
+    const int N = 13;
+    dd s = dd_make(odd ? kInvFact[2 * (N - 1)].hi : kInvFact[2 * N - 1].hi,
+                   odd ? kInvFact[2 * (N - 1)].lo : kInvFact[2 * N - 1].lo);
+    if ((N - 1) & 1) s = dd_neg(s);
+#pragma unroll
+    for (int k = N - 2; k >= 0; k--) {
+        dd c = dd_make(odd ? kInvFact[2 * k].hi : kInvFact[2 * k + 1].hi, odd ? kInvFact[2 * k].lo : kInvFact[2 * k + 1].lo);
+        if (k & 1) c = dd_neg(c);
+        s = dd_add(c, dd_mul(y, s));
+    }
+    if (!odd) s = dd_mul(r, s);
+    return q >= 2 ? dd_neg(s) : s;
+}
+
 /* correctly rounded sin, cos (|x| < 2^20; beyond that the plain libm value) */
 VX_HD_COLD double cr_sin(double x) {
     if (!(fabs(x) < 1048576.0)) return sin(x);
     if (x == 0.0) return x;
-    dd s, c;
-    dd_sincos(x, &s, &c);
-    return s.hi;
+    return dd_sin(x).hi;
 }
 VX_HD_COLD double cr_cos(double x) {
     if (!(fabs(x) < 1048576.0)) return cos(x);

@@ -285,6 +285,7 @@ struct Sim {
     DevBuf bldAlt, blfAlt, blflAlt, bldSide, blfSide, blflSide;
     bool fusedFp64Buffers();
     void swapFp64Buffers();
+    void swapTemps(); /* the halves of the temperatures (actuated FP64 steps) */
     bool stepFp64Fused(int nsteps);
     bool fusedFp64Finish(int launched);
     int stepRobots(const float* dt, int nsteps, int* done, int* divergedAt);
