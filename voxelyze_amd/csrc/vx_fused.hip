@@ -231,11 +231,12 @@ __device__ __forceinline__ void subtract_contacts(const FusedPtrs& s, const VoxM
     }
 }
 
-/* Driven: instances for contact-batch steps (the watch-list test on the positions written) and
-   prescribed-displacement ramps; the others carry neither, and none of their registers. */
+/* Driven: instances for contact-batch steps (the watch-list test on the positions written),
+   prescribed-displacement ramps and actuation; the others carry none of them, nor their registers. */
 template <bool ForcesOnly, bool Poisson, bool MatsLds, bool Driven>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(VX_FUSED64_WAVES, 8))) k_step_fp64(FusedPtrs s0) {
     FusedPtrs s = s0;
+    if (!Driven && !ForcesOnly) s.vphase = nullptr;
     if (MatsLds) {
         __shared__ VoxMat svm[kLdsVoxMats];
         __shared__ LinkMat slm[kLdsLinkMats];
@@ -351,6 +352,7 @@ constexpr int kEndsWideMax = 256 * kEndsTile; /* one workgroup of six waves a CU
 template <int PerWave, bool Poisson, bool MatsLds, bool Driven>
 __global__ void __launch_bounds__(6 / PerWave * kEndsTile) __attribute__((amdgpu_waves_per_eu(PerWave == 1 ? 2 : 3, 8))) k_step_fp64_ends(FusedPtrs s0) {
     FusedPtrs s = s0;
+    if (!Driven) s.vphase = nullptr;
     const int nv = s.nv;
     if (s.halt && s.halt[0] <= s.k) return; /* the whole grid: a halt recorded by this step is k + 1 */
     const int lane = threadIdx.x & (kEndsTile - 1);
@@ -528,7 +530,7 @@ void launch_step_fp64(const FusedPtrs& s, int block, bool forcesOnly, hipStream_
     if (s.nv <= 0) return;
     const dim3 grid((unsigned)((s.nv + block - 1) / block));
     const bool lds = VX_MATS_LDS && !forcesOnly && s.nvmats <= kLdsVoxMats && s.nlmats <= kLdsLinkMats;
-    const bool driven = s.haltTest || s.ramps;
+    const bool driven = s.haltTest || s.ramps || s.vphase;
     if (forcesOnly) {
         if (s.poisson) hipLaunchKernelGGL((k_step_fp64<true, true, false, false>), grid, dim3(block), 0, st, s);
         else hipLaunchKernelGGL((k_step_fp64<true, false, false, false>), grid, dim3(block), 0, st, s);
@@ -551,7 +553,7 @@ void launch_step_fp64_ends(const FusedPtrs& s, hipStream_t st) {
     const int perWave = s.nv <= kEndsWideMax ? 1 : 2;
     const dim3 grid((unsigned)((s.nv + kEndsTile - 1) / kEndsTile)), block(6 / perWave * kEndsTile);
     const bool lds = VX_MATS_LDS && s.nvmats <= kLdsVoxMats && s.nlmats <= kLdsLinkMats;
-    const bool driven = s.haltTest || s.ramps;
+    const bool driven = s.haltTest || s.ramps || s.vphase;
 #define VX_ENDS64(W, P, L)                                                                                \
     if (driven) hipLaunchKernelGGL((k_step_fp64_ends<W, P, L, true>), grid, block, 0, st, s);            \
     else hipLaunchKernelGGL((k_step_fp64_ends<W, P, L, false>), grid, block, 0, st, s)
