@@ -1,5 +1,6 @@
-"""The FP64 step with a voxel's link directions split over the waves of a workgroup
-(k_step_fp64_ends) against the split FP64 step, bit for bit: every size at which its tiling or the
+"""The steps with a voxel's link directions split over the waves of a workgroup, bit for bit:
+k_step_fp64_ends against the split FP64 step, k_step_mixed_ends (mixed and FP64 fused) against
+k_step_mixed, which a pinned launch configuration selects: every size at which its tiling or the
 rule that picks it changes, and its own machinery (divergence, idle robots, contacts, ramps, the
 volumetric terms) in both of its forms."""
 import numpy as np
@@ -8,7 +9,7 @@ import pytest
 import backends as B
 from voxelyze_amd import workloads as W
 
-TILE, WIDE, LARGEST = 64, 16384, 294912   # voxels of a tile; of the widest form; of the kernel at all
+TILE, WIDE = 64, 16384   # voxels of a tile; of the widest form
 
 
 def lattice(path, nv, nu=0.0, bilinear=False):
@@ -41,7 +42,7 @@ def assert_same(a, b, what):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("nv", [1, TILE - 1, TILE, TILE + 1, WIDE, WIDE + 1, LARGEST, LARGEST + 1])
+@pytest.mark.parametrize("nv", [1, TILE - 1, TILE, TILE + 1, WIDE, WIDE + 1, 294912, 294913])
 def test_sizes_at_the_edges(nv):
     print(f"[ends] {nv} voxels", flush=True)
     a, b = lattice(0, nv), lattice(1, nv)
@@ -112,3 +113,86 @@ def test_diverging_and_idle_robots(side, actuated):
     assert [a.robotTime(r) for r in range(4)] == [b.robotTime(r) for r in range(4)]
     assert_same(a, b, "robots")
     assert [a.voxel(i).temperature() for i in (0, 30, f, f + 9)] == [b.voxel(i).temperature() for i in (0, 30, f, f + 9)]
+
+
+MIXED, FUSED64 = 1, 2
+
+
+def same_bits_pinned(build, precision, run, what):
+    """the form the size picks, and the per-voxel kernel by a pinned launch configuration"""
+    a, b = build(), build()
+    for sim in (a, b):
+        sim.setPrecision(precision)
+    assert b.abi.set_launch_config(b.handle, 0, 64, 0) == 1
+    ra, rb = run(a), run(b)
+    assert np.array_equal(ra, rb), what
+    assert_same(a, b, what)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("precision,nv", [(MIXED, n) for n in (1, TILE + 1, WIDE, WIDE + 1, 368640, 368641)] +
+                         [(FUSED64, n) for n in (TILE - 1, WIDE, WIDE + 1, 131072, 131073)])
+def test_mixed_sizes_at_the_edges(precision, nv):
+    print(f"[ends] precision {precision}, {nv} voxels", flush=True)
+    build = lambda: lattice(0, nv)  # noqa: E731
+
+    def run(sim):
+        dt = sim.recommendedTimeStep()
+        return [sim.step(dt, n) for n in (1, 5, 4)]
+    same_bits_pinned(build, precision, run, f"{nv} voxels")
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("precision", [MIXED, FUSED64])
+@pytest.mark.parametrize("nv", [1000, WIDE + 500])
+@pytest.mark.parametrize("model", ["bilinear", "contacts and ramps", "moduli"])
+def test_mixed_options_in_both_forms(model, nv, precision):
+    print(f"[ends] {model}, {nv} voxels, precision {precision}", flush=True)
+
+    def build():
+        sim = lattice(0, nv, bilinear=model == "bilinear")
+        v = [sim.voxel(i).external() for i in (0, 5, 9, nv - 1)]
+        v[0].setFixedAll()
+        v[1].setFixed(1 | 16)
+        v[2].setForce(0.0, 0.02, 0.5)
+        if model == "contacts and ramps":
+            sim.enableCollisions(True)
+            v[3].setDisplacementRamp((0.0, 0.0, 0.0), (0.0, 0.0, -3.0))
+        if model == "moduli":
+            sim.setModuli(np.linspace(5e5, 2e6, nv))
+        return sim
+
+    def run(sim):
+        dt = 0.3 * sim.recommendedTimeStep()
+        return [sim.step(dt, n) for n in (1, 90, 40)]
+    same_bits_pinned(build, precision, run, model)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("precision", [MIXED, FUSED64])
+@pytest.mark.parametrize("side", [6, 26])
+def test_mixed_diverging_and_idle_robots(side, precision):
+    print(f"[ends] robots beside a {side}^3 block, precision {precision}", flush=True)
+
+    def build():
+        sim = B.maker(B.product_abi(), 0)(0.005)
+        mats = W.robot_materials(sim)
+        sim.setGravity(1.0)
+        sim.enableFloor(True)
+        for r, (n, mat) in enumerate(((3, 2), (side, 3), (4, 0), (3, 1))):
+            if r:
+                sim.addRobot()
+            g = np.arange(n ** 3)
+            sim.setVoxels(np.full(n ** 3, mats[mat].index, np.int32), np.stack([g % n, (g // n) % n, g // n ** 2], 1))
+        sim.setActuation(True, 0.0, 20.0, 2.0)
+        sim.setPhases(np.linspace(0.0, 6.0, sim.voxelCount()))
+        f, _ = sim.robotVoxels(2)
+        sim.voxel(f).external().setForce(1e4, 0.0, 0.0)
+        return sim
+
+    def run(sim):
+        dt = np.array([sim.robotRecommendedTimeStep(r) for r in range(4)], np.float32)
+        dt[3] = 0.0
+        done = [sim.robotStep(n, dt) for n in (7, 60, 1)]
+        return np.array(done + [[sim.robotTime(r) for r in range(4)], [sim.voxel(i).temperature() for i in (0, 30, 40, 60)]])
+    same_bits_pinned(build, precision, run, "robots")

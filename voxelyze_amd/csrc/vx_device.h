@@ -192,6 +192,19 @@ __device__ __forceinline__ void st_nt(T* p, T v) { __builtin_nontemporal_store(v
 template <class T>
 __device__ __forceinline__ T ld_nt(const T* p) { return __builtin_nontemporal_load(p); }
 
+/* the step's output link state: past the caches, or through them where the next step's reads of
+   the same workgroup find it there (a model whose state the L2s hold) */
+template <bool Cached, class T>
+__device__ __forceinline__ void put(T* p, T v) {
+    if (Cached) *p = v;
+    else st_nt(p, v);
+}
+
+/* the step kernels that split a voxel's link directions over waves take tiles of 64 voxels; their
+   widest form has one wave for each of the six, and one such workgroup finds room on a CU */
+constexpr int kEndsTile = 64;
+constexpr int kEndsWideMax = 256 * kEndsTile;
+
 /* The watch list's stale test (CVoxelyze::updateCollisions, src/Voxelyze.cpp:686-696) made by
    the step of a contact batch on the position it leaves for voxel i (the position the next
    step starts from): if a surface voxel moved farther than recalcDist since the last rebuild,

@@ -75,14 +75,6 @@ __device__ __forceinline__ double axis_size(const VoxMat& m, int axis) {
     return axis == 0 ? m.sizeX : axis == 1 ? m.sizeY : m.sizeZ;
 }
 
-/* the step's output link state: past the caches, or through them where the next step's reads of
-   the same workgroup find it there (a model whose state the L2s hold) */
-template <bool Cached, class T>
-__device__ __forceinline__ void put(T* p, T v) {
-    if (Cached) *p = v;
-    else st_nt(p, v);
-}
-
 /* what one end of a link reads: the neighbour's pose and material, the link's material and state */
 struct LinkIn {
     int meta, mo;
@@ -347,8 +339,6 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(VX_FUS
    The blocks map to the XCDs in contiguous ranges and the stores go through the caches, so that
    the next step finds a tile's state, and most of its neighbours', in the same L2 (45,352 voxels:
    15.9 linear and non-temporal, 15.0 contiguous, 13.8 contiguous and cached). */
-constexpr int kEndsTile = 64;
-constexpr int kEndsWideMax = 256 * kEndsTile; /* one workgroup of six waves a CU */
 template <int PerWave, bool Poisson, bool MatsLds, bool Driven>
 __global__ void __launch_bounds__(6 / PerWave * kEndsTile) __attribute__((amdgpu_waves_per_eu(PerWave == 1 ? 2 : 3, 8))) k_step_fp64_ends(FusedPtrs s0) {
     FusedPtrs s = s0;

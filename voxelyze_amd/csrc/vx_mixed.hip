@@ -155,28 +155,66 @@ template <> __device__ __forceinline__ BeamK<double> beam_of_moduli<double>(floa
     return k;
 }
 
+/* What one end of a link reads: the neighbour's pose, temperature and material, the link's
+   material and state.  Early 2: all asked for together, so that the link's arithmetic waits once
+   (the six-wave form, which has registers to spare); 1: all but the link's previous pose (the
+   three-wave form in float: 44 us a step at 235,932 voxels, 58 with Early 0); 0: each where it is
+   used (the per-voxel kernel: 180 us on the 1M-site lattice, 212 with Early 1; the three-wave form
+   in double: 18.9 us at 45,352 voxels, 21.8 with Early 1, which spills). */
+template <typename T> struct MixIn {
+    int meta, mo;
+    uint32_t fl;
+    T pose[9], maxStrain, strainOffset;
+    double rest;
+    float to;
+    dvec po;
+    dquat qo;
+};
+template <typename T, int Early>
+__device__ __forceinline__ void mix_load(const MixPtrs& s, int slot, int o, MixIn<T>& in) {
+    const int nv = s.nv, S = 3 * nv;
+    const T* ls = (const T*)s.lsIn;
+    const double* __restrict__ vd = s.vdIn;
+    if (Early) {
+        in.meta = s.lmeta[slot];
+        in.fl = s.lflIn[slot];
+        if (Early == 2)
+            for (int c = 0; c < 9; c++) in.pose[c] = ls[c * S + slot];
+        in.maxStrain = ls[MS_MAX * S + slot];
+        in.strainOffset = ls[MS_OFF * S + slot];
+        in.mo = s.vmat[o];
+        if (s.vphase) in.to = s.vtempIn[o];
+    }
+    if (!s.vphase) in.rest = s.lrest[slot];
+    in.po = dv(vd[VPX * nv + o], vd[VPY * nv + o], vd[VPZ * nv + o]);
+    in.qo = dq(vd[VQW * nv + o], vd[VQX * nv + o], vd[VQY * nv + o], vd[VQZ * nv + o]);
+}
+
 /* One link (CVX_Link::updateForces, VX_Link.cpp:149-217): pose extraction in FP64, beam
    forces, damping and link state in T (float: the mixed step; double: the FP64 fused step).
    Returns the force and moment on the requested end (in that voxel's frame) and, when
    owner, the new link state. */
-template <typename T>
-__device__ void link_fused(const MixPtrs& s, int slot, int n, int p, int axis, bool wantPos, bool owner, double rest,
+template <typename T, int Early, bool Cached>
+__device__ __forceinline__ void link_fused(const MixPtrs& s, const MixIn<T>& in, int slot, int n, int p, int mn, int mp,
+                           int axis, bool wantPos, bool owner, double rest,
                            float prevDt, dvec posN, dquat qN, dvec posP, dquat qP, dvec* outF, dvec* outM) {
     const int S = 3 * s.nv;
-    LinkMat m = s.lmats[s.lmeta[slot]];
+    LinkMat m = s.lmats[Early ? in.meta : s.lmeta[slot]];
+    auto mat = [&](int v, int known) -> const VoxMat& { return s.vmats[Early ? known : s.vmat[v]]; };
     if (s.vE) { /* per-voxel moduli: linear link of the harmonic-mean modulus (VX_MaterialLink.cpp:70,121-141) */
-        const LinkK lk = link_constants(combined_modulus(s.vE[n], s.vE[p]), (float)s.vmats[s.vmat[n]].nomSize);
+        const LinkK lk = link_constants(combined_modulus(s.vE[n], s.vE[p]), (float)mat(n, mn).nomSize);
         m.E = lk.E; m.a2 = lk.a2; m.b1 = lk.b1; m.b2 = lk.b2; m.b3 = lk.b3;
         m.sqA1 = lk.sqA1; m.sqA2xIp = lk.sqA2xIp; m.sqB1 = lk.sqB1; m.sqB2xFMp = lk.sqB2xFMp; m.sqB3xIp = lk.sqB3xIp;
         m.linear = 1;
         m.epsilonFail = -1.0f;
     }
     BeamK<T> k = beam_of<T>(m);
-    if (sizeof(T) == 8 && s.vE) k = beam_of_moduli<T>(s.vE[n], s.vE[p], (float)s.vmats[s.vmat[n]].nomSize);
-    uint32_t fl = s.lflIn[slot];
+    if (sizeof(T) == 8 && s.vE) k = beam_of_moduli<T>(s.vE[n], s.vE[p], (float)mat(n, mn).nomSize);
+    uint32_t fl = Early ? in.fl : s.lflIn[slot];
     bool small = (fl & LF_SMALL) != 0, lvv = (fl & LF_LVV) != 0;
     const T* ls = (const T*)s.lsIn;
-    T maxStrain = ls[MS_MAX * S + slot], strainOffset = ls[MS_OFF * S + slot];
+    T maxStrain = Early ? in.maxStrain : ls[MS_MAX * S + slot], strainOffset = Early ? in.strainOffset : ls[MS_OFF * S + slot];
+    auto prev = [&](int c) { return Early == 2 ? in.pose[c] : ls[c * S + slot]; }; /* c < 9 */
 
     /* orientLink in FP64 up to the small quantities */
     dvec d = toAxisX(axis, dv(posP.x - posN.x, posP.y - posN.y, posP.z - posN.z));
@@ -225,14 +263,14 @@ __device__ void link_fused(const MixPtrs& s, int slot, int n, int p, int axis, b
         mN = v3<T>(k.a2 * (a2v.x - a1v.x), -k.b2 * p2.z - k.b3 * (2 * a1v.y + a2v.y), k.b2 * p2.y - k.b3 * (2 * a1v.z + a2v.z));
         mP = v3<T>(k.a2 * (a1v.x - a2v.x), -k.b2 * p2.z - k.b3 * (a1v.y + 2 * a2v.y), k.b2 * p2.y - k.b3 * (a1v.z + 2 * a2v.z));
         if (lvvIn) {
-            const V3<T> dP = v3<T>(T(0.5) * (p2.x - ls[MS_P2X * S + slot]), T(0.5) * (p2.y - ls[MS_P2Y * S + slot]),
-                               T(0.5) * (p2.z - ls[MS_P2Z * S + slot]));
-            const V3<T> d1 = v3<T>(T(0.5) * (a1v.x - ls[MS_A1X * S + slot]), T(0.5) * (a1v.y - ls[MS_A1Y * S + slot]),
-                               T(0.5) * (a1v.z - ls[MS_A1Z * S + slot]));
-            const V3<T> d2 = v3<T>(T(0.5) * (a2v.x - ls[MS_A2X * S + slot]), T(0.5) * (a2v.y - ls[MS_A2Y * S + slot]),
-                               T(0.5) * (a2v.z - ls[MS_A2Z * S + slot]));
-            const float dmN = s.vmats[s.vmat[n]].dampNum / prevDt;
-            const float dmP = s.vmats[s.vmat[p]].dampNum / prevDt;
+            const V3<T> dP = v3<T>(T(0.5) * (p2.x - prev(MS_P2X)), T(0.5) * (p2.y - prev(MS_P2Y)),
+                               T(0.5) * (p2.z - prev(MS_P2Z)));
+            const V3<T> d1 = v3<T>(T(0.5) * (a1v.x - prev(MS_A1X)), T(0.5) * (a1v.y - prev(MS_A1Y)),
+                               T(0.5) * (a1v.z - prev(MS_A1Z)));
+            const V3<T> d2 = v3<T>(T(0.5) * (a2v.x - prev(MS_A2X)), T(0.5) * (a2v.y - prev(MS_A2Y)),
+                               T(0.5) * (a2v.z - prev(MS_A2Z)));
+            const float dmN = mat(n, mn).dampNum / prevDt;
+            const float dmP = mat(p, mp).dampNum / prevDt;
             const V3<T> pc = v3<T>(k.sqA1 * dP.x, k.sqB1 * dP.y - k.sqB2xFMp * (d1.z + d2.z), k.sqB1 * dP.z + k.sqB2xFMp * (d1.y + d2.y));
             fN.x += dmN * pc.x; fN.y += dmN * pc.y; fN.z += dmN * pc.z;
             fP.x -= dmP * pc.x; fP.y -= dmP * pc.y; fP.z -= dmP * pc.z;
@@ -266,15 +304,15 @@ __device__ void link_fused(const MixPtrs& s, int slot, int n, int p, int axis, b
     }
     if (owner) {
         T* o = (T*)s.lsOut;
-        st_nt<T>(&o[MS_P2X * S + slot], p2.x); st_nt<T>(&o[MS_P2Y * S + slot], p2.y);
-        st_nt<T>(&o[MS_P2Z * S + slot], p2.z);
-        st_nt<T>(&o[MS_A1X * S + slot], a1v.x); st_nt<T>(&o[MS_A1Y * S + slot], a1v.y);
-        st_nt<T>(&o[MS_A1Z * S + slot], a1v.z);
-        st_nt<T>(&o[MS_A2X * S + slot], a2v.x); st_nt<T>(&o[MS_A2Y * S + slot], a2v.y);
-        st_nt<T>(&o[MS_A2Z * S + slot], a2v.z);
-        st_nt<T>(&o[MS_MAX * S + slot], maxStrain); st_nt<T>(&o[MS_OFF * S + slot], strainOffset);
-        st_nt<T>(&o[MS_STRAIN * S + slot], axialStrain); st_nt<T>(&o[MS_STRESS * S + slot], stress);
-        st_nt(&s.lflOut[slot], (uint32_t)((lvv ? LF_LVV : 0u) | (small ? LF_SMALL : 0u)));
+        put<Cached>(&o[MS_P2X * S + slot], p2.x); put<Cached>(&o[MS_P2Y * S + slot], p2.y);
+        put<Cached>(&o[MS_P2Z * S + slot], p2.z);
+        put<Cached>(&o[MS_A1X * S + slot], a1v.x); put<Cached>(&o[MS_A1Y * S + slot], a1v.y);
+        put<Cached>(&o[MS_A1Z * S + slot], a1v.z);
+        put<Cached>(&o[MS_A2X * S + slot], a2v.x); put<Cached>(&o[MS_A2Y * S + slot], a2v.y);
+        put<Cached>(&o[MS_A2Z * S + slot], a2v.z);
+        put<Cached>(&o[MS_MAX * S + slot], maxStrain); put<Cached>(&o[MS_OFF * S + slot], strainOffset);
+        put<Cached>(&o[MS_STRAIN * S + slot], axialStrain); put<Cached>(&o[MS_STRESS * S + slot], stress);
+        put<Cached>(&s.lflOut[slot], (uint32_t)((lvv ? LF_LVV : 0u) | (small ? LF_SMALL : 0u)));
         if (axialStrain > 100) {
             atomicMin(&s.rdiv[s.vrobot[n]], s.k);
             atomicOr(&s.ctl[0], 1);
@@ -310,121 +348,76 @@ __device__ void frozen_copy(const MixPtrs& s, int i, int rob, int d) {
     }
 }
 
-#ifndef VX_FUSED_WAVES
-#define VX_FUSED_WAVES 3
-#endif
-/* (Staging the material tables in LDS, as the FP64 step does, made this kernel 50 % slower on
-   the drop lattice at the same registers and occupancy: 192 -> 291 us.) */
-/* Batch: instances for contact-batch steps whose successor is in the batch, which test the
-   watch list on the positions they write; the others carry no part of that test. */
-template <typename T, bool Batch>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(VX_FUSED_WAVES, 8))) k_step_mixed(MixPtrs s) {
-    const int i = lane_index(s.xcd);
+/* voxel i's end of its link in direction dir to neighbour o: end force f and moment mm */
+template <typename T, int Early, bool Cached>
+__device__ __forceinline__ void mix_end(const MixPtrs& s, int i, int o, int mi, int dir, int rob, float prevDt, float tempI,
+                                        const dvec& pos0, const dquat& q0, dvec* f, dvec* mm) {
     const int nv = s.nv;
-    if (i >= nv) return;
-    if (s.halt && s.halt[0] <= s.k) return; /* a contact batch halted before this step: nothing moves */
-    const int rob = s.vrobot[i];
-    const int d = s.rdiv[rob];
-    if (d < s.k) {
-        frozen_copy<T>(s, i, rob, d);
-        if (Batch && s.haltTest)
-            halt_if_stale(s.halt, s.k + 1, s.colLast, s.recalcSq, s.vflIn, nv, i, s.vdOut[VPX * nv + i],
-                          s.vdOut[VPY * nv + i], s.vdOut[VPZ * nv + i]);
-        return;
-    }
-    const float dt = s.rdt[rob];
-    const float prevDt = s.k == 0 ? s.rprev[rob] : dt;
-    if (i == 0 || s.vrobot[i - 1] != rob) s.rtimeOut[rob] = s.rtimeIn[rob] + dt; /* currentTime += dt */
-    const double* __restrict__ vd = s.vdIn;
-    const dvec pos0 = dv(vd[VPX * nv + i], vd[VPY * nv + i], vd[VPZ * nv + i]);
-    const dquat q0 = dq(vd[VQW * nv + i], vd[VQX * nv + i], vd[VQY * nv + i], vd[VQZ * nv + i]);
-    uint32_t flags = s.vflIn[i];
-    const float tempI = s.vtempIn[i];
-    const int mi = s.vmat[i];
-
-    /* link phase for this voxel's <= 6 links, summed in direction order */
-    dvec lf = dv(0.0, 0.0, 0.0), lm = dv(0.0, 0.0, 0.0);
-#pragma unroll 1
-    for (int dir = 0; dir < 6; dir++) {
-        const int o = s.vnbr[dir * nv + i];
-        if (o < 0) continue;
-        const int axis = dir >> 1;
-        const bool neg = (dir & 1) == 0; /* this voxel is the link's negative end */
-        const int slot = neg ? axis * nv + i : axis * nv + o;
-        double rest;
-        if (s.vphase) { /* actuated: rest length from the two temperatures (VX_Link.cpp:137-140) */
-            const VoxMat& mt = s.vmats[mi];
-            const VoxMat& mo = s.vmats[s.vmat[o]];
-            const double si = axis == 0 ? mt.sizeX : axis == 1 ? mt.sizeY : mt.sizeZ;
-            const double so = axis == 0 ? mo.sizeX : axis == 1 ? mo.sizeY : mo.sizeZ;
-            double bi, bo;
-            if (sizeof(T) == 8) {
-                /* FP64 fused step: temperatures and sizes in double, smooth in the phases */
-                const double tn = s.rtimeIn[rob];
-                const double ti = fused_temperature_fp64(s.actBase, s.actAmp, s.actFreq, tn, s.vphase[i]);
-                const double to = fused_temperature_fp64(s.actBase, s.actAmp, s.actFreq, tn, s.vphase[o]);
-                bi = si * (1.0 + ti * (double)mt.alphaCTE);
-                bo = so * (1.0 + to * (double)mo.alphaCTE);
-            } else {
-                bi = base_size(si, tempI, mt.alphaCTE);
-                bo = base_size(so, s.vtempIn[o], mo.alphaCTE);
-            }
-            rest = neg ? 0.5 * (bi + bo) : 0.5 * (bo + bi);
+    const int axis = dir >> 1;
+    const bool neg = (dir & 1) == 0; /* this voxel is the link's negative end */
+    const int slot = neg ? axis * nv + i : axis * nv + o;
+    MixIn<T> in;
+    mix_load<T, Early>(s, slot, o, in);
+    double rest = in.rest;
+    if (s.vphase) { /* actuated: rest length from the two temperatures (VX_Link.cpp:137-140) */
+        const VoxMat& mt = s.vmats[mi];
+        const VoxMat& mo = s.vmats[Early ? in.mo : s.vmat[o]];
+        const double si = axis == 0 ? mt.sizeX : axis == 1 ? mt.sizeY : mt.sizeZ;
+        const double so = axis == 0 ? mo.sizeX : axis == 1 ? mo.sizeY : mo.sizeZ;
+        double bi, bo;
+        if (sizeof(T) == 8) {
+            /* FP64 fused step: temperatures and sizes in double, smooth in the phases */
+            const double tn = s.rtimeIn[rob];
+            const double ti = fused_temperature_fp64(s.actBase, s.actAmp, s.actFreq, tn, s.vphase[i]);
+            const double to = fused_temperature_fp64(s.actBase, s.actAmp, s.actFreq, tn, s.vphase[o]);
+            bi = si * (1.0 + ti * (double)mt.alphaCTE);
+            bo = so * (1.0 + to * (double)mo.alphaCTE);
         } else {
-            rest = s.lrest[slot];
+            bi = base_size(si, tempI, mt.alphaCTE);
+            bo = base_size(so, Early ? in.to : s.vtempIn[o], mo.alphaCTE);
         }
-        const dvec po = dv(vd[VPX * nv + o], vd[VPY * nv + o], vd[VPZ * nv + o]);
-        const dquat qo = dq(vd[VQW * nv + o], vd[VQX * nv + o], vd[VQY * nv + o], vd[VQZ * nv + o]);
-        dvec f, mm;
-        /* one call site: the negative end first */
-        link_fused<T>(s, slot, neg ? i : o, neg ? o : i, axis, !neg, neg, rest, prevDt, neg ? pos0 : po, neg ? q0 : qo,
-                      neg ? po : pos0, neg ? qo : q0, &f, &mm);
-        lf.x += f.x; lf.y += f.y; lf.z += f.z;
-        lm.x += mm.x; lm.y += mm.y; lm.z += mm.z;
+        rest = neg ? 0.5 * (bi + bo) : 0.5 * (bo + bi);
     }
-    if (s.vphase) s.vtempOut[i] = fused_actuation(s.actBase, s.actAmp, s.actFreq, s.rtimeIn[rob] + dt, s.vphase[i]);
-    if (s.tapeSums) {
-        double* ts = s.tapeSums;
-        ts[i] = lf.x; ts[nv + i] = lf.y; ts[2 * nv + i] = lf.z;
-        ts[3 * nv + i] = lm.x; ts[4 * nv + i] = lm.y; ts[5 * nv + i] = lm.z;
-    }
+    /* one call site: the negative end first */
+    link_fused<T, Early, Cached>(s, in, slot, neg ? i : o, neg ? o : i, neg ? mi : in.mo, neg ? in.mo : mi, axis, !neg, neg, rest, prevDt,
+                  neg ? pos0 : in.po, neg ? q0 : in.qo, neg ? in.po : pos0, neg ? in.qo : q0, f, mm);
+}
 
-    VoxMat m = s.vmats[mi];
-    if (s.vE) voxel_modulus(&m, s.vE[i]);
-    /* the voxel's modulus-dependent constants; the FP64 fused step forms a per-voxel modulus's
-       in double, as it does the links', so that its loss is smooth in the moduli */
-    const bool smoothE = sizeof(T) == 8 && s.vE;
-    double cGT = m.globalTransC, cGR = m.globalRotC, cCT = m.collisionTransC, kPen = m.penetrationStiff;
-    if (smoothE) {
-        const double E = s.vE[i], L = m.nomSize;
-        const double c = 2.0 * sqrt((double)m.mass * E * L), ci = 2.0 * sqrt((double)m.momentInertia * E * L * L * L);
-        cGT = (double)m.zetaGlobal * c;
-        cCT = (double)m.zetaCollision * c;
-        cGR = (double)m.zetaGlobal * ci;
-        kPen = 2.0 * E * L;
+/* the voxel's modulus-dependent constants; the FP64 fused step forms a per-voxel modulus's in
+   double, as it does the links', so that its loss is smooth in the moduli */
+struct MixVox {
+    VoxMat m;
+    bool smoothE;
+    double cGT, cGR, cCT, kPen;
+};
+template <typename T>
+__device__ __forceinline__ MixVox mix_vox(const MixPtrs& s, int i, int mi) {
+    MixVox v;
+    v.m = s.vmats[mi];
+    if (s.vE) voxel_modulus(&v.m, s.vE[i]);
+    v.smoothE = sizeof(T) == 8 && s.vE;
+    v.cGT = v.m.globalTransC; v.cGR = v.m.globalRotC; v.cCT = v.m.collisionTransC; v.kPen = v.m.penetrationStiff;
+    if (v.smoothE) {
+        const double E = s.vE[i], L = v.m.nomSize;
+        const double c = 2.0 * sqrt((double)v.m.mass * E * L), ci = 2.0 * sqrt((double)v.m.momentInertia * E * L * L * L);
+        v.cGT = (double)v.m.zetaGlobal * c;
+        v.cCT = (double)v.m.zetaCollision * c;
+        v.cGR = (double)v.m.zetaGlobal * ci;
+        v.kPen = 2.0 * E * L;
     }
-    const int e = s.vext[i];
-    const ExtRec* ex = e >= 0 ? &s.exts[e] : nullptr;
-    double* __restrict__ out = s.vdOut;
-    if (ex && (ex->dof & 0x3F) == 0x3F) {
-        const double sz = m.nomSize;
-        out[VPX * nv + i] = s.vijk[i] * sz + ex->tx;
-        out[VPY * nv + i] = s.vijk[nv + i] * sz + ex->ty;
-        out[VPZ * nv + i] = s.vijk[2 * nv + i] * sz + ex->tz;
-        out[VQW * nv + i] = ex->qw; out[VQX * nv + i] = ex->qx; out[VQY * nv + i] = ex->qy; out[VQZ * nv + i] = ex->qz;
-        out[VLX * nv + i] = 0.0; out[VLY * nv + i] = 0.0; out[VLZ * nv + i] = 0.0;
-        out[VAX * nv + i] = 0.0; out[VAY * nv + i] = 0.0; out[VAZ * nv + i] = 0.0;
-        s.vflOut[i] = flags;
-        if (Batch && s.haltTest)
-            halt_if_stale(s.halt, s.k + 1, s.colLast, s.recalcSq, s.vflIn, nv, i, out[VPX * nv + i], out[VPY * nv + i],
-                          out[VPZ * nv + i]);
-        return;
-    }
-    /* the momenta only this lane reads: loaded past the caches */
-    dvec pos = pos0, lin = dv(ld_nt(&vd[VLX * nv + i]), ld_nt(&vd[VLY * nv + i]), ld_nt(&vd[VLZ * nv + i]));
-    dvec ang = dv(ld_nt(&vd[VAX * nv + i]), ld_nt(&vd[VAY * nv + i]), ld_nt(&vd[VAZ * nv + i]));
-    dquat q = q0;
+    return v;
+}
 
+/* the translation of one voxel from its link force sum on, in place (VX_Voxel.cpp:174-196) */
+template <typename T>
+__device__ __forceinline__ void mix_translate(const MixPtrs& s, const MixVox& v, const ExtRec* ex, int i, int rob, float dt,
+                                              float tempI, const dvec& lf, const dquat& q, dvec& pos, dvec& lin,
+                                              uint32_t& flags) {
+    const int nv = s.nv;
+    const double* __restrict__ vd = s.vdIn;
+    const VoxMat& m = v.m;
+    const double cGT = v.cGT, cCT = v.cCT, kPen = v.kPen;
+    const bool smoothE = v.smoothE;
     dvec t = qrot(q, lf);
     if (ex) { t.x += ex->fx; t.y += ex->fy; t.z += ex->fz; }
     t.x -= cGT * (m.massInverse * lin.x);
@@ -533,7 +526,12 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(VX_FUS
         flags &= ~VF_STATIC;
     }
     pos.x += trn.x; pos.y += trn.y; pos.z += trn.z;
+}
 
+/* its rotation from the link moment sum on (VX_Voxel.cpp:198-208) */
+__device__ __forceinline__ void mix_rotate(const MixVox& v, const ExtRec* ex, float dt, const dvec& lm, dvec& ang, dquat& q) {
+    const VoxMat& m = v.m;
+    const double cGR = v.cGR;
     dvec mo = qrot(q, lm);
     if (ex) { mo.x += ex->mx; mo.y += ex->my; mo.z += ex->mz; }
     mo.x -= cGR * (m.momentInertiaInverse * ang.x);
@@ -542,24 +540,129 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(VX_FUS
     ang.x += dt * mo.x; ang.y += dt * mo.y; ang.z += dt * mo.z;
     const float dti = dt * m.momentInertiaInverse;
     q = qmul(d_fromrv(dv(dti * ang.x, dti * ang.y, dti * ang.z)), q);
-    if (ex) {
-        const double sz = m.nomSize;
-        const int dof = ex->dof;
-        if (dof & 1) { pos.x = s.vijk[i] * sz + ex->tx; lin.x = 0.0; }
-        if (dof & 2) { pos.y = s.vijk[nv + i] * sz + ex->ty; lin.y = 0.0; }
-        if (dof & 4) { pos.z = s.vijk[2 * nv + i] * sz + ex->tz; lin.z = 0.0; }
-        if (dof & 56) {
-            if ((dof & 56) == 56) {
-                q = dq(ex->qw, ex->qx, ex->qy, ex->qz);
-                ang = dv(0.0, 0.0, 0.0);
-            } else {
-                dvec rv = d_torv(q);
-                if (dof & 8) { rv.x = 0.0; ang.x = 0.0; }
-                if (dof & 16) { rv.y = 0.0; ang.y = 0.0; }
-                if (dof & 32) { rv.z = 0.0; ang.z = 0.0; }
-                q = d_fromrv(rv);
-            }
+}
+
+/* partial dof fixes (VX_Voxel.cpp:210-228) */
+__device__ __forceinline__ void mix_fix_translation(const MixPtrs& s, const VoxMat& m, const ExtRec* ex, int i, dvec& pos,
+                                                    dvec& lin) {
+    const int nv = s.nv;
+    const double sz = m.nomSize;
+    const int dof = ex->dof;
+    if (dof & 1) { pos.x = s.vijk[i] * sz + ex->tx; lin.x = 0.0; }
+    if (dof & 2) { pos.y = s.vijk[nv + i] * sz + ex->ty; lin.y = 0.0; }
+    if (dof & 4) { pos.z = s.vijk[2 * nv + i] * sz + ex->tz; lin.z = 0.0; }
+}
+__device__ __forceinline__ void mix_fix_rotation(const ExtRec* ex, dvec& ang, dquat& q) {
+    const int dof = ex->dof;
+    if (dof & 56) {
+        if ((dof & 56) == 56) {
+            q = dq(ex->qw, ex->qx, ex->qy, ex->qz);
+            ang = dv(0.0, 0.0, 0.0);
+        } else {
+            dvec rv = d_torv(q);
+            if (dof & 8) { rv.x = 0.0; ang.x = 0.0; }
+            if (dof & 16) { rv.y = 0.0; ang.y = 0.0; }
+            if (dof & 32) { rv.z = 0.0; ang.z = 0.0; }
+            q = d_fromrv(rv);
         }
+    }
+}
+/* a fully fixed voxel sits at its prescribed pose (VX_Voxel.cpp:167-172) */
+__device__ __forceinline__ void mix_pinned(const MixPtrs& s, const VoxMat& m, const ExtRec* ex, int i, double* __restrict__ out) {
+    const int nv = s.nv;
+    const double sz = m.nomSize;
+    out[VPX * nv + i] = s.vijk[i] * sz + ex->tx;
+    out[VPY * nv + i] = s.vijk[nv + i] * sz + ex->ty;
+    out[VPZ * nv + i] = s.vijk[2 * nv + i] * sz + ex->tz;
+    out[VQW * nv + i] = ex->qw; out[VQX * nv + i] = ex->qx; out[VQY * nv + i] = ex->qy; out[VQZ * nv + i] = ex->qz;
+    out[VLX * nv + i] = 0.0; out[VLY * nv + i] = 0.0; out[VLZ * nv + i] = 0.0;
+    out[VAX * nv + i] = 0.0; out[VAY * nv + i] = 0.0; out[VAZ * nv + i] = 0.0;
+}
+
+__device__ __forceinline__ void plain(MixPtrs& s) {
+    s.vE = nullptr;
+    s.vphase = nullptr;
+    s.tapeSums = nullptr;
+    s.colCnt = nullptr;
+}
+
+#ifndef VX_FUSED_WAVES
+#define VX_FUSED_WAVES 3
+#endif
+/* (Staging the material tables in LDS, as the FP64 step does, made this kernel 50 % slower on
+   the drop lattice at the same registers and occupancy: 192 -> 291 us.) */
+/* What bounds it: at 3 waves a SIMD the memory latency of each link end, then the vector unit (45 %
+   busy on the lattice). */
+/* Batch: instances for contact-batch steps whose successor is in the batch, which test the
+   watch list on the positions they write; the others carry no part of that test.
+   Plain: no actuation, per-voxel moduli, contacts or tape, nor their registers (1M-site lattice:
+   193 us a step without this instance, 180 with it). */
+template <typename T, bool Batch, bool Plain>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(VX_FUSED_WAVES, 8))) k_step_mixed(MixPtrs s) {
+    if (Plain) plain(s);
+    const int i = lane_index(s.xcd);
+    const int nv = s.nv;
+    if (i >= nv) return;
+    if (s.halt && s.halt[0] <= s.k) return; /* a contact batch halted before this step: nothing moves */
+    const int rob = s.vrobot[i];
+    const int d = s.rdiv[rob];
+    if (d < s.k) {
+        frozen_copy<T>(s, i, rob, d);
+        if (Batch && s.haltTest)
+            halt_if_stale(s.halt, s.k + 1, s.colLast, s.recalcSq, s.vflIn, nv, i, s.vdOut[VPX * nv + i],
+                          s.vdOut[VPY * nv + i], s.vdOut[VPZ * nv + i]);
+        return;
+    }
+    const float dt = s.rdt[rob];
+    const float prevDt = s.k == 0 ? s.rprev[rob] : dt;
+    if (i == 0 || s.vrobot[i - 1] != rob) s.rtimeOut[rob] = s.rtimeIn[rob] + dt; /* currentTime += dt */
+    const double* __restrict__ vd = s.vdIn;
+    const dvec pos0 = dv(vd[VPX * nv + i], vd[VPY * nv + i], vd[VPZ * nv + i]);
+    const dquat q0 = dq(vd[VQW * nv + i], vd[VQX * nv + i], vd[VQY * nv + i], vd[VQZ * nv + i]);
+    uint32_t flags = s.vflIn[i];
+    const float tempI = s.vtempIn[i];
+    const int mi = s.vmat[i];
+
+    /* link phase for this voxel's <= 6 links, summed in direction order */
+    dvec lf = dv(0.0, 0.0, 0.0), lm = dv(0.0, 0.0, 0.0);
+#pragma unroll 1
+    for (int dir = 0; dir < 6; dir++) {
+        const int o = s.vnbr[dir * nv + i];
+        if (o < 0) continue;
+        dvec f, mm;
+        mix_end<T, 0, false>(s, i, o, mi, dir, rob, prevDt, tempI, pos0, q0, &f, &mm);
+        lf.x += f.x; lf.y += f.y; lf.z += f.z;
+        lm.x += mm.x; lm.y += mm.y; lm.z += mm.z;
+    }
+    if (s.vphase) s.vtempOut[i] = fused_actuation(s.actBase, s.actAmp, s.actFreq, s.rtimeIn[rob] + dt, s.vphase[i]);
+    if (s.tapeSums) {
+        double* ts = s.tapeSums;
+        ts[i] = lf.x; ts[nv + i] = lf.y; ts[2 * nv + i] = lf.z;
+        ts[3 * nv + i] = lm.x; ts[4 * nv + i] = lm.y; ts[5 * nv + i] = lm.z;
+    }
+
+    const MixVox v = mix_vox<T>(s, i, mi);
+    const int e = s.vext[i];
+    const ExtRec* ex = e >= 0 ? &s.exts[e] : nullptr;
+    double* __restrict__ out = s.vdOut;
+    if (ex && (ex->dof & 0x3F) == 0x3F) {
+        mix_pinned(s, v.m, ex, i, out);
+        s.vflOut[i] = flags;
+        if (Batch && s.haltTest)
+            halt_if_stale(s.halt, s.k + 1, s.colLast, s.recalcSq, s.vflIn, nv, i, out[VPX * nv + i], out[VPY * nv + i],
+                          out[VPZ * nv + i]);
+        return;
+    }
+    /* the momenta only this lane reads: loaded past the caches */
+    dvec pos = pos0, lin = dv(ld_nt(&vd[VLX * nv + i]), ld_nt(&vd[VLY * nv + i]), ld_nt(&vd[VLZ * nv + i]));
+    dvec ang = dv(ld_nt(&vd[VAX * nv + i]), ld_nt(&vd[VAY * nv + i]), ld_nt(&vd[VAZ * nv + i]));
+    dquat q = q0;
+
+    mix_translate<T>(s, v, ex, i, rob, dt, tempI, lf, q, pos, lin, flags);
+    mix_rotate(v, ex, dt, lm, ang, q);
+    if (ex) {
+        mix_fix_translation(s, v.m, ex, i, pos, lin);
+        mix_fix_rotation(ex, ang, q);
     }
     st_nt(&out[VPX * nv + i], pos.x); st_nt(&out[VPY * nv + i], pos.y); st_nt(&out[VPZ * nv + i], pos.z);
     st_nt(&out[VLX * nv + i], lin.x); st_nt(&out[VLY * nv + i], lin.y); st_nt(&out[VLZ * nv + i], lin.z);
@@ -567,6 +670,97 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(VX_FUS
     st_nt(&out[VQW * nv + i], q.w); st_nt(&out[VQX * nv + i], q.x); st_nt(&out[VQY * nv + i], q.y);
     st_nt(&out[VQZ * nv + i], q.z);
     st_nt(&s.vflOut[i], flags);
+    if (Batch && s.haltTest) halt_if_stale(s.halt, s.k + 1, s.colLast, s.recalcSq, s.vflIn, nv, i, pos.x, pos.y, pos.z);
+}
+
+/* The same step for models that do not fill the chip (k_step_fp64_ends has the why): a voxel's
+   link directions run side by side in the waves of a workgroup, PerWave to a wave, and meet in
+   LDS; wave 0 integrates the translations, wave 1 the rotations, wave 2 sets the next
+   temperatures.  The same bits as k_step_mixed.  us per step of a two-material lattice,
+   k_step_mixed at its best launch shape -> here, in float: 290 voxels 16.2 -> 6.1, 14,048 voxels
+   17.5 -> 6.2 (PerWave 1), 17,676 voxels 18.0 -> 10.4, 112,451 voxels 29.0 -> 23.8, 332,769 voxels
+   67.7 -> 59.8 (PerWave 2); in double: 290 voxels 19.2 -> 6.8, 45,352 voxels 28.0 -> 18.9. */
+template <typename T, int PerWave, bool Batch, bool Plain>
+__global__ void __launch_bounds__(6 / PerWave * kEndsTile) __attribute__((amdgpu_waves_per_eu(PerWave == 1 ? 2 : 3, 8))) k_step_mixed_ends(MixPtrs s) {
+    if (Plain) plain(s);
+    const int nv = s.nv;
+    if (s.halt && s.halt[0] <= s.k) return; /* the whole grid: a halt recorded by this step is k + 1 */
+    __shared__ T ends[6][6][kEndsTile];
+    const int lane = threadIdx.x & (kEndsTile - 1);
+    const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x / kEndsTile);
+    const int at = xcd_block() * kEndsTile + lane;
+    const int i = at < nv ? at : nv - 1; /* a lane past the end reads the last voxel's */
+    const double* __restrict__ vd = s.vdIn;
+    int o = s.vnbr[PerWave * wave * nv + i];
+    const int rob = s.vrobot[i], mi = s.vmat[i];
+    const dvec pos0 = dv(vd[VPX * nv + i], vd[VPY * nv + i], vd[VPZ * nv + i]);
+    const dquat q0 = dq(vd[VQW * nv + i], vd[VQX * nv + i], vd[VQY * nv + i], vd[VQZ * nv + i]);
+    const float tempI = s.vtempIn[i];
+    const int d = s.rdiv[rob];
+    const float dt = s.rdt[rob];
+    const bool live = at < nv && d >= s.k;
+    if (at < nv && !live && wave == 0) {
+        frozen_copy<T>(s, i, rob, d);
+        if (Batch && s.haltTest)
+            halt_if_stale(s.halt, s.k + 1, s.colLast, s.recalcSq, s.vflIn, nv, i, s.vdOut[VPX * nv + i],
+                          s.vdOut[VPY * nv + i], s.vdOut[VPZ * nv + i]);
+    }
+    if (live) {
+        const float prevDt = s.k == 0 ? s.rprev[rob] : dt;
+#pragma unroll 1
+        for (int dir = PerWave * wave; dir < PerWave * (wave + 1); dir++) {
+            if (PerWave > 1 && dir > PerWave * wave) o = s.vnbr[dir * nv + i];
+            dvec f = dv(0.0, 0.0, 0.0), mm = dv(0.0, 0.0, 0.0);
+            if (o >= 0) mix_end<T, PerWave == 1 ? 2 : sizeof(T) == 4 ? 1 : 0, true>(s, i, o, mi, dir, rob, prevDt, tempI, pos0, q0, &f, &mm);
+            ends[dir][0][lane] = (T)f.x; ends[dir][1][lane] = (T)f.y; ends[dir][2][lane] = (T)f.z;
+            ends[dir][3][lane] = (T)mm.x; ends[dir][4][lane] = (T)mm.y; ends[dir][5][lane] = (T)mm.z;
+        }
+    }
+    __syncthreads();
+    if (!live) return;
+    if (wave == 2 && s.vphase)
+        s.vtempOut[i] = fused_actuation(s.actBase, s.actAmp, s.actFreq, s.rtimeIn[rob] + dt, s.vphase[i]);
+    if (wave > 1) return;
+    const int c0 = 3 * wave;
+    dvec sum = dv(0.0, 0.0, 0.0);
+    for (int e = 0; e < 6; e++) {
+        sum.x += ends[e][c0][lane]; sum.y += ends[e][c0 + 1][lane]; sum.z += ends[e][c0 + 2][lane];
+    }
+    if (s.tapeSums) {
+        double* ts = s.tapeSums + (size_t)c0 * nv;
+        ts[i] = sum.x; ts[nv + i] = sum.y; ts[2 * nv + i] = sum.z;
+    }
+    const MixVox v = mix_vox<T>(s, i, mi);
+    const int e = s.vext[i];
+    const ExtRec* ex = e >= 0 ? &s.exts[e] : nullptr;
+    const bool pinned = ex && (ex->dof & 0x3F) == 0x3F;
+    double* __restrict__ out = s.vdOut;
+    if (wave == 1) {
+        if (pinned) return;
+        dvec ang = dv(vd[VAX * nv + i], vd[VAY * nv + i], vd[VAZ * nv + i]);
+        dquat q = q0;
+        mix_rotate(v, ex, dt, sum, ang, q);
+        if (ex) mix_fix_rotation(ex, ang, q);
+        out[VAX * nv + i] = ang.x; out[VAY * nv + i] = ang.y; out[VAZ * nv + i] = ang.z;
+        out[VQW * nv + i] = q.w; out[VQX * nv + i] = q.x; out[VQY * nv + i] = q.y; out[VQZ * nv + i] = q.z;
+        return;
+    }
+    if (i == 0 || s.vrobot[i - 1] != rob) s.rtimeOut[rob] = s.rtimeIn[rob] + dt; /* currentTime += dt */
+    uint32_t flags = s.vflIn[i];
+    if (pinned) {
+        mix_pinned(s, v.m, ex, i, out);
+        s.vflOut[i] = flags;
+        if (Batch && s.haltTest)
+            halt_if_stale(s.halt, s.k + 1, s.colLast, s.recalcSq, s.vflIn, nv, i, out[VPX * nv + i], out[VPY * nv + i],
+                          out[VPZ * nv + i]);
+        return;
+    }
+    dvec pos = pos0, lin = dv(vd[VLX * nv + i], vd[VLY * nv + i], vd[VLZ * nv + i]);
+    mix_translate<T>(s, v, ex, i, rob, dt, tempI, sum, q0, pos, lin, flags);
+    if (ex) mix_fix_translation(s, v.m, ex, i, pos, lin);
+    out[VPX * nv + i] = pos.x; out[VPY * nv + i] = pos.y; out[VPZ * nv + i] = pos.z;
+    out[VLX * nv + i] = lin.x; out[VLY * nv + i] = lin.y; out[VLZ * nv + i] = lin.z;
+    s.vflOut[i] = flags;
     if (Batch && s.haltTest) halt_if_stale(s.halt, s.k + 1, s.colLast, s.recalcSq, s.vflIn, nv, i, pos.x, pos.y, pos.z);
 }
 
@@ -582,15 +776,35 @@ void launch_mixed_temps(const MixPtrs& s, float* temp, hipStream_t st) {
         hipLaunchKernelGGL(k_mixed_temps, dim3((unsigned)((s.nv + 255) / 256)), dim3(256), 0, st, s, temp);
 }
 
+void launch_step_mixed_ends(const MixPtrs& s, bool fp64, hipStream_t st) {
+    if (s.nv <= 0) return;
+    const int perWave = s.nv <= kEndsWideMax ? 1 : 2;
+    const dim3 grid((unsigned)((s.nv + kEndsTile - 1) / kEndsTile)), block(6 / perWave * kEndsTile);
+    const bool plain = !s.vE && !s.vphase && !s.tapeSums && !s.colCnt;
+#define VX_ENDSMIX(T, B, P)                                                                           \
+    if (perWave == 1) hipLaunchKernelGGL((k_step_mixed_ends<T, 1, B, P>), grid, block, 0, st, s);    \
+    else hipLaunchKernelGGL((k_step_mixed_ends<T, 2, B, P>), grid, block, 0, st, s)
+    if (fp64) {
+        if (s.haltTest) { VX_ENDSMIX(double, true, false); }
+        else { VX_ENDSMIX(double, false, false); }
+    } else {
+        if (s.haltTest) { VX_ENDSMIX(float, true, false); }
+        else if (plain) { VX_ENDSMIX(float, false, true); }
+        else { VX_ENDSMIX(float, false, false); }
+    }
+#undef VX_ENDSMIX
+}
 void launch_step_mixed(const MixPtrs& s, bool fp64, int block, hipStream_t st) {
     if (s.nv <= 0) return;
     const dim3 grid((unsigned)((s.nv + block - 1) / block));
+    const bool plain = !s.vE && !s.vphase && !s.tapeSums && !s.colCnt;
     if (fp64) {
-        if (s.haltTest) hipLaunchKernelGGL((k_step_mixed<double, true>), grid, dim3(block), 0, st, s);
-        else hipLaunchKernelGGL((k_step_mixed<double, false>), grid, dim3(block), 0, st, s);
+        if (s.haltTest) hipLaunchKernelGGL((k_step_mixed<double, true, false>), grid, dim3(block), 0, st, s);
+        else hipLaunchKernelGGL((k_step_mixed<double, false, false>), grid, dim3(block), 0, st, s);
     } else {
-        if (s.haltTest) hipLaunchKernelGGL((k_step_mixed<float, true>), grid, dim3(block), 0, st, s);
-        else hipLaunchKernelGGL((k_step_mixed<float, false>), grid, dim3(block), 0, st, s);
+        if (s.haltTest) hipLaunchKernelGGL((k_step_mixed<float, true, false>), grid, dim3(block), 0, st, s);
+        else if (plain) hipLaunchKernelGGL((k_step_mixed<float, false, true>), grid, dim3(block), 0, st, s);
+        else hipLaunchKernelGGL((k_step_mixed<float, false, false>), grid, dim3(block), 0, st, s);
     }
 }
 

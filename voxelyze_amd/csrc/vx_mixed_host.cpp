@@ -12,6 +12,7 @@
 namespace vx {
 
 void launch_step_mixed(const MixPtrs& s, bool fp64, int block, hipStream_t st);
+void launch_step_mixed_ends(const MixPtrs& s, bool fp64, hipStream_t st);
 void launch_mixed_temps(const MixPtrs& s, float* temp, hipStream_t st);
 uint64_t graph_key(const void* args, size_t n, int path, int nsteps, int flags);
 void launch_col_stale(const DevPtrs& s, const ContactPtrs& c, int gen, hipStream_t st);
@@ -169,7 +170,8 @@ bool Sim::stepMixed(int nsteps, MixTape* tape) {
     mp.actFreq = actFreq;
     mp.vE = modOn ? (const float*)bvE.p : nullptr;
     /* a launch without contacts, tape or timing is recorded as a graph and replayed */
-    const bool tune = tuning(0);
+    const bool ends = endsPath(0, precision == 2 ? kEndsMaxFused64 : kEndsMaxMixed);
+    const bool tune = !ends && tuning(0);
     const bool timed = profiling || tune;
     const bool graph = useGraphs && !collisions && !tape && !timed && nsteps > 1 && nsteps <= 2048;
     const LaunchCfg chosen = tuner[0].chosen;
@@ -191,7 +193,7 @@ bool Sim::stepMixed(int nsteps, MixTape* tape) {
         k0.rtimeIn = dp.rtime; k0.rtimeOut = (float*)brtimeAlt.p;
         k0.lsIn = bms[lcur].p; k0.lsOut = bms[lcur ^ 1].p;
         k0.lflIn = (const uint32_t*)bmfl[lcur].p; k0.lflOut = (uint32_t*)bmfl[lcur ^ 1].p;
-        key = graph_key(&k0, sizeof k0, 1 + precision, nsteps, ((actOn ? 1 : 0) | (chosen.block << 1)) ^ rampKey());
+        key = graph_key(&k0, sizeof k0, (ends ? 8 : 1) + precision, nsteps, ((actOn ? 1 : 0) | (chosen.block << 1)) ^ rampKey());
         bool replayed = false;
         if (!graphLaunch(key, &replayed)) return false;
         if (replayed) { /* the host side of the ping-pong, as the recorded launch left it */
@@ -299,7 +301,8 @@ bool Sim::stepMixed(int nsteps, MixTape* tape) {
         mp.xcd = cfg.xcd;
         launchRamps();
         if (timed) (void)hipEventRecord(events[2 * k], stream);
-        launch_step_mixed(mp, precision == 2, cfg.block, stream);
+        if (ends) launch_step_mixed_ends(mp, precision == 2, stream);
+        else launch_step_mixed(mp, precision == 2, cfg.block, stream);
         if (timed) (void)hipEventRecord(events[2 * k + 1], stream);
         swapVoxelBuffers();
         lcur ^= 1;

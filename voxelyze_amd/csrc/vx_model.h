@@ -258,6 +258,10 @@ struct Sim {
        282,309 voxels 68.2 / 63.4, 332,769 voxels 77.5 / 82.2, 943,896 voxels 226 / 251). */
     bool endsPath(int t, int maxVoxels);
     static constexpr int kEndsMaxFp64 = 294912;
+    /* the mixed step's state is smaller (368,744 voxels: k_step_mixed 69.7, k_step_mixed_ends 69.1;
+       387,158: 73.0 / 75.4), the FP64 fused step's form with three waves runs short of registers
+       (112,451 voxels 41.5 / 38.1, 235,932: 84.8 / 91.1) */
+    static constexpr int kEndsMaxMixed = 368640, kEndsMaxFused64 = 131072;
     /* kernel timing */
     bool profiling = false;
     std::vector<hipEvent_t> events;
