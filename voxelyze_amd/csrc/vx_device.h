@@ -95,12 +95,15 @@ struct LinPtrs {
     const double* xfix;     /* 6 * nv: prescribed values (only where fixed) */
     const double* f;        /* 6 * nv: external force and moment (only where free) */
     double *x, *r, *z, *p, *q;
+    double* pNext;          /* the next search direction where forming it is fused into the product */
     float* minv;            /* 21 * nv: packed lower triangle of the inverse diagonal block */
-    double* part;           /* per-workgroup partial sums, 2 per workgroup */
+    int nblk, per;          /* workgroups of an iteration's kernels, 256-voxel blocks of each */
+    double* part;           /* per-workgroup partial sums, 2 per workgroup: r.z and r.r */
+    double* partQ;          /* p.q */
     double* scal;           /* device scalars, see enum below */
     int* bad;               /* [0] a voxel's diagonal block is singular */
 };
-enum { S_RZ = 0, S_PQ, S_ALPHA, S_BETA, S_RR, S_BB, S_COUNT };
+enum { S_RZ = 0 /* 2: by parity of the iteration */, S_BETA = 2, S_RR, S_BB, S_COUNT };
 
 /* per external record (VX_External.h:93-98) */
 struct ExtRec {

@@ -14,6 +14,8 @@
  * deterministic.  Solution vectors are structure-of-arrays, 6 x nv doubles.
  */
 #include "vx_device.h"
+#include <algorithm>
+
 #include "vx_math.h"
 
 #pragma clang fp contract(off)
@@ -90,17 +92,12 @@ struct Plain {
     int nv;
     __device__ void operator()(int i, double* o) const { load6(a, nv, i, o); }
 };
-/* y_i = (K u)_i over the voxel's links; `mask` zeroes the fixed components of u (the other
-   voxel's and its own) and of y.  own = u_i on return. */
+/* y_i = (K u)_i over the voxel's links; own = u_i on return */
 template <class Load>
-__device__ __forceinline__ void apply_row(const LinPtrs& s, const Load& u, int i, bool mask, double* own, double* y) {
+__device__ __forceinline__ void apply_row(const LinPtrs& s, const Load& u, int i, double* own, double* y) {
     const int nv = s.nv;
-    const int fi = mask ? s.fixed[i] : 0;
     u(i, own);
-    for (int j = 0; j < 6; j++) {
-        if (fi & (1 << j)) own[j] = 0.0;
-        y[j] = 0.0;
-    }
+    for (int j = 0; j < 6; j++) y[j] = 0.0;
 #if VX_LIN_UNROLL
 #pragma unroll
 #else
@@ -114,16 +111,8 @@ __device__ __forceinline__ void apply_row(const LinPtrs& s, const Load& u, int i
         const LinkBlk k = link_blk(s.lmats[s.lmeta[slot]], axis);
         double oth[6];
         u(o, oth);
-        if (mask) {
-            const int fo = s.fixed[o];
-            for (int j = 0; j < 6; j++)
-                if (fo & (1 << j)) oth[j] = 0.0;
-        }
         link_apply(k, i < o, own, oth, y);
     }
-    if (mask)
-        for (int j = 0; j < 6; j++)
-            if (fi & (1 << j)) y[j] = 0.0;
 }
 
 /* workgroup sums of two values into part[2*blockIdx.x + 0/1] (lanes within a wavefront by
@@ -146,36 +135,57 @@ __device__ __forceinline__ void block_sum2(double a, double b, double* part) {
     }
 }
 
-/* one workgroup: the partial sums in workgroup order, then the scalars of the phase (0:
-   set-up, 1: after the matrix product, 2: after the update).  A separate launch rather than
-   the last workgroup of the producing kernel: making each workgroup's sums visible to another
-   XCD's workgroup would need a device-scope release (an L2 write-back) per workgroup. */
-__global__ void __launch_bounds__(256) k_lin_reduce(LinPtrs s, int nblk, int phase) {
-    __shared__ double sa[256], sb[256];
+/* The sum of all workgroups' partial sums, formed by every workgroup that needs it (the same order
+   in each, so all hold the same bits).  The partials of at most kLinMaxBlocks workgroups are 16 KB
+   that the L2s hold; a reduction in a launch of its own cost 5.1 us twice an iteration on a
+   79,200-voxel block, where the rest of the iteration took 24. */
+constexpr int kLinMaxBlocks = 1024;
+/* up to here the direction is formed inside the product (us an iteration, a pass of its own against
+   fused: 79,200 voxels 24.8 / 19.3, 224,000 voxels 42.0 / 39.2), and what one kernel writes goes
+   through the caches to the next kernel's workgroup on the same XCD; above, the vectors leave the
+   L2s and both cost (1,048,576 voxels 157 against 164 cached) */
+constexpr int kLinFusedMax = 262144;
+__device__ __forceinline__ void all_sum2(const double* part, int nblk, double* outA, double* outB) {
+    __shared__ double sa[8], sb[8];
     double a = 0.0, b = 0.0;
     for (int k = threadIdx.x; k < nblk; k += blockDim.x) {
-        a += s.part[2 * k];
-        b += s.part[2 * k + 1];
+        a += part[2 * k];
+        b += part[2 * k + 1];
     }
-    sa[threadIdx.x] = a;
-    sb[threadIdx.x] = b;
+    for (int off = 32; off > 0; off >>= 1) {
+        a += __shfl_xor(a, off, 64);
+        b += __shfl_xor(b, off, 64);
+    }
+    const int w = threadIdx.x >> 6, waves = (int)blockDim.x >> 6;
+    if ((threadIdx.x & 63) == 0) { sa[w] = a; sb[w] = b; }
     __syncthreads();
+    a = sa[0];
+    b = sb[0];
+    for (int k = 1; k < waves; k++) { a += sa[k]; b += sb[k]; }
+    *outA = a;
+    *outB = b;
+    __syncthreads();
+}
+/* beta of iteration it from the sums the update (or the set-up: r.z against 0) left; workgroup 0
+   keeps r.z for the update and for the next iteration's beta */
+__device__ __forceinline__ double lin_beta(const LinPtrs& s, int it) {
+    double rz, rr;
+    all_sum2(s.part, s.nblk, &rz, &rr);
+    const double old = s.scal[S_RZ + (it & 1)];
+    if (blockIdx.x == 0 && threadIdx.x == 0) s.scal[S_RZ + ((it + 1) & 1)] = rz;
+    return old != 0.0 ? rz / old : 0.0;
+}
+
+/* after the set-up (init) or a chunk of iterations: the residual r.r the host looks at; the set-up
+   also starts r.z of "the iteration before" at 0, so that the first beta is 0 */
+__global__ void __launch_bounds__(256) k_lin_residual(LinPtrs s, int init) {
+    double rz, rr;
+    all_sum2(s.part, s.nblk, &rz, &rr);
     if (threadIdx.x != 0) return;
-    double ta = 0.0, tb = 0.0;
-    for (int k = 0; k < (int)blockDim.x; k++) { ta += sa[k]; tb += sb[k]; }
-    double* sc = s.scal;
-    if (phase == 0) {
-        sc[S_RZ] = ta;
-        sc[S_BB] = tb;
-        sc[S_RR] = tb;
-        sc[S_BETA] = 0.0;
-    } else if (phase == 1) {
-        sc[S_PQ] = ta;
-        sc[S_ALPHA] = ta != 0.0 ? sc[S_RZ] / ta : 0.0;
-    } else {
-        sc[S_BETA] = sc[S_RZ] != 0.0 ? ta / sc[S_RZ] : 0.0;
-        sc[S_RZ] = ta;
-        sc[S_RR] = tb;
+    s.scal[S_RR] = rr;
+    if (init) {
+        s.scal[S_BB] = rr;
+        s.scal[S_RZ] = 0.0;
     }
 }
 
@@ -215,14 +225,15 @@ __global__ void __launch_bounds__(256) k_lin_prep(LinPtrs s, uint8_t* fixed, dou
 
 /* set-up: b = f - K x_fixed on the free components; the preconditioner; x = 0, r = b,
    z = M r, p = z; partial sums of r.z and b.b */
-__global__ void __launch_bounds__(256) k_lin_setup(LinPtrs s) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+__global__ void __launch_bounds__(512) k_lin_setup(LinPtrs s) {
     double rz = 0.0, bb = 0.0;
-    if (i < s.nv) {
+    for (int t = 0; t < s.per; t++) {
+        const int i = ((int)blockIdx.x * s.per + t) * (int)blockDim.x + (int)threadIdx.x;
+        if (i >= s.nv) break;
         const int nv = s.nv;
         const int fi = s.fixed[i];
         double kx[6], xo[6];
-        apply_row(s, Plain{s.xfix, nv}, i, false, xo, kx);
+        apply_row(s, Plain{s.xfix, nv}, i, xo, kx);
         double b[6];
         for (int j = 0; j < 6; j++) b[j] = (fi & (1 << j)) ? 0.0 : s.f[j * nv + i] - kx[j];
         /* the voxel's diagonal block, fixed rows and columns replaced by the identity */
@@ -297,12 +308,14 @@ __global__ void __launch_bounds__(256) k_lin_setup(LinPtrs s) {
 }
 
 /* the search direction p = z + beta p (beta = 0 on the first iteration, when p = z already) */
-__global__ void __launch_bounds__(256) k_lin_direction(LinPtrs s) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= s.nv) return;
+__global__ void __launch_bounds__(256) k_lin_direction(LinPtrs s, int it) {
+    const double beta = lin_beta(s, it);
     const int nv = s.nv;
-    const double beta = s.scal[S_BETA];
-    for (int j = 0; j < 6; j++) st_nt(&s.p[j * nv + i], s.z[j * nv + i] + beta * s.p[j * nv + i]);
+    for (int t = 0; t < s.per; t++) {
+        const int i = ((int)blockIdx.x * s.per + t) * 256 + (int)threadIdx.x;
+        if (i >= nv) return;
+        for (int j = 0; j < 6; j++) st_nt(&s.p[j * nv + i], s.z[j * nv + i] + beta * s.p[j * nv + i]);
+    }
 }
 
 /* the link material table staged in LDS by every workgroup when it fits (0.170 -> 0.168 ms
@@ -311,58 +324,126 @@ __global__ void __launch_bounds__(256) k_lin_direction(LinPtrs s) {
 #define VX_LIN_MATS_LDS 1
 #endif
 constexpr int kLinLdsLinkMats = 64;
-/* q = K p on the free components; partial sums of p.q.  (Forming z + beta p here, where p is
-   read, instead of in its own pass doubles the neighbour reads and was 3-5 % slower.) */
+template <bool MatsLds>
+__device__ __forceinline__ void stage_link_mats(LinPtrs& s, LinkMat* slm) {
+    if (!MatsLds) return;
+    const int nl32 = s.nlmats * (int)(sizeof(LinkMat) / 4);
+    for (int t = threadIdx.x; t < nl32; t += blockDim.x) ((uint32_t*)slm)[t] = ((const uint32_t*)s.lmats)[t];
+    s.lmats = slm;
+}
+/* q = K p on the free components; partial sums of p.q.  A direction is 0 on every fixed component
+   (z and the first p are), so only q is masked.
+   XCD-contiguous blocks, so the neighbours a voxel gathers along x and y are read in the
+   same XCD's L2 (on a 128x128x64 block it fetched 6 % less than with the default
+   round-robin placement; the z neighbours, three lattice layers of vectors apart, do not
+   all stay in a 4 MB L2) */
 template <bool MatsLds>
 __global__ void __launch_bounds__(256) k_lin_apply(LinPtrs s0) {
     LinPtrs s = s0;
-    if (MatsLds) { /* the link material table in LDS (every lane takes part before any returns) */
-        __shared__ LinkMat slm[kLinLdsLinkMats];
-        const int nl32 = s0.nlmats * (int)(sizeof(LinkMat) / 4);
-        for (int t = threadIdx.x; t < nl32; t += blockDim.x) ((uint32_t*)slm)[t] = ((const uint32_t*)s0.lmats)[t];
-        __syncthreads();
-        s.lmats = slm;
-    }
-    /* XCD-contiguous blocks, so the neighbours a voxel gathers along x and y are read in the
-       same XCD's L2 (on a 128x128x64 block it fetched 6 % less than with the default
-       round-robin placement; the z neighbours, three lattice layers of vectors apart, do not
-       all stay in a 4 MB L2) */
-    const int i = lane_index(1);
+    __shared__ LinkMat slm[MatsLds ? kLinLdsLinkMats : 1];
+    stage_link_mats<MatsLds>(s, slm);
+    __syncthreads();
+    const int nv = s.nv;
     double pq = 0.0;
-    if (i < s.nv) {
-        const int nv = s.nv;
+    for (int t = 0; t < s.per; t++) {
+        const int i = (xcd_block() * s.per + t) * 256 + (int)threadIdx.x;
+        if (i >= nv) break;
         double own[6], y[6];
-        apply_row(s, Plain{s.p, nv}, i, true, own, y);
+        apply_row(s, Plain{s.p, nv}, i, own, y);
+        const int fi = s.fixed[i];
         for (int j = 0; j < 6; j++) {
+            if (fi & (1 << j)) y[j] = 0.0;
             st_nt(&s.q[j * nv + i], y[j]);
             pq += own[j] * y[j];
         }
     }
-    block_sum2(pq, 0.0, s.part);
+    block_sum2(pq, 0.0, s.partQ);
+}
+/* The same with the direction p = z + beta p formed where it is read, for the voxel (which writes
+   it to pNext) and for the neighbours it gathers, instead of in a pass of its own: one launch
+   fewer for twice the neighbour reads.  One block a workgroup (per 1).  Everything is asked for
+   before the sums of the workgroups are waited for, and the chain of an iteration is then two
+   loads and two reductions a kernel. */
+template <bool MatsLds>
+__global__ void __launch_bounds__(512) k_lin_apply_fused(LinPtrs s0, int it) {
+    LinPtrs s = s0;
+    __shared__ LinkMat slm[MatsLds ? kLinLdsLinkMats : 1];
+    const int nv = s.nv;
+    const int at = xcd_block() * (int)blockDim.x + (int)threadIdx.x;
+    const int i = at < nv ? at : nv - 1;
+    int nb[6], meta[6];
+    for (int dir = 0; dir < 6; dir++) nb[dir] = s.vnbr[dir * nv + i];
+    double z[6], p[6], zn[6][6], pn[6][6];
+    for (int j = 0; j < 6; j++) z[j] = s.z[j * nv + i], p[j] = s.p[j * nv + i];
+    const int fi = s.fixed[i];
+    stage_link_mats<MatsLds>(s, slm);
+    for (int dir = 0; dir < 6; dir++) {
+        const int o = nb[dir] >= 0 ? nb[dir] : i;
+        meta[dir] = s.lmeta[(dir >> 1) * nv + ((dir & 1) == 0 ? i : o)];
+        for (int j = 0; j < 6; j++) zn[dir][j] = s.z[j * nv + o], pn[dir][j] = s.p[j * nv + o];
+    }
+    const double beta = lin_beta(s, it); /* its barriers publish the material table too */
+    double own[6], y[6];
+    for (int j = 0; j < 6; j++) {
+        own[j] = z[j] + beta * p[j];
+        y[j] = 0.0;
+    }
+    for (int dir = 0; dir < 6; dir++) {
+        if (nb[dir] < 0) continue;
+        double oth[6];
+        for (int j = 0; j < 6; j++) oth[j] = zn[dir][j] + beta * pn[dir][j];
+        link_apply(link_blk(s.lmats[meta[dir]], dir >> 1), i < nb[dir], own, oth, y);
+    }
+    double pq = 0.0;
+    if (at < nv)
+        for (int j = 0; j < 6; j++) {
+            if (fi & (1 << j)) y[j] = 0.0;
+            s.pNext[j * nv + i] = own[j];
+            s.q[j * nv + i] = y[j];
+            pq += own[j] * y[j];
+        }
+    block_sum2(pq, 0.0, s.partQ);
 }
 
-/* x += alpha p, r -= alpha q, z = M r; partial sums of r.z and r.r */
-__global__ void __launch_bounds__(256) k_lin_update(LinPtrs s) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    double rz = 0.0, rr2 = 0.0;
-    if (i < s.nv) {
-        const int nv = s.nv;
-        const double alpha = s.scal[S_ALPHA];
-        const int fi = s.fixed[i];
-        double r[6];
+/* x += alpha p, r -= alpha q, z = M r; partial sums of r.z and r.r; the first block's operands are
+   asked for before alpha's sum is waited for */
+template <bool Cached>
+__global__ void __launch_bounds__(512) k_lin_update(LinPtrs s, int it) {
+    const int nv = s.nv;
+    double x[6], p[6], r[6], q[6];
+    float m[21];
+    int fi = 0, i = (Cached ? xcd_block() : (int)blockIdx.x) * s.per * (int)blockDim.x + (int)threadIdx.x;
+    auto load = [&]() {
+        fi = s.fixed[i];
         for (int j = 0; j < 6; j++) {
-            st_nt(&s.x[j * nv + i], s.x[j * nv + i] + alpha * s.p[j * nv + i]);
-            r[j] = s.r[j * nv + i] - alpha * s.q[j * nv + i];
-            st_nt(&s.r[j * nv + i], r[j]);
+            r[j] = s.r[j * nv + i];
+            q[j] = s.q[j * nv + i];
+            x[j] = s.x[j * nv + i];
+            p[j] = s.p[j * nv + i];
+        }
+        for (int c = 0; c < 21; c++) m[c] = s.minv[c * nv + i];
+    };
+    if (i < nv) load();
+    double pq, none;
+    all_sum2(s.partQ, s.nblk, &pq, &none);
+    const double alpha = pq != 0.0 ? s.scal[S_RZ + ((it + 1) & 1)] / pq : 0.0;
+    double rz = 0.0, rr2 = 0.0;
+    for (int t = 0; t < s.per && i < nv; t++) {
+        if (t > 0) load();
+        for (int j = 0; j < 6; j++) {
+            put<Cached>(&s.x[j * nv + i], x[j] + alpha * p[j]);
+            r[j] = r[j] - alpha * q[j];
+            put<Cached>(&s.r[j * nv + i], r[j]);
         }
         for (int rr = 0; rr < 6; rr++) {
             double e = 0.0;
-            for (int c = 0; c < 6; c++) e += (double)s.minv[tri(rr, c) * nv + i] * r[c];
+            for (int c = 0; c < 6; c++) e += (double)m[tri(rr, c)] * r[c];
             if (fi & (1 << rr)) e = 0.0;
-            st_nt(&s.z[rr * nv + i], e);
+            put<Cached>(&s.z[rr * nv + i], e);
             rz += r[rr] * e;
             rr2 += r[rr] * r[rr];
         }
+        i += (int)blockDim.x;
     }
     block_sum2(rz, rr2, s.part);
 }
@@ -390,7 +471,17 @@ __global__ void __launch_bounds__(256) k_lin_post(LinPtrs s, double* vd, const i
 
 static inline unsigned nblocks(int n) { return (unsigned)((n + 255) / 256); }
 
-int lin_blocks(int nv) { return (int)nblocks(nv); }
+/* voxels of a block: where the fused product's 208 registers let a CU hold them all (512 lanes),
+   one workgroup on each of the 256 CUs; else 256.  A 79,200-voxel block in 310 workgroups of 256
+   lanes takes 19.3 us an iteration, in 248 of 320 17.8 */
+static int lin_block(int nv) { return nv <= 256 * 512 ? 64 * std::max(1, (nv + 256 * 64 - 1) / (256 * 64)) : 256; }
+
+/* workgroups of an iteration's kernels and the blocks each takes */
+void lin_blocks(int nv, int* nblk, int* per) {
+    const int b = lin_block(nv), nb = (nv + b - 1) / b;
+    *per = (nb + kLinMaxBlocks - 1) / kLinMaxBlocks;
+    *nblk = (nb + *per - 1) / *per;
+}
 
 void launch_lin_prep(const LinPtrs& s, uint8_t* fixed, double* xfix, double* f, const double* vd, const int* vext,
                      const ExtRec* exts, const int* vijk, double size, hipStream_t st) {
@@ -398,18 +489,30 @@ void launch_lin_prep(const LinPtrs& s, uint8_t* fixed, double* xfix, double* f, 
                        size);
 }
 void launch_lin_setup(const LinPtrs& s, hipStream_t st) {
-    const unsigned nb = nblocks(s.nv);
-    hipLaunchKernelGGL(k_lin_setup, dim3(nb), dim3(256), 0, st, s);
-    hipLaunchKernelGGL(k_lin_reduce, dim3(1), dim3(256), 0, st, s, (int)nb, 0);
+    hipLaunchKernelGGL(k_lin_setup, dim3(s.nblk), dim3(lin_block(s.nv)), 0, st, s);
+    hipLaunchKernelGGL(k_lin_residual, dim3(1), dim3(256), 0, st, s, 1);
 }
-void launch_lin_iteration(const LinPtrs& s, hipStream_t st) {
-    const unsigned nb = nblocks(s.nv);
-    hipLaunchKernelGGL(k_lin_direction, dim3(nb), dim3(256), 0, st, s);
-    if (VX_LIN_MATS_LDS && s.nlmats <= kLinLdsLinkMats) hipLaunchKernelGGL(k_lin_apply<true>, dim3(nb), dim3(256), 0, st, s);
-    else hipLaunchKernelGGL(k_lin_apply<false>, dim3(nb), dim3(256), 0, st, s);
-    hipLaunchKernelGGL(k_lin_reduce, dim3(1), dim3(256), 0, st, s, (int)nb, 1);
-    hipLaunchKernelGGL(k_lin_update, dim3(nb), dim3(256), 0, st, s);
-    hipLaunchKernelGGL(k_lin_reduce, dim3(1), dim3(256), 0, st, s, (int)nb, 2);
+void launch_lin_residual(const LinPtrs& s, hipStream_t st) {
+    hipLaunchKernelGGL(k_lin_residual, dim3(1), dim3(256), 0, st, s, 0);
+}
+/* iteration it of a chunk that starts at an even one; where the direction is fused the two halves
+   of p change places (s is the chunk's own copy) */
+void launch_lin_iteration(LinPtrs& s, int it, hipStream_t st) {
+    const dim3 grid(s.nblk), block(lin_block(s.nv));
+    const bool lds = VX_LIN_MATS_LDS && s.nlmats <= kLinLdsLinkMats;
+    if (s.nv <= kLinFusedMax) {
+        if (lds) hipLaunchKernelGGL(k_lin_apply_fused<true>, grid, block, 0, st, s, it);
+        else hipLaunchKernelGGL(k_lin_apply_fused<false>, grid, block, 0, st, s, it);
+        double* const t = s.p;
+        s.p = s.pNext;
+        s.pNext = t;
+    } else {
+        hipLaunchKernelGGL(k_lin_direction, grid, block, 0, st, s, it);
+        if (lds) hipLaunchKernelGGL(k_lin_apply<true>, grid, block, 0, st, s);
+        else hipLaunchKernelGGL(k_lin_apply<false>, grid, block, 0, st, s);
+    }
+    if (s.nv <= kLinFusedMax) hipLaunchKernelGGL(k_lin_update<true>, grid, block, 0, st, s, it);
+    else hipLaunchKernelGGL(k_lin_update<false>, grid, block, 0, st, s, it);
 }
 void launch_lin_post(const LinPtrs& s, double* vd, const int* vijk, double size, hipStream_t st) {
     hipLaunchKernelGGL(k_lin_post, dim3(nblocks(s.nv)), dim3(256), 0, st, s, vd, vijk, size);

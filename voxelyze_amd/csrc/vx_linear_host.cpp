@@ -17,11 +17,12 @@
 
 namespace vx {
 
-int lin_blocks(int nv);
+void lin_blocks(int nv, int* nblk, int* per);
 void launch_lin_prep(const LinPtrs& s, uint8_t* fixed, double* xfix, double* f, const double* vd, const int* vext,
                      const ExtRec* exts, const int* vijk, double size, hipStream_t st);
 void launch_lin_setup(const LinPtrs& s, hipStream_t st);
-void launch_lin_iteration(const LinPtrs& s, hipStream_t st);
+void launch_lin_iteration(LinPtrs& s, int it, hipStream_t st);
+void launch_lin_residual(const LinPtrs& s, hipStream_t st);
 void launch_lin_post(const LinPtrs& s, double* vd, const int* vijk, double size, hipStream_t st);
 
 #define HIPCHK(call)                                       \
@@ -32,7 +33,7 @@ void launch_lin_post(const LinPtrs& s, double* vd, const int* vijk, double size,
 
 /* iterations between two convergence checks (each check is one 8-byte read-back); they are
    recorded once as a HIP graph and replayed */
-static const int kChunk = 24;
+static const int kChunk = 24; /* even: an iteration's scalars and halves go by its parity */
 
 namespace {
 struct GraphGuard {
@@ -61,10 +62,11 @@ bool Sim::linearSolve(double tol, int maxIter, int* itersOut, double* residualOu
     if (!(tol > 0.0)) tol = 1e-10;
     if (maxIter <= 0) maxIter = 100000;
     if (!syncUp()) return false;
-    const int nb = lin_blocks(n);
+    LinPtrs lp;
+    lin_blocks(n, &lp.nblk, &lp.per);
     const size_t V = (size_t)n;
     auto align = [](size_t b) { return (b + 255) & ~(size_t)255; };
-    const size_t bytes = 7 * align(V * 48) + align(V * 4 * 21) + align(V) + align((size_t)nb * 16) +
+    const size_t bytes = 8 * align(V * 48) + align(V * 4 * 21) + align(V) + 2 * align((size_t)lp.nblk * 16) +
                          align(S_COUNT * 8) + align(4);
     if (!blin.ensure(bytes)) {
         err = "device allocation failed";
@@ -76,7 +78,6 @@ bool Sim::linearSolve(double tol, int maxIter, int* itersOut, double* residualOu
         base += align(b);
         return (void*)p;
     };
-    LinPtrs lp;
     lp.nv = n;
     lp.vnbr = dp.vnbr;
     lp.lmeta = dp.lmeta;
@@ -90,11 +91,13 @@ bool Sim::linearSolve(double tol, int maxIter, int* itersOut, double* residualOu
     lp.r = (double*)carve(V * 48);
     lp.z = (double*)carve(V * 48);
     lp.p = (double*)carve(V * 48);
+    lp.pNext = (double*)carve(V * 48);
     lp.q = (double*)carve(V * 48);
     lp.minv = (float*)carve(V * 4 * 21);
     uint8_t* dfixed = (uint8_t*)carve(V);
     lp.fixed = dfixed;
-    lp.part = (double*)carve((size_t)nb * 16);
+    lp.part = (double*)carve((size_t)lp.nblk * 16);
+    lp.partQ = (double*)carve((size_t)lp.nblk * 16);
     lp.scal = (double*)carve(S_COUNT * 8);
     lp.bad = (int*)carve(4);
     if ((size_t)(base - (char*)blin.p) > blin.bytes) {
@@ -121,7 +124,9 @@ bool Sim::linearSolve(double tol, int maxIter, int* itersOut, double* residualOu
         const double target = tol * tol * bb;
         GraphGuard graph;
         HIPCHK(hipStreamBeginCapture(stream, hipStreamCaptureModeThreadLocal));
-        for (int c = 0; c < kChunk; c++) launch_lin_iteration(lp, stream);
+        LinPtrs chunk = lp;
+        for (int c = 0; c < kChunk; c++) launch_lin_iteration(chunk, c, stream);
+        launch_lin_residual(chunk, stream);
         HIPCHK(hipStreamEndCapture(stream, &graph.g));
         HIPCHK(hipGraphInstantiate(&graph.e, graph.g, nullptr, nullptr, 0));
         while (rr > target && it < maxIter) {
