@@ -29,9 +29,7 @@ struct StateCheckpoint {
     DevBuf vd, vflags, vtemp, vprevdt, vps, ld, lf, lflags, vf, ms, mfl, clast, ccount, coff, cpart;
 };
 
-static hipError_t d2d(void* dst, const void* src, size_t bytes, hipStream_t st) {
-    return bytes ? hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToDevice, st) : hipSuccess;
-}
+void launch_copy_list(const CopyList& c, hipStream_t st);
 
 bool Sim::checkpointSave(int slot) {
     if (slot < 0 || slot >= kCheckpointSlots) {
@@ -62,22 +60,23 @@ bool Sim::checkpointSave(int slot) {
         err = "device allocation failed";
         return false;
     }
-    HIPCHK(d2d(c.vd.p, dp.vd, VD_COUNT * n * 8, stream));
-    HIPCHK(d2d(c.vflags.p, dp.vflags, n * 4, stream));
-    HIPCHK(d2d(c.vtemp.p, dp.vtemp, n * 4, stream));
-    HIPCHK(d2d(c.vprevdt.p, dp.vprevdt, n * 4, stream));
-    HIPCHK(d2d(c.vps.p, dp.vps, 3 * n * 4, stream));
-    HIPCHK(d2d(c.ld.p, dp.ld, LDEV_COUNT * S * 8, stream));
-    HIPCHK(d2d(c.lf.p, dp.lf, LF_COUNT * S * 4, stream));
-    HIPCHK(d2d(c.lflags.p, dp.lflags, S * 4, stream));
-    HIPCHK(d2d(c.vf.p, dp.vf, VF_COUNT * n * 8, stream));
+    CopyList list;
+    list.add(c.vd.p, dp.vd, VD_COUNT * n * 8);
+    list.add(c.vflags.p, dp.vflags, n * 4);
+    list.add(c.vtemp.p, dp.vtemp, n * 4);
+    list.add(c.vprevdt.p, dp.vprevdt, n * 4);
+    list.add(c.vps.p, dp.vps, 3 * n * 4);
+    list.add(c.ld.p, dp.ld, LDEV_COUNT * S * 8);
+    list.add(c.lf.p, dp.lf, LF_COUNT * S * 4);
+    list.add(c.lflags.p, dp.lflags, S * 4);
+    list.add(c.vf.p, dp.vf, VF_COUNT * n * 8);
     if (fused()) {
         if (!c.ms.ensure(std::max(one, MS_COUNT * S * lsElem())) || !c.mfl.ensure(std::max(one, S * 4))) {
             err = "device allocation failed";
             return false;
         }
-        HIPCHK(d2d(c.ms.p, bms[lcur].p, MS_COUNT * S * lsElem(), stream));
-        HIPCHK(d2d(c.mfl.p, bmfl[lcur].p, S * 4, stream));
+        list.add(c.ms.p, bms[lcur].p, MS_COUNT * S * lsElem());
+        list.add(c.mfl.p, bmfl[lcur].p, S * 4);
     }
     if (c.collisions) {
         const size_t ce = (size_t)std::max(colEntries, 0);
@@ -86,11 +85,13 @@ bool Sim::checkpointSave(int slot) {
             err = "device allocation failed";
             return false;
         }
-        HIPCHK(d2d(c.clast.p, cp.last, 3 * n * 4, stream));
-        HIPCHK(d2d(c.ccount.p, cp.pairCount, n * 4, stream));
-        HIPCHK(d2d(c.coff.p, cp.pairOff, n * 4, stream));
-        if (ce) HIPCHK(d2d(c.cpart.p, cp.partners, ce * 4, stream));
+        list.add(c.clast.p, cp.last, 3 * n * 4);
+        list.add(c.ccount.p, cp.pairCount, n * 4);
+        list.add(c.coff.p, cp.pairOff, n * 4);
+        if (ce) list.add(c.cpart.p, cp.partners, ce * 4);
     }
+    launch_copy_list(list, stream);
+    HIPCHK(hipGetLastError());
     HIPCHK(hipStreamSynchronize(stream));
     return true;
 }
@@ -107,19 +108,20 @@ bool Sim::checkpointRestore(int slot) {
     }
     if (!syncUp()) return false; /* pending host edits land first, then the state is replaced */
     const size_t n = (size_t)nv(), S = 3 * n;
-    HIPCHK(d2d(dp.vd, c.vd.p, VD_COUNT * n * 8, stream));
-    HIPCHK(d2d(dp.vflags, c.vflags.p, n * 4, stream));
-    HIPCHK(d2d(dp.vtemp, c.vtemp.p, n * 4, stream));
-    if (fused() && bvtempAlt.p) HIPCHK(d2d(bvtempAlt.p, c.vtemp.p, n * 4, stream));
-    HIPCHK(d2d(dp.vprevdt, c.vprevdt.p, n * 4, stream));
-    HIPCHK(d2d(dp.vps, c.vps.p, 3 * n * 4, stream));
-    HIPCHK(d2d(dp.ld, c.ld.p, LDEV_COUNT * S * 8, stream));
-    HIPCHK(d2d(dp.lf, c.lf.p, LF_COUNT * S * 4, stream));
-    HIPCHK(d2d(dp.lflags, c.lflags.p, S * 4, stream));
-    HIPCHK(d2d(dp.vf, c.vf.p, VF_COUNT * n * 8, stream));
+    CopyList list;
+    list.add(dp.vd, c.vd.p, VD_COUNT * n * 8);
+    list.add(dp.vflags, c.vflags.p, n * 4);
+    list.add(dp.vtemp, c.vtemp.p, n * 4);
+    if (fused() && bvtempAlt.p) list.add(bvtempAlt.p, c.vtemp.p, n * 4);
+    list.add(dp.vprevdt, c.vprevdt.p, n * 4);
+    list.add(dp.vps, c.vps.p, 3 * n * 4);
+    list.add(dp.ld, c.ld.p, LDEV_COUNT * S * 8);
+    list.add(dp.lf, c.lf.p, LF_COUNT * S * 4);
+    list.add(dp.lflags, c.lflags.p, S * 4);
+    list.add(dp.vf, c.vf.p, VF_COUNT * n * 8);
     if (fused()) {
-        HIPCHK(d2d(bms[lcur].p, c.ms.p, MS_COUNT * S * lsElem(), stream));
-        HIPCHK(d2d(bmfl[lcur].p, c.mfl.p, S * 4, stream));
+        list.add(bms[lcur].p, c.ms.p, MS_COUNT * S * lsElem());
+        list.add(bmfl[lcur].p, c.mfl.p, S * 4);
     }
     if (c.collisions && collisions) {
         if (cp.nv != nv() || !bcLast.p) {
@@ -132,16 +134,18 @@ bool Sim::checkpointRestore(int slot) {
         }
         cp.partners = (int*)bcPartners.p;
         cp.cf = (float*)bcF.p;
-        HIPCHK(d2d(cp.last, c.clast.p, 3 * n * 4, stream));
-        HIPCHK(d2d(cp.pairCount, c.ccount.p, n * 4, stream));
-        HIPCHK(d2d(cp.pairOff, c.coff.p, n * 4, stream));
-        if (ce) HIPCHK(d2d(cp.partners, c.cpart.p, ce * 4, stream));
+        list.add(cp.last, c.clast.p, 3 * n * 4);
+        list.add(cp.pairCount, c.ccount.p, n * 4);
+        list.add(cp.pairOff, c.coff.p, n * 4);
+        if (ce) list.add(cp.partners, c.cpart.p, ce * 4);
         colEntries = c.colEntries;
         collisionsStale = c.collisionsStale;
         nearbyStale = c.nearbyStale;
     } else {
         collisionsStale = nearbyStale = true;
     }
+    launch_copy_list(list, stream);
+    HIPCHK(hipGetLastError());
     HIPCHK(hipStreamSynchronize(stream));
     rtime = c.rtime;
     rprev = c.rprev;

@@ -379,6 +379,36 @@ struct FusedPtrs {
     const float* vps;         /* the voxels' Poisson strains for this step (3 * nv) */
 };
 
+/* one robot's launch inputs: dt, previousDt, clock and divergence record */
+struct LaunchIn {
+    float dt, prev, time;
+    int div;
+};
+
+/* device copies made by one launch (checkpoints of small models are a dozen of some kilobytes) */
+struct CopyList {
+    static constexpr int kMax = 20;
+    int n = 0;
+    const void* src[kMax];
+    void* dst[kMax];
+    unsigned long long bytes[kMax]; /* multiples of 4, from 16-byte aligned addresses */
+    void add(void* d, const void* s, unsigned long long b) {
+        if (!b) return;
+        src[n] = s;
+        dst[n] = d;
+        bytes[n++] = b;
+    }
+};
+
+/* a range of voxels packed in row order for the host: null fields are not read */
+struct PackPtrs {
+    const double* vd;
+    const uint32_t* vfl;
+    int nv, first, count;
+    double *pos, *orient, *lin, *ang;
+    uint32_t* flags;
+};
+
 /* a kernel launch configuration chosen by the autotuner */
 struct LaunchCfg {
     int block;  /* workgroup size */

@@ -491,15 +491,6 @@ __global__ void __launch_bounds__(256) k_fused_temps(FusedPtrs s, int moved) {
     s.vtempIn[i] = actuation_temperature(s.actBase, s.actAmp, s.actFreq, s.rtimeIn[rob], s.vphase[i]);
 }
 
-/* after a launch: previousDt of every voxel whose robot completed at least one step */
-__global__ void __launch_bounds__(256) k_fused_prevdt(const int* vrobot, const int* rdiv, const float* rdt,
-                                                     float* vprevdt, int nv) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= nv) return;
-    const int r = vrobot[i];
-    if (rdiv[r] > 0) vprevdt[i] = rdt[r];
-}
-
 /* a robot that diverged in the launch's last step takes back its voxels (and clock, and for
    the mixed step its temperatures) from before that step, which the other ping-pong buffer
    holds */
@@ -563,11 +554,6 @@ void launch_step_fp64_ends(const FusedPtrs& s, hipStream_t st) {
 void launch_fused_temps(const FusedPtrs& s, bool moved, hipStream_t st) {
     if (s.nv > 0)
         hipLaunchKernelGGL(k_fused_temps, dim3((unsigned)((s.nv + 255) / 256)), dim3(256), 0, st, s, moved ? 1 : 0);
-}
-void launch_fused_prevdt(const int* vrobot, const int* rdiv, const float* rdt, float* vprevdt, int nv, hipStream_t st) {
-    if (nv > 0)
-        hipLaunchKernelGGL(k_fused_prevdt, dim3((unsigned)((nv + 255) / 256)), dim3(256), 0, st, vrobot, rdiv, rdt,
-                           vprevdt, nv);
 }
 void launch_fused_restore(double* vd, const double* vdPrev, uint32_t* vfl, const uint32_t* vflPrev, float* vtemp,
                           const float* vtempPrev, float* rtime, const float* rtimePrev, int nv, int first, int count,

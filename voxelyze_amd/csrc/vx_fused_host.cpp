@@ -14,7 +14,6 @@ namespace vx {
 void launch_step_fp64(const FusedPtrs& s, int block, bool forcesOnly, hipStream_t st);
 void launch_step_fp64_ends(const FusedPtrs& s, hipStream_t st);
 void launch_fused_temps(const FusedPtrs& s, bool moved, hipStream_t st);
-void launch_fused_prevdt(const int* vrobot, const int* rdiv, const float* rdt, float* vprevdt, int nv, hipStream_t st);
 void launch_fused_restore(double* vd, const double* vdPrev, uint32_t* vfl, const uint32_t* vflPrev, float* vtemp,
                           const float* vtempPrev, float* rtime, const float* rtimePrev, int nv, int first, int count,
                           int rob, hipStream_t st);
@@ -269,16 +268,10 @@ bool Sim::stepFp64Fused(int nsteps) {
 bool Sim::fusedFp64Finish(int launched) {
     const int n = nv(), R = nRobots();
     if (actOn && launched > 0) swapTemps(); /* back to the temperatures of the last step */
-    launch_fused_prevdt(dp.vrobot, dp.rdiv, dp.rdt, dp.vprevdt, n, stream);
-    HIPCHK(hipGetLastError());
-    /* the divergence record and the clocks in one copy: when no robot diverged they are also
-       what endLaunch needs, and the launch ends with this one synchronisation */
-    if (!pinned((size_t)8 * R)) return false;
-    std::vector<int> div(R);
-    HIPCHK(hipMemcpyAsync(pin, dp.rdiv, (size_t)4 * R, hipMemcpyDeviceToHost, stream));
-    HIPCHK(hipMemcpyAsync(pin + (size_t)4 * R, dp.rtime, (size_t)4 * R, hipMemcpyDeviceToHost, stream));
-    HIPCHK(hipStreamSynchronize(stream));
-    memcpy(div.data(), pin, (size_t)4 * R);
+    /* the divergence record and the clocks: when no robot diverged they are also what endLaunch
+       needs, and the launch ends with this one synchronisation */
+    std::vector<int> div;
+    if (!launchRecord(dp.vprevdt, &div)) return false;
     bool earlier = false, restored = false;
     for (int r = 0; r < R; r++) {
         const int d = div[r];

@@ -401,6 +401,99 @@ void launch_ext_ramps(ExtRec* exts, const RampRec* ramps, int n, const float* rt
     if (n > 0) hipLaunchKernelGGL(k_ext_ramps, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, exts, ramps, n, rtime, vrobot);
 }
 
+/* The inputs of a launch, from the kernel's arguments (one robot) or from pinned host memory, which
+   the device reads and writes itself: one launch in place of four copies and a fill before the
+   steps, and one in place of two copies (and the previousDt pass) after them.  One step of a
+   320-voxel model: 55 -> 23 us. */
+__global__ void __launch_bounds__(256) k_launch_begin(LaunchIn one, const float* pin, int R, float* rdt, float* rprev,
+                                                      float* rtime, int* rdiv, int* ctl) {
+    const int r = blockIdx.x * blockDim.x + threadIdx.x;
+    if (r < 4) ctl[r] = 0;
+    if (r >= R) return;
+    rdt[r] = R == 1 ? one.dt : pin[r];
+    rprev[r] = R == 1 ? one.prev : pin[R + r];
+    rtime[r] = R == 1 ? one.time : pin[2 * R + r];
+    rdiv[r] = R == 1 ? one.div : __float_as_int(pin[3 * R + r]);
+}
+/* the divergence record and the clocks to pinned host memory; previousDt of every voxel whose
+   robot completed at least one step (vprevdt null: the fused steps with their own link state) */
+__global__ void __launch_bounds__(256) k_launch_end(const int* rdiv, const float* rtime, int R, int* pinDiv, float* pinTime,
+                                                    const int* vrobot, const float* rdt, float* vprevdt, int nv) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < R) {
+        pinDiv[i] = rdiv[i];
+        pinTime[i] = rtime[i];
+    }
+    if (!vprevdt || i >= nv) return;
+    const int r = vrobot[i];
+    if (rdiv[r] > 0) vprevdt[i] = rdt[r];
+}
+void launch_launch_begin(const LaunchIn& one, const void* pin, int R, float* rdt, float* rprev, float* rtime, int* rdiv,
+                         int* ctl, hipStream_t st) {
+    hipLaunchKernelGGL(k_launch_begin, dim3(blocks(R < 4 ? 4 : R, 256)), dim3(256), 0, st, one, (const float*)pin, R, rdt, rprev,
+                       rtime, rdiv, ctl);
+}
+void launch_launch_end(const int* rdiv, const float* rtime, int R, void* pin, const int* vrobot, const float* rdt,
+                       float* vprevdt, int nv, hipStream_t st) {
+    const int n = vprevdt && nv > R ? nv : R;
+    hipLaunchKernelGGL(k_launch_end, dim3(blocks(n, 256)), dim3(256), 0, st, rdiv, rtime, R, (int*)pin,
+                       (float*)((char*)pin + (size_t)4 * R), vrobot, rdt, vprevdt, nv);
+}
+
+/* Voxels [first, first + count) in row order (x y z, w x y z, ...), written straight to pinned host
+   memory: each workgroup turns its 256 rows in LDS so that its stores are whole lines on the bus.
+   The host used to copy every component and interleave them (positions of 320 voxels 39 -> 14 us, of
+   1,048,576 voxels 3.05 -> 1.25 ms). */
+template <int C>
+__device__ __forceinline__ void pack_field(const PackPtrs& s, const int* comp, double* out, double* rows) {
+    if (!out) return;
+    const int base = blockIdx.x * 256, t = threadIdx.x;
+    const int n = s.count - base < 256 ? s.count - base : 256;
+    if (t < n)
+        for (int c = 0; c < C; c++) rows[t * C + c] = s.vd[(size_t)comp[c] * s.nv + s.first + base + t];
+    __syncthreads();
+    for (int k = t; k < n * C; k += 256) out[(size_t)base * C + k] = rows[k];
+    __syncthreads();
+}
+__global__ void __launch_bounds__(256) k_pack_voxels(PackPtrs s) {
+    __shared__ double rows[256 * 4];
+    const int pos[3] = {VPX, VPY, VPZ}, ori[4] = {VQW, VQX, VQY, VQZ}, lin[3] = {VLX, VLY, VLZ}, ang[3] = {VAX, VAY, VAZ};
+    pack_field<3>(s, pos, s.pos, rows);
+    pack_field<4>(s, ori, s.orient, rows);
+    pack_field<3>(s, lin, s.lin, rows);
+    pack_field<3>(s, ang, s.ang, rows);
+    const int i = blockIdx.x * 256 + threadIdx.x;
+    if (s.flags && i < s.count) s.flags[i] = s.vfl[s.first + i];
+}
+void launch_pack_voxels(const PackPtrs& s, hipStream_t st) {
+    if (s.count > 0) hipLaunchKernelGGL(k_pack_voxels, dim3(blocks(s.count, 256)), dim3(256), 0, st, s);
+}
+
+/* every copy of a list; a workgroup takes 16 KB of one of them (a checkpoint of 320 voxels restored:
+   52 -> 14 us, of 1,048,576 voxels 309 -> 280 us) */
+constexpr int kCopyChunk = 256 * 16 * 4;
+__global__ void __launch_bounds__(256) k_copy_list(CopyList c) {
+    unsigned long long b = blockIdx.x;
+    int k = 0;
+    for (; k < c.n - 1; k++) {
+        const unsigned long long nb = (c.bytes[k] + kCopyChunk - 1) / kCopyChunk;
+        if (b < nb) break;
+        b -= nb;
+    }
+    const unsigned long long off = b * kCopyChunk, left = c.bytes[k] - off;
+    const unsigned n = (unsigned)(left < kCopyChunk ? left : kCopyChunk), v = n / 16;
+    const uint4* src = (const uint4*)((const char*)c.src[k] + off);
+    uint4* dst = (uint4*)((char*)c.dst[k] + off);
+    for (unsigned t = threadIdx.x; t < v; t += 256) dst[t] = src[t];
+    const unsigned w = v * 4 + threadIdx.x;
+    if (w < n / 4) ((unsigned*)dst)[w] = ((const unsigned*)src)[w];
+}
+void launch_copy_list(const CopyList& c, hipStream_t st) {
+    unsigned long long nb = 0;
+    for (int k = 0; k < c.n; k++) nb += (c.bytes[k] + kCopyChunk - 1) / kCopyChunk;
+    if (nb) hipLaunchKernelGGL(k_copy_list, dim3((unsigned)nb), dim3(256), 0, st, c);
+}
+
 /* Staging of vxg_robot_com_noalloc: the per-robot centres of mass (3 doubles per robot, at
    most kScratchRobots robots, 1.5 MiB) written by k_robot_com before the copy to the caller.
    Each GPU holds its own copy for the life of the process.  In host code `scratch` names a

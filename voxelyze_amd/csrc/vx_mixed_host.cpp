@@ -329,8 +329,8 @@ bool Sim::stepMixed(int nsteps, MixTape* tape) {
         if (!graphStore(key, g)) return false;
     }
     HIPCHK(hipGetLastError());
-    HIPCHK(hipStreamSynchronize(stream));
     if (timed) {
+        HIPCHK(hipStreamSynchronize(stream));
         for (int k = 0; k < launched; k++) {
             float ms = 0;
             if (hipEventElapsedTime(&ms, events[2 * k], events[2 * k + 1]) != hipSuccess) continue;
@@ -348,12 +348,8 @@ bool Sim::stepMixed(int nsteps, MixTape* tape) {
    voxels, temperatures and clock from before that step (the other ping-pong half) */
 bool Sim::mixedFinish(int launched) {
     const int n = nv(), R = nRobots();
-    if (!pinned((size_t)8 * R)) return false;
-    std::vector<int> div(R);
-    HIPCHK(hipMemcpyAsync(pin, dp.rdiv, (size_t)4 * R, hipMemcpyDeviceToHost, stream));
-    HIPCHK(hipMemcpyAsync(pin + (size_t)4 * R, dp.rtime, (size_t)4 * R, hipMemcpyDeviceToHost, stream));
-    HIPCHK(hipStreamSynchronize(stream));
-    memcpy(div.data(), pin, (size_t)4 * R);
+    std::vector<int> div;
+    if (!launchRecord(nullptr, &div)) return false;
     bool restored = false;
     for (int r = 0; r < R; r++) {
         if (div[r] != launched - 1 || rfirst[r] == rfirst[r + 1]) continue;

@@ -14,6 +14,7 @@
 #include <string.h>
 
 #include <algorithm>
+#include <cstring>
 
 #pragma clang fp contract(off)
 
@@ -28,6 +29,11 @@ void launch_robot_state(const DevPtrs& s, const int* rfirst, int info, int type,
 void launch_robot_com(const DevPtrs& s, const int* rfirst, double* com, int nrobots, hipStream_t st);
 void launch_ext_ramps(ExtRec* exts, const RampRec* ramps, int n, const float* rtime, const int* vrobot, hipStream_t st);
 hipError_t scratch_address(void** out);
+void launch_launch_begin(const LaunchIn& one, const void* pin, int R, float* rdt, float* rprev, float* rtime, int* rdiv,
+                         int* ctl, hipStream_t st);
+void launch_launch_end(const int* rdiv, const float* rtime, int R, void* pin, const int* vrobot, const float* rdt,
+                       float* vprevdt, int nv, hipStream_t st);
+void launch_pack_voxels(const PackPtrs& s, hipStream_t st);
 void launch_col_stale(const DevPtrs& s, const ContactPtrs& c, int gen, hipStream_t st);
 void launch_col_keys(const DevPtrs& s, const ContactPtrs& c, int nbuckets, hipStream_t st);
 hipError_t col_sort(const ContactPtrs& c, void* tmp, size_t* tmpBytes, hipStream_t st);
@@ -1183,24 +1189,56 @@ bool Sim::syncForces() {
     return true;
 }
 
-/* a few voxels straight from the device, leaving the mirror stale */
+/* voxels straight from the device, leaving the mirror stale: packed by the device into pinned
+   memory in chunks of at most kReadHalf bytes, each copied out while the next is packed */
 bool Sim::readVoxelRange(int first, int count, double* pos, double* orient, double* lin, double* ang, uint32_t* flags) {
-    const int n = nv();
-    std::vector<double> buf((size_t)count);
-    auto get = [&](int c, double* out, int stride, int off) -> bool {
-        if (hipMemcpy(buf.data(), dp.vd + (size_t)c * n + first, (size_t)count * 8, hipMemcpyDeviceToHost) != hipSuccess)
-            return false;
-        for (int k = 0; k < count; k++) out[(size_t)k * stride + off] = buf[k];
-        return true;
+    static const size_t kReadHalf = (size_t)2 << 20;
+    const size_t row = (pos ? 24 : 0) + (orient ? 32 : 0) + (lin ? 24 : 0) + (ang ? 24 : 0) + (flags ? 4 : 0);
+    if (!row || count <= 0) return true;
+    const size_t chunk = std::min<size_t>((size_t)count, kReadHalf / row / 256 * 256);
+    const int nchunks = (int)(((size_t)count + chunk - 1) / chunk);
+    const size_t half = (chunk * row + 255) & ~(size_t)255;
+    if (!pinned(nchunks > 1 ? 2 * half : half)) return false;
+    while (events.size() < 2) {
+        hipEvent_t ev;
+        HIPCHK(hipEventCreate(&ev));
+        events.push_back(ev);
+    }
+    auto fields = [&](int k, size_t* a, size_t* n, PackPtrs* p) {
+        *a = (size_t)k * chunk;
+        *n = std::min(chunk, (size_t)count - *a);
+        char* b = pin + (k & 1 ? half : 0);
+        auto take = [&](bool want, size_t bytes) { /* each block stays 8-byte aligned: flags come last */
+            char* q = b;
+            if (want) b += *n * bytes;
+            return want ? q : nullptr;
+        };
+        *p = PackPtrs{dp.vd, dp.vflags, nv(), first + (int)*a, (int)*n, nullptr, nullptr, nullptr, nullptr, nullptr};
+        p->pos = (double*)take(pos, 24);
+        p->orient = (double*)take(orient, 32);
+        p->lin = (double*)take(lin, 24);
+        p->ang = (double*)take(ang, 24);
+        p->flags = (uint32_t*)take(flags, 4);
     };
-    bool ok = true;
-    if (pos) ok = ok && get(VPX, pos, 3, 0) && get(VPY, pos, 3, 1) && get(VPZ, pos, 3, 2);
-    if (orient) ok = ok && get(VQW, orient, 4, 0) && get(VQX, orient, 4, 1) && get(VQY, orient, 4, 2) && get(VQZ, orient, 4, 3);
-    if (lin) ok = ok && get(VLX, lin, 3, 0) && get(VLY, lin, 3, 1) && get(VLZ, lin, 3, 2);
-    if (ang) ok = ok && get(VAX, ang, 3, 0) && get(VAY, ang, 3, 1) && get(VAZ, ang, 3, 2);
-    if (flags) ok = ok && hipMemcpy(flags, dp.vflags + first, (size_t)count * 4, hipMemcpyDeviceToHost) == hipSuccess;
-    if (!ok) err = "device read failed";
-    return ok;
+    for (int k = 0; k <= nchunks; k++) {
+        size_t a, n;
+        PackPtrs p;
+        if (k < nchunks) {
+            fields(k, &a, &n, &p);
+            launch_pack_voxels(p, stream);
+            HIPCHK(hipGetLastError());
+            HIPCHK(hipEventRecord(events[k & 1], stream));
+        }
+        if (k == 0) continue;
+        HIPCHK(hipEventSynchronize(events[(k - 1) & 1]));
+        fields(k - 1, &a, &n, &p);
+        if (pos) memcpy(pos + 3 * a, p.pos, n * 24);
+        if (orient) memcpy(orient + 4 * a, p.orient, n * 32);
+        if (lin) memcpy(lin + 3 * a, p.lin, n * 24);
+        if (ang) memcpy(ang + 3 * a, p.ang, n * 24);
+        if (flags) memcpy(flags + a, p.flags, n * 4);
+    }
+    return true;
 }
 
 /* nsteps x CVoxelyze::doTimeStep(dt) (src/Voxelyze.cpp:251-284) */
@@ -1300,11 +1338,9 @@ bool Sim::beginLaunch(int nsteps) {
         ptime[r] = rtime[r];
         pdiv[r] = launchDt[r] == 0 ? -1 : NO_DIVERGENCE;
     }
-    HIPCHK(hipMemcpyAsync(brdt.p, pdt, b, hipMemcpyHostToDevice, stream));
-    HIPCHK(hipMemcpyAsync(brprev.p, pprev, b, hipMemcpyHostToDevice, stream));
-    HIPCHK(hipMemcpyAsync(dp.rtime, ptime, b, hipMemcpyHostToDevice, stream));
-    HIPCHK(hipMemcpyAsync(dp.rdiv, pdiv, b, hipMemcpyHostToDevice, stream));
-    HIPCHK(hipMemsetAsync(dp.ctl, 0, 4 * sizeof(int), stream));
+    launch_launch_begin(LaunchIn{pdt[0], pprev[0], ptime[0], pdiv[0]}, pin, R, (float*)brdt.p, (float*)brprev.p, dp.rtime,
+                        dp.rdiv, dp.ctl, stream);
+    HIPCHK(hipGetLastError());
     if (profiling) {
         const size_t need = (size_t)4 * nsteps;
         while (events.size() < need) {
@@ -1313,6 +1349,18 @@ bool Sim::beginLaunch(int nsteps) {
             events.push_back(ev);
         }
     }
+    return true;
+}
+
+/* the launch's divergence record and clocks in pin (as endLaunch reads them), and the record;
+   ends the launch with its one synchronisation */
+bool Sim::launchRecord(float* vprevdt, std::vector<int>* div) {
+    const int R = nRobots();
+    if (!pinned((size_t)8 * R)) return false;
+    launch_launch_end(dp.rdiv, dp.rtime, R, pin, dp.vrobot, dp.rdt, vprevdt, nv(), stream);
+    HIPCHK(hipGetLastError());
+    HIPCHK(hipStreamSynchronize(stream));
+    div->assign((const int*)pin, (const int*)pin + R);
     return true;
 }
 

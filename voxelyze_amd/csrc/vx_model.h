@@ -295,6 +295,7 @@ struct Sim {
     int stepRobots(const float* dt, int nsteps, int* done, int* divergedAt);
     std::vector<float> launchDt; /* per robot dt of the current launch */
     bool beginLaunch(int nsteps);
+    bool launchRecord(float* vprevdt, std::vector<int>* div);
     bool endLaunch(int nsteps, int* done);
     bool anyDiverged(int k, bool* all);
     bool robotCom(double* com);
