@@ -83,12 +83,15 @@ def test_options_in_both_forms(model, nv):
 @pytest.mark.gpu
 @pytest.mark.parametrize("side", [6, 26])
 @pytest.mark.parametrize("actuated", [False, True])
-def test_diverging_and_idle_robots(side, actuated):
-    print(f"[ends] robots beside a {side}^3 block, actuated {actuated}", flush=True)
+@pytest.mark.parametrize("nu", [0.0, 0.3])
+def test_diverging_and_idle_robots(side, actuated, nu):
+    print(f"[ends] robots beside a {side}^3 block, actuated {actuated}, Poisson's ratio {nu}", flush=True)
     sims = []
     for path in (0, 1):
         sim = B.maker(B.product_abi(), path)(0.005)
         mats = W.robot_materials(sim)
+        for m in mats:
+            m.setPoissonsRatio(nu)
         sim.setGravity(1.0)
         sim.enableFloor(True)
         for r, (n, mat) in enumerate(((3, 2), (side, 3), (4, 0), (3, 1))):
@@ -105,8 +108,9 @@ def test_diverging_and_idle_robots(side, actuated):
         sims.append(sim)
     a, b = sims
     dt = np.array([a.robotRecommendedTimeStep(r) for r in range(4)], np.float32)
+    assert [b.robotRecommendedTimeStep(r) for r in range(4)] == list(dt)
     dt[3] = 0.0
-    for n in (7, 60, 1):
+    for n in (7, 60, 60, 1):
         da, db = a.robotStep(n, dt), b.robotStep(n, dt)
         assert np.array_equal(da, db)
     assert da[2] < 1 or a.robotTime(2) < 60 * dt[2]

@@ -376,7 +376,10 @@ struct FusedPtrs {
     int offsetConst;          /* 1: the same for the strain offsets (every link material linear) */
     int xcd;
     int poisson;              /* a material has Poisson's ratio != 0 */
-    const float* vps;         /* the voxels' Poisson strains for this step (3 * nv) */
+    float* vps;               /* the voxels' Poisson strains for this step (3 * nv) */
+    float* vpsOut;            /* k_step_fp64_ends: a step writes the next step's unless it is the */
+    int psNext;               /* launch's last (psNext 0) */
+    const float* lratio;      /* strainRatio of each link slot */
 };
 
 /* one robot's launch inputs: dt, previousDt, clock and divergence record */

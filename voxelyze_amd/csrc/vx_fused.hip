@@ -44,6 +44,11 @@ namespace vx {
 __device__ void frozen_fp64(const FusedPtrs& s, int i, int rob, int d) {
     const int nv = s.nv, nl = s.nl;
     const bool idle = d < 0;
+    if (s.vpsOut) /* as the temperatures */
+        for (int c = 0; c < 3; c++) {
+            if (idle) s.vpsOut[c * nv + i] = s.vps[c * nv + i];
+            else if (s.k == d + 1) s.vps[c * nv + i] = s.vpsOut[c * nv + i];
+        }
     if (s.vphase) { /* both halves keep the temperatures of the last step that counted */
         if (idle) s.vtempOut[i] = s.vtempIn[i];
         else if (s.k == d + 1) s.vtempIn[i] = s.vtempOut[i];
@@ -116,7 +121,7 @@ __device__ __forceinline__ void link_load(const FusedPtrs& s, int i, int o, int 
 template <bool ForcesOnly, bool Neg, bool Poisson, bool Cached>
 __device__ __forceinline__ void link_end(const FusedPtrs& s, LinkIn& in, int i, int o, int mi, int dir, int rob,
                                          float prevDt, float tempI, const dvec& pos0, const dquat& q0,
-                                         dvec& f, dvec& mm) {
+                                         dvec& f, dvec& mm, float& strain) {
     const int nv = s.nv, nl = s.nl;
     const int axis = dir >> 1;
     const int n = Neg ? i : o, p = Neg ? o : i;
@@ -147,6 +152,7 @@ __device__ __forceinline__ void link_end(const FusedPtrs& s, LinkIn& in, int i, 
     LinkEval e;
     link_eval_fp64<Poisson>(m, s.curveStrain + m.curveOff, s.curveStress + m.curveOff, axis, Neg ? pos0 : po,
                    Neg ? q0 : qo, Neg ? po : pos0, Neg ? qo : q0, rest, old, dmN, dmP, &e);
+    strain = e.strain;
     f = Neg ? e.fN : e.fP;
     mm = Neg ? e.mN : e.mP;
     if (s.storeForces) {
@@ -280,13 +286,14 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(VX_FUS
         }
         /* the two ends as separate instances, each computing only its own end vectors */
         dvec f, mm;
+        float strain;
         LinkIn in;
         if ((dir & 1) == 0) {
             link_load<true, Poisson>(s, i, o, dir, in);
-            link_end<ForcesOnly, true, Poisson, false>(s, in, i, o, mi, dir, rob, prevDt, tempI, pos0, q0, f, mm);
+            link_end<ForcesOnly, true, Poisson, false>(s, in, i, o, mi, dir, rob, prevDt, tempI, pos0, q0, f, mm, strain);
         } else {
             link_load<false, Poisson>(s, i, o, dir, in);
-            link_end<ForcesOnly, false, Poisson, false>(s, in, i, o, mi, dir, rob, prevDt, tempI, pos0, q0, f, mm);
+            link_end<ForcesOnly, false, Poisson, false>(s, in, i, o, mi, dir, rob, prevDt, tempI, pos0, q0, f, mm, strain);
         }
         sf.x += f.x; sf.y += f.y; sf.z += f.z;
         sm.x += mm.x; sm.y += mm.y; sm.z += mm.z;
@@ -327,6 +334,9 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(VX_FUS
    sums the forces in direction order and integrates the translations while wave 1 does the same
    with the moments and rotations.  Each link end is evaluated by link_end on the same inputs and
    the sums keep their order (an absent link adds +0.0), so the bits are k_step_fp64's.
+   With a Poisson's ratio, wave 2 forms the voxel's Poisson strain for the next step from the
+   strains its links just took, which k_poisson_fp64 otherwise does in a launch before every step
+   (8,385 voxels: 15.2 us a step with that launch, 9.3 without).
 
    What bounds it: the chain of dependent loads and FP64 operations of one link (2.7 us of the 5 us
    a workgroup lives; 2.5 us more pass between two launches), which k_step_fp64 walks through six
@@ -350,6 +360,7 @@ __global__ void __launch_bounds__(6 / PerWave * kEndsTile) __attribute__((amdgpu
     const int at = xcd_block() * kEndsTile + lane;
     const double* __restrict__ vd = s.vdIn;
     __shared__ double ends[6][6][kEndsTile];
+    __shared__ float strains[6][Poisson ? kEndsTile : 1]; /* at the voxel's ends */
     __shared__ VoxMat svm[MatsLds ? kLdsVoxMats : 1];
     __shared__ LinkMat slm[MatsLds ? kLdsLinkMats : 1];
     const int c0 = 3 * wave; /* wave 0 integrates the translations, wave 1 the rotations */
@@ -413,25 +424,41 @@ __global__ void __launch_bounds__(6 / PerWave * kEndsTile) __attribute__((amdgpu
         for (int dir = PerWave * wave; dir < PerWave * (wave + 1); dir++) {
             if (PerWave > 1) o = s.vnbr[dir * nv + i];
             dvec f = dv(0.0, 0.0, 0.0), mm = dv(0.0, 0.0, 0.0);
+            float strain = 0.0f;
             if (o >= 0) {
                 LinkIn in;
                 if ((dir & 1) == 0) {
                     link_load<true, Poisson>(s, i, o, dir, in);
-                    link_end<false, true, Poisson, true>(s, in, i, o, mi, dir, rob, prevDt, tempI, pos0, q0, f, mm);
+                    link_end<false, true, Poisson, true>(s, in, i, o, mi, dir, rob, prevDt, tempI, pos0, q0, f, mm, strain);
                 } else {
                     link_load<false, Poisson>(s, i, o, dir, in);
-                    link_end<false, false, Poisson, true>(s, in, i, o, mi, dir, rob, prevDt, tempI, pos0, q0, f, mm);
+                    link_end<false, false, Poisson, true>(s, in, i, o, mi, dir, rob, prevDt, tempI, pos0, q0, f, mm, strain);
                 }
             } else if (s.storeForces) {
                 for (int c = 0; c < 6; c++) s.vf[vf_index(dir, c, nv, i)] = 0.0;
             }
             ends[dir][0][lane] = f.x; ends[dir][1][lane] = f.y; ends[dir][2][lane] = f.z;
             ends[dir][3][lane] = mm.x; ends[dir][4][lane] = mm.y; ends[dir][5][lane] = mm.z;
+            if (Poisson && o >= 0 && s.psNext)
+                strains[dir][lane] = axial_strain_end(strain, s.lratio[(dir >> 1) * nv + ((dir & 1) ? o : i)], (dir & 1) != 0);
         }
     }
     __syncthreads();
     if (!live) return;
     if (wave == 2) next_temperature(s, i, rob, dt);
+    if (Poisson && wave == 2 && s.psNext) {
+        /* the next step's Poisson strain (a voxel that k_poisson_fp64 would leave keeps its own) */
+        const VoxMat& m = s.vmats[mi];
+        const uint32_t fl = s.vflIn[i];
+        const int e = s.vext[i];
+        const ExtRec* ex = e >= 0 ? &s.exts[e] : nullptr;
+        float ps[3];
+        if (m.nu != 0.0f && (fl & (0x3Fu * VF_LINK0)) && !(ex && (ex->dof & 0x3F) == 0x3F))
+            poisson_strain(m, ex, fl, [&](int dir) { return strains[dir][lane]; }, ps);
+        else
+            for (int c = 0; c < 3; c++) ps[c] = s.vps[c * nv + i];
+        for (int c = 0; c < 3; c++) s.vpsOut[c * nv + i] = ps[c];
+    }
     if (wave > 1) return;
     if (PerWave > 1) {
         mom = dv(vd[(VLX + c0) * nv + i], vd[(VLY + c0) * nv + i], vd[(VLZ + c0) * nv + i]);
@@ -474,7 +501,9 @@ __global__ void __launch_bounds__(6 / PerWave * kEndsTile) __attribute__((amdgpu
     if (ex) voxel_fix_translation(m, ex, s.vijk, nv, i, pos, lin);
     out[VPX * nv + i] = pos.x; out[VPY * nv + i] = pos.y; out[VPZ * nv + i] = pos.z;
     out[VLX * nv + i] = lin.x; out[VLY * nv + i] = lin.y; out[VLZ * nv + i] = lin.z;
-    s.vflOut[i] = flags & ~(uint32_t)VF_PS_VALID; /* poissonsStrainInvalid = true (VX_Voxel.cpp:231) */
+    /* poissonsStrainInvalid = true (VX_Voxel.cpp:231); the next step's strain is valid again */
+    const bool psValid = Poisson && s.psNext && m.nu != 0.0f && (flags & (0x3Fu * VF_LINK0));
+    s.vflOut[i] = psValid ? flags | VF_PS_VALID : flags & ~(uint32_t)VF_PS_VALID;
     if (Driven && s.haltTest) halt_if_stale(s.halt, s.k + 1, s.colLast, s.recalcSq, s.vflIn, nv, i, pos.x, pos.y, pos.z);
 }
 

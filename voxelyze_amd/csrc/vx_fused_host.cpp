@@ -31,7 +31,8 @@ uint64_t graph_key(const void* args, size_t n, int path, int nsteps, int flags);
 /* the "out" half of the voxel and link state, and the saved link state of diverged robots */
 bool Sim::fusedFp64Buffers() {
     const size_t vc = (size_t)std::max(nv(), 1), sc = 3 * vc;
-    if (!bvdAlt.ensure((size_t)VD_COUNT * vc * 8) || !bvflAlt.ensure(vc * 4) || !bvtempAlt.ensure(vc * 4) || !bldAlt.ensure((size_t)LDEV_COUNT * sc * 8) ||
+    if (!bvdAlt.ensure((size_t)VD_COUNT * vc * 8) || !bvflAlt.ensure(vc * 4) || !bvtempAlt.ensure(vc * 4) ||
+        (poisson && !bvpsAlt.ensure(3 * vc * 4)) || !bldAlt.ensure((size_t)LDEV_COUNT * sc * 8) ||
         !blfAlt.ensure((size_t)LF_COUNT * sc * 4) || !blflAlt.ensure(sc * 4) || !bldSide.ensure((size_t)LDEV_COUNT * sc * 8) ||
         !blfSide.ensure((size_t)LF_COUNT * sc * 4) || !blflSide.ensure(sc * 4)) {
         err = "device allocation failed";
@@ -46,6 +47,12 @@ void Sim::swapTemps() {
     dp.vtemp = (float*)bvtemp.p;
 }
 
+void Sim::swapPoisson() {
+    std::swap(bvps.p, bvpsAlt.p);
+    std::swap(bvps.bytes, bvpsAlt.bytes);
+    dp.vps = (float*)bvps.p;
+}
+
 /* the step's output state becomes the current one */
 void Sim::swapFp64Buffers() {
     auto sw = [](DevBuf& a, DevBuf& b) {
@@ -55,6 +62,7 @@ void Sim::swapFp64Buffers() {
     sw(bvd, bvdAlt);
     sw(bvflags, bvflAlt);
     if (actOn) swapTemps(); /* the next step's temperatures (fusedFp64Finish) */
+    if (psInStep) swapPoisson();
     sw(brtime, brtimeAlt);
     sw(bld, bldAlt);
     sw(blf, blfAlt);
@@ -76,6 +84,8 @@ bool Sim::stepFp64Fused(int nsteps) {
         nearbyStale = true;
     }
     if (!fusedFp64Buffers()) return false;
+    const bool ends = endsPath(3, kEndsMaxFp64);
+    psInStep = ends && poisson;
     FusedPtrs fp{};
     fp.nv = nv();
     fp.nl = 3 * nv();
@@ -106,12 +116,14 @@ bool Sim::stepFp64Fused(int nsteps) {
     fp.actAmp = actAmp;
     fp.actFreq = actFreq;
     fp.poisson = dp.poisson;
-    fp.vps = dp.vps;
+    fp.lratio = dp.lratio;
     auto bind = [&](FusedPtrs& a) {
         a.vdIn = dp.vd;
         a.vdOut = (double*)bvdAlt.p;
         a.vflIn = dp.vflags;
         a.vflOut = (uint32_t*)bvflAlt.p;
+        a.vps = dp.vps;
+        a.vpsOut = psInStep ? (float*)bvpsAlt.p : nullptr;
         a.vtempIn = dp.vtemp;
         a.vtempOut = (float*)bvtempAlt.p;
         a.ldIn = dp.ld;
@@ -123,7 +135,6 @@ bool Sim::stepFp64Fused(int nsteps) {
         a.rtimeIn = dp.rtime;
         a.rtimeOut = (float*)brtimeAlt.p;
     };
-    const bool ends = endsPath(3, kEndsMaxFp64);
     const bool tune = !ends && tuning(3);
     const bool timed = profiling || tune;
     const bool graph = useGraphs && !collisions && !timed && nsteps > 1 && nsteps <= kGraphMaxStepsFused;
@@ -151,6 +162,10 @@ bool Sim::stepFp64Fused(int nsteps) {
         if (moved) swapTemps();
         bind(fp);
         launch_fused_temps(fp, moved, stream);
+    }
+    if (psInStep && (bvps.p > bvpsAlt.p) != (bvd.p > bvdAlt.p)) { /* the same for the Poisson strains */
+        HIPCHK(hipMemcpyAsync(bvpsAlt.p, dp.vps, (size_t)12 * nv(), hipMemcpyDeviceToDevice, stream));
+        swapPoisson();
     }
     uint64_t key = 0;
     if (graph) {
@@ -218,10 +233,10 @@ bool Sim::stepFp64Fused(int nsteps) {
         fp.colLast = collisions ? cp.last : nullptr;
         fp.recalcSq = cp.recalcSq;
         fp.storeForces = (k == nsteps - 1 || lastStep) ? 1 : 0;
-        fp.tempNext = k < nsteps - 1 && !lastStep ? 1 : 0;
+        fp.tempNext = fp.psNext = k < nsteps - 1 && !lastStep ? 1 : 0;
         const LaunchCfg cfg = tune ? tuner[3].next(&cand[k]) : chosen;
         fp.xcd = cfg.xcd;
-        launch_poisson_fp64(dp, k, stream); /* the Poisson strains this step's links read */
+        if (!psInStep || k == 0) launch_poisson_fp64(dp, k, stream); /* the Poisson strains this step's links read */
         if (timed) (void)hipEventRecord(events[2 * k], stream);
         if (ends) launch_step_fp64_ends(fp, stream);
         else launch_step_fp64(fp, cfg.block, false, stream);
@@ -268,6 +283,7 @@ bool Sim::stepFp64Fused(int nsteps) {
 bool Sim::fusedFp64Finish(int launched) {
     const int n = nv(), R = nRobots();
     if (actOn && launched > 0) swapTemps(); /* back to the temperatures of the last step */
+    if (psInStep && launched > 0) swapPoisson();
     /* the divergence record and the clocks: when no robot diverged they are also what endLaunch
        needs, and the launch ends with this one synchronisation */
     std::vector<int> div;

@@ -203,7 +203,10 @@ __global__ void __launch_bounds__(256) k_poisson_fp64(DevPtrs s, int k) {
     if (m.nu == 0.0f) return;
     const int e = s.vext[i];
     float ps[3];
-    poisson_strain(m, e >= 0 ? &s.exts[e] : nullptr, fl, s.vnbr, s.lf, s.lratio, s.nv, s.nl, i, ps);
+    poisson_strain(m, e >= 0 ? &s.exts[e] : nullptr, fl, [&](int dir) {
+        const int slot = (dir >> 1) * s.nv + ((dir & 1) ? s.vnbr[dir * s.nv + i] : i);
+        return axial_strain_end(s.lf[LSTRAIN * s.nl + slot], s.lratio[slot], (dir & 1) != 0);
+    }, ps);
     s.vps[i] = ps[0];
     s.vps[s.nv + i] = ps[1];
     s.vps[2 * s.nv + i] = ps[2];

@@ -289,7 +289,10 @@ struct Sim {
     DevBuf bldAlt, blfAlt, blflAlt, bldSide, blfSide, blflSide;
     bool fusedFp64Buffers();
     void swapFp64Buffers();
-    void swapTemps(); /* the halves of the temperatures (actuated FP64 steps) */
+    void swapTemps();   /* the halves of the temperatures (actuated FP64 steps) */
+    void swapPoisson(); /* the halves of the Poisson strains (steps that form the next one's) */
+    bool psInStep = false;
+    DevBuf bvpsAlt;
     bool stepFp64Fused(int nsteps);
     bool fusedFp64Finish(int launched);
     int stepRobots(const float* dt, int nsteps, int* done, int* divergedAt);

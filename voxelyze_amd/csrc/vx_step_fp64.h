@@ -50,20 +50,18 @@ __device__ __forceinline__ float axial_strain_end(float strain, float ratio, boo
    result lies within one double ulp of a float rounding boundary */
 __device__ __forceinline__ float powf_rounded(float x, float y) { return (float)pow((double)x, (double)y); }
 
-/* CVX_Voxel::strain(true) (VX_Voxel.cpp:300-334): voxel i's Poisson strain from its links'
-   current strains (lf, strainRatio per slot), averaged per axis; axes not in tension take
-   (1 + strain of the tensioned axes)^-nu - 1 */
-__device__ __forceinline__ void poisson_strain(const VoxMat& m, const ExtRec* ex, uint32_t flags, const int* __restrict__ vnbr,
-                                               const float* __restrict__ lf, const float* __restrict__ lratio, int nv,
-                                               int nl, int i, float out[3]) {
+/* CVX_Voxel::strain(true) (VX_Voxel.cpp:300-334): a voxel's Poisson strain from its links' current
+   strains, averaged per axis (end(dir): the strain at its end of the link in direction dir, read
+   where the flags have the link); axes not in tension take (1 + strain of the tensioned axes)^-nu - 1 */
+template <class End>
+__device__ __forceinline__ void poisson_strain(const VoxMat& m, const ExtRec* ex, uint32_t flags, End end, float out[3]) {
     float r[3] = {0.0f, 0.0f, 0.0f};
     int nb[3] = {0, 0, 0};
+#pragma unroll
     for (int dir = 0; dir < 6; dir++) {
         if (!(flags & (VF_LINK0 << dir))) continue;
-        const int axis = dir >> 1;
-        const int slot = axis * nv + ((dir & 1) ? vnbr[dir * nv + i] : i);
-        r[axis] += axial_strain_end(lf[LSTRAIN * nl + slot], lratio[slot], (dir & 1) != 0);
-        nb[axis]++;
+        r[dir >> 1] += end(dir);
+        nb[dir >> 1]++;
     }
     bool tension[3];
     for (int a = 0; a < 3; a++) {
