@@ -662,6 +662,8 @@ struct AdjPtrs {
     double* lamT;            /* nv: dL/dT of the last voxel step */
     double* slots;           /* 6 dirs * AS_COUNT * nv */
     double* lamLink;         /* 9 * 3nv: dL/d(stored link pose p2, a1v, a2v) */
+    int* links;              /* 3 * nv: the negative voxels of the links, listed per axis */
+    int* linkCount;          /* 3 */
     double* gTheta;          /* nv */
     double* gPhase;          /* nv */
     /* self-collision: the partner lists step k used, and dL/d(each voxel's summed force) */

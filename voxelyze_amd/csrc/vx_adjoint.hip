@@ -11,9 +11,8 @@
  *   k_adj_contacts (self-collision on) one lane per voxel over its partner list: the
  *                 transpose of the pair forces it and its partners summed, kept for its
  *                 own state and parameters.
- *   k_adj_links   one lane per voxel and axis (grid.y), for the link it is the negative
- *                 end of along that axis: link_vjp, writing each end's dL/d(pose), log-modulus
- *                 and temperature
+ *   k_adj_links   one lane per link (k_adj_list lists them once per reverse pass):
+ *                 link_vjp, writing each end's dL/d(pose), log-modulus and temperature
  *                 contributions into per-voxel slots (direction 2a of the negative voxel,
  *                 2a+1 of the positive one, as the forward hands forces over) and
  *                 dL/d(the link's stored local pose) for the step before.
@@ -242,12 +241,7 @@ template <int axis>
 __device__ __forceinline__ void adj_link(const AdjPtrs& a, int n) {
     const int nv = a.nv, S = 3 * nv;
     const int slot = axis * nv + n;
-    const int p = a.vnbr[(2 * axis) * nv + n];
-    if (a.vnbr[(2 * axis + 1) * nv + n] < 0) write_slot(a, 2 * axis + 1, n, dv(0, 0, 0), qzero(), 0.0, 0.0);
-    if (p < 0) {
-        write_slot(a, 2 * axis, n, dv(0, 0, 0), qzero(), 0.0, 0.0);
-        return;
-    }
+    const int p = a.vnbr[(2 * axis) * nv + n]; /* a listed link has both ends */
     const double* vd = a.t.vd;
     const LinkMat lm = a.lmats[a.lmeta[slot]];
     VoxMat mn = a.vmats[a.vmat[n]], mp = a.vmats[a.vmat[p]];
@@ -301,38 +295,78 @@ __device__ __forceinline__ void adj_link(const AdjPtrs& a, int n) {
     write_slot(a, 2 * axis + 1, p, o.lposP, o.lqP, o.lthetaLink * wp, ltp);
 }
 
+/* The links of every axis, listed by their negative voxel, once per reverse pass: links[axis * nv ..]
+   and linkCount[axis].  The slots of the directions a voxel has no link in are zeroed here and
+   stay so: no reverse step writes them.  The order of the blocks' shares is open, but every link
+   writes its own slots only, so gradients do not depend on it.  linkCount starts at zero. */
+__global__ void __launch_bounds__(256) k_adj_list(AdjPtrs a) {
+    __shared__ int waveCount[4], base;
+    const int i = (int)blockIdx.x * 256 + (int)threadIdx.x, wave = (int)threadIdx.x >> 6, lane = (int)threadIdx.x & 63;
+    const int axis = (int)blockIdx.y, nv = a.nv;
+    bool has = false;
+    if (i < nv) {
+        has = a.vnbr[(2 * axis) * nv + i] >= 0;
+        if (!has) write_slot(a, 2 * axis, i, dv(0, 0, 0), qzero(), 0.0, 0.0);
+        if (a.vnbr[(2 * axis + 1) * nv + i] < 0) write_slot(a, 2 * axis + 1, i, dv(0, 0, 0), qzero(), 0.0, 0.0);
+    }
+    const unsigned long long mask = __ballot(has);
+    if (lane == 0) waveCount[wave] = __popcll(mask);
+    __syncthreads();
+    if (threadIdx.x == 0) base = atomicAdd(&a.linkCount[axis], waveCount[0] + waveCount[1] + waveCount[2] + waveCount[3]);
+    __syncthreads();
+    int at = base + __popcll(mask & ((1ull << lane) - 1));
+    for (int w = 0; w < wave; w++) at += waveCount[w];
+    if (has) a.links[(size_t)axis * nv + at] = i;
+}
+
 /* One lane per link at 2 waves per SIMD (256 VGPRs, a few spilled): on the 2.9M-voxel
    differentiable batch over 2,000 steps, 1.72 ms per reverse step against 1.91 ms for one lane
    doing a voxel's three links, 2.76 ms at 1 wave and 3.27 ms at 3 waves; the gradient bits do
-   not change (every link writes its own slots). */
+   not change (every link writes its own slots).
+   The lanes hold listed links and no absent ones: FP64 issue (4,044 instructions a wave) and
+   register-bound residency set the time, so a lane without a link costs what one with a link
+   does.  8 bodies of 32 x 32 x 16 sites, 70 % filled (188,000 links of 275,000 voxel-axis pairs):
+   52.5 us per reverse step against 71 us for one lane per voxel and axis; building the lists is
+   21 us per reverse pass.  Blocks of the three axes over the same voxels run on one die, which
+   then reads their states once. */
 #ifndef VX_ADJ_WAVES
 #define VX_ADJ_WAVES 2
 #endif
-#ifndef VX_ADJ_LANE_PER_LINK
-#define VX_ADJ_LANE_PER_LINK 1
-#endif
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(VX_ADJ_WAVES, 8))) k_adj_links(AdjPtrs a) {
-    const int n = (int)blockIdx.x * 256 + (int)threadIdx.x;
-    if (n >= a.nv) return;
-#if VX_ADJ_LANE_PER_LINK
-    switch (blockIdx.y) {
-        case 0: adj_link<0>(a, n); break;
-        case 1: adj_link<1>(a, n); break;
-        default: adj_link<2>(a, n); break;
+    const int c0 = a.linkCount[0], c1 = a.linkCount[1], c2 = a.linkCount[2];
+    const int b0 = (c0 + 255) / 256, b1 = (c1 + 255) / 256, b2 = (c2 + 255) / 256, total = b0 + b1 + b2;
+    const int share = (total + 7) / 8; /* consecutive blocks go to the eight dies in turn */
+    int b = ((int)blockIdx.x & 7) * share + ((int)blockIdx.x >> 3);
+    if (((int)blockIdx.x >> 3) >= share || b >= total) return;
+    /* the axes in turn while each has blocks left, the rest of each after that */
+    const int m = min(b0, min(b1, b2));
+    int axis;
+    if (b < 3 * m) {
+        axis = b % 3;
+        b /= 3;
+    } else {
+        b += m - 3 * m;
+        if (b < b0) axis = 0;
+        else if ((b += m - b0) < b1) axis = 1;
+        else { axis = 2; b += m - b1; }
     }
-#else
-    adj_link<0>(a, n);
-    adj_link<1>(a, n);
-    adj_link<2>(a, n);
-#endif
+    const int at = b * 256 + (int)threadIdx.x;
+    switch (axis) {
+        case 0: if (at < c0) adj_link<0>(a, a.links[at]); break;
+        case 1: if (at < c1) adj_link<1>(a, a.links[(size_t)a.nv + at]); break;
+        default: if (at < c2) adj_link<2>(a, a.links[2 * (size_t)a.nv + at]); break;
+    }
 }
 
 void launch_adj_voxels(const AdjPtrs& a, hipStream_t st) {
     if (a.nv > 0) hipLaunchKernelGGL(k_adj_voxels, dim3((unsigned)((a.nv + 255) / 256)), dim3(256), 0, st, a);
 }
-void launch_adj_links(const AdjPtrs& a, hipStream_t st) {
+void launch_adj_list(const AdjPtrs& a, hipStream_t st) {
+    if (a.nv > 0) hipLaunchKernelGGL(k_adj_list, dim3((unsigned)((a.nv + 255) / 256), 3), dim3(256), 0, st, a);
+}
+void launch_adj_links(const AdjPtrs& a, hipStream_t st) { /* blocks past the last listed link return at once */
     if (a.nv > 0)
-        hipLaunchKernelGGL(k_adj_links, dim3((unsigned)((a.nv + 255) / 256), VX_ADJ_LANE_PER_LINK ? 3 : 1), dim3(256), 0, st, a);
+        hipLaunchKernelGGL(k_adj_links, dim3(((unsigned)((a.nv + 255) / 256) * 3 + 7) / 8 * 8), dim3(256), 0, st, a);
 }
 void launch_adj_contacts(const AdjPtrs& a, hipStream_t st) {
     if (a.nv > 0 && a.colCnt) hipLaunchKernelGGL(k_adj_contacts, dim3((unsigned)((a.nv + 255) / 256)), dim3(256), 0, st, a);

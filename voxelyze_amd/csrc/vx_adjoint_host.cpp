@@ -23,6 +23,7 @@
 namespace vx {
 
 void launch_adj_voxels(const AdjPtrs& a, hipStream_t st);
+void launch_adj_list(const AdjPtrs& a, hipStream_t st);
 void launch_adj_links(const AdjPtrs& a, hipStream_t st);
 void launch_adj_contacts(const AdjPtrs& a, hipStream_t st);
 
@@ -49,7 +50,7 @@ struct AdjointState {
     int nseg = 0;
     bool valid = false;             /* a complete rollout is recorded */
     DevBuf tapeBuf, times_d, dt_d, rprev_d;
-    DevBuf lamFinal, part, lamSum, lamT, slots, lamLink, gTheta, gPhase, lamF;
+    DevBuf lamFinal, part, lamSum, lamT, slots, lamLink, gTheta, gPhase, lamF, links;
     std::vector<std::unique_ptr<ColSnap>> colSnaps; /* partner lists of the recomputed steps */
 };
 
@@ -223,7 +224,7 @@ bool Sim::adjointBackward(const double* dLdpos, double* gThetaOut, double* gPhas
     if (!a->lamFinal.ensure(3 * n * 8) || !a->part.ensure(13 * n * 8) || !a->lamSum.ensure(6 * n * 8) ||
         !a->lamT.ensure(n * 8) || !a->slots.ensure(6 * 9 * n * 8) || !a->lamLink.ensure(9 * S * 8) ||
         !a->gTheta.ensure(n * 8) || !a->gPhase.ensure(n * 8) || !a->times_d.ensure(a->times.size() * 4) ||
-        (collisions && !a->lamF.ensure(3 * n * 8)) ||
+        !a->links.ensure((3 * n + 3) * 4) || (collisions && !a->lamF.ensure(3 * n * 8)) ||
         !a->dt_d.ensure((size_t)R * 4) || !a->rprev_d.ensure((size_t)R * 4)) {
         err = "device allocation failed (adjoint)";
         return false;
@@ -257,6 +258,7 @@ bool Sim::adjointBackward(const double* dLdpos, double* gThetaOut, double* gPhas
     HIPCHK(hipMemsetAsync(a->lamT.p, 0, n * 8, stream));
     HIPCHK(hipMemsetAsync(a->gTheta.p, 0, n * 8, stream));
     HIPCHK(hipMemsetAsync(a->gPhase.p, 0, n * 8, stream));
+    HIPCHK(hipMemsetAsync((int*)a->links.p + 3 * n, 0, 3 * 4, stream));
 
     AdjPtrs ap{};
     ap.nv = (int)n;
@@ -285,8 +287,12 @@ bool Sim::adjointBackward(const double* dLdpos, double* gThetaOut, double* gPhas
     ap.lamLink = (double*)a->lamLink.p;
     ap.gTheta = (double*)a->gTheta.p;
     ap.gPhase = (double*)a->gPhase.p;
+    ap.links = (int*)a->links.p;
+    ap.linkCount = (int*)a->links.p + 3 * n;
     ap.lamF = collisions ? (double*)a->lamF.p : nullptr;
     if (collisions) tape.colSnaps = &a->colSnaps;
+    launch_adj_list(ap, stream);
+    HIPCHK(hipGetLastError());
     const float* times = (const float*)a->times_d.p;
     std::vector<int> done(R);
     for (int sgm = nseg - 1; sgm >= 0; sgm--) {
