@@ -134,7 +134,7 @@ static bool restore(Sim* s, const Checkpoint& c) {
     if (e != hipSuccess) return s->fail("restore", e);
     s->rtime = c.rtime;
     s->rprev = c.rprev;
-    s->hostStale = true;
+    s->stateMoved();
     return true;
 }
 
@@ -150,7 +150,7 @@ static bool restoreInto(Sim* s, const Checkpoint& c, const MixTape& t) {
     if (!restoreContacts(s, c)) return false;
     s->rtime = c.rtime;
     s->rprev = c.rprev;
-    s->hostStale = true;
+    s->stateMoved();
     return true;
 }
 

@@ -104,17 +104,7 @@ API int vxg_linear_solve(vxg_sim* h, double tol, int maxIter, int* iterations, d
 }
 
 /* CVoxelyze::resetTime (src/Voxelyze.cpp:313-321) */
-API void vxg_reset_time(vxg_sim* h) {
-    Sim* s = S(h);
-    s->syncDown();
-    for (auto& t : s->rtime) t = 0.0f;
-    for (auto& p : s->rprev) p = 0.0f;
-    for (int v = 0; v < s->nv(); v++) s->resetVoxel(v);
-    for (int l = 0; l < s->nl(); l++) s->resetLink(l);
-    s->forcesStale = false; /* every end force is zero now; the next link phase rewrites the slots */
-    s->nearbyStale = s->collisionsStale = true;
-    s->dirty |= Sim::D_VSTATE | Sim::D_LSTATE | Sim::D_TEMP | Sim::D_REST;
-}
+API void vxg_reset_time(vxg_sim* h) { S(h)->resetTime(); }
 API float vxg_current_time(vxg_sim* h) { return S(h)->rtime[S(h)->curRobot]; }
 API int vxg_collision_count(vxg_sim* h) {
     Sim* s = S(h);
@@ -503,7 +493,7 @@ API int vxg_voxel_set_modulus(vxg_sim* h, int first, int count, const float* E) 
             return 0;
         }
     }
-    s->syncDown();
+    s->actuatedTempsDown();
     for (int k = 0; k < count; k++) s->vE[first + k] = E[k];
     s->modOn = true;
     s->dirty |= Sim::D_MOD;
@@ -511,7 +501,7 @@ API int vxg_voxel_set_modulus(vxg_sim* h, int first, int count, const float* E) 
 }
 API void vxg_clear_moduli(vxg_sim* h) {
     Sim* s = S(h);
-    s->syncDown();
+    s->actuatedTempsDown();
     s->modOn = false;
     for (int v = 0; v < s->nv(); v++) s->vE[v] = s->vmat[v]->E;
     s->dirty |= Sim::D_MOD;

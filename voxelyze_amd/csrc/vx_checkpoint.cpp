@@ -149,7 +149,7 @@ bool Sim::checkpointRestore(int slot) {
     HIPCHK(hipStreamSynchronize(stream));
     rtime = c.rtime;
     rprev = c.rprev;
-    hostStale = true;
+    stateMoved();
     return true;
 }
 

@@ -412,6 +412,18 @@ struct PackPtrs {
     uint32_t* flags;
 };
 
+/* the fused step's state arrays, set to the state of a reset */
+struct ResetPtrs {
+    int nv;
+    const VoxMat* vmats;
+    const int *vmat, *vijk, *lpos;
+    double *vd, *ld;
+    uint32_t *vfl, *lfl, *mfl;
+    float *vtemp, *vtempAlt, *vprevdt, *lf;
+    void* ms;                 /* MS_COUNT * 3nv, float or double */
+    int msDouble;
+};
+
 /* a kernel launch configuration chosen by the autotuner */
 struct LaunchCfg {
     int block;  /* workgroup size */

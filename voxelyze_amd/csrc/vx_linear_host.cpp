@@ -151,7 +151,7 @@ bool Sim::linearSolve(double tol, int maxIter, int* itersOut, double* residualOu
     launch_lin_post(lp, dp.vd, dp.vijk, voxSize, stream);
     HIPCHK(hipGetLastError());
     HIPCHK(hipStreamSynchronize(stream));
-    hostStale = true;
+    stateMoved();
     return true;
 }
 

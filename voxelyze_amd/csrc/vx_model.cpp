@@ -34,6 +34,7 @@ void launch_launch_begin(const LaunchIn& one, const void* pin, int R, float* rdt
 void launch_launch_end(const int* rdiv, const float* rtime, int R, void* pin, const int* vrobot, const float* rdt,
                        float* vprevdt, int nv, hipStream_t st);
 void launch_pack_voxels(const PackPtrs& s, hipStream_t st);
+void launch_reset_state(const ResetPtrs& r, hipStream_t st);
 void launch_col_stale(const DevPtrs& s, const ContactPtrs& c, int gen, hipStream_t st);
 void launch_col_keys(const DevPtrs& s, const ContactPtrs& c, int nbuckets, hipStream_t st);
 hipError_t col_sort(const ContactPtrs& c, void* tmp, size_t* tmpBytes, hipStream_t st);
@@ -474,6 +475,7 @@ void Sim::updateRestLength(int li) {
     };
     ld[LREST][li] = 0.5 * (base(lneg[li]) + base(lpos[li]));
     dirty |= D_REST;
+    restMoved = true;
 }
 
 /* CVX_Link::reset (src/VX_Link.cpp:61-75) */
@@ -484,6 +486,45 @@ void Sim::resetLink(int li) {
     lflags[li] = LF_SMALL;
     updateRestLength(li);
     updateTransverseInfo(li);
+}
+
+/* CVoxelyze::resetTime (src/Voxelyze.cpp:313-321) */
+void Sim::resetTime() {
+    const bool there = resetOnDevice();
+    if (!there) syncDown();
+    for (auto& t : rtime) t = 0.0f;
+    for (auto& p : rprev) p = 0.0f;
+    nearbyStale = collisionsStale = true;
+    if (there) return;
+    for (int v = 0; v < nv(); v++) resetVoxel(v);
+    for (int l = 0; l < nl(); l++) resetLink(l);
+    forcesStale = false; /* every end force is zero now; the next link phase rewrites the slots */
+    dirty |= D_VSTATE | D_LSTATE | D_TEMP | D_REST;
+    linksAtReset = true;
+    restMoved = false;
+}
+/* The fused steps' state is reset where it is, and the mirror follows when it is next read.  It needs the
+   device's arrays laid out and the state in them newest or equal (nothing but phases, moduli, externals,
+   temperatures and rest lengths waits for its upload), and what the host alone keeps of the links, which a download
+   does not bring back, as a reset leaves it.  Any other reset goes through the mirror: the first one, one
+   after an edit, the split FP64 step's and those with a Poisson's ratio. */
+bool Sim::resetOnDevice() {
+    if (!fused() || (dirty & ~(unsigned)(D_PHASE | D_MOD | D_EXT | D_TEMP | D_REST)) || !linksAtReset || poisson ||
+        hasPoissonMaterial() || nv() == 0 || !ensureDevice())
+        return false;
+    ResetPtrs r{nv(), dp.vmats, dp.vmat, dp.vijk, dp.lpos, dp.vd, dp.ld, dp.vflags, dp.lflags, (uint32_t*)bmfl[lcur].p,
+                dp.vtemp, (float*)bvtempAlt.p, dp.vprevdt, dp.lf, bms[lcur].p, precision == 2};
+    launch_reset_state(r, stream);
+    if (hipGetLastError() != hipSuccess || hipStreamSynchronize(stream) != hipSuccess) return false;
+    std::fill(vtemp.begin(), vtemp.end(), 0.0f);
+    if (restMoved) {
+        const unsigned keep = dirty;
+        for (int l = 0; l < nl(); l++) updateRestLength(l);
+        dirty = keep;
+        restMoved = false;
+    }
+    hostStale = tempsAtReset = true;
+    return true;
 }
 
 /* ------------------------------------------------ Poisson's ratio != 0 (volume effects) */
@@ -1173,6 +1214,7 @@ bool Sim::syncDown() {
 bool Sim::syncForces() {
     if (!syncDown()) return false;
     if (!forcesStale) return true;
+    linksAtReset = false;
     const int n = nv(), L = nl();
     std::vector<double> f((size_t)VF_COUNT * n);
     if (n) HIPCHK(hipMemcpy(f.data(), dp.vf, (size_t)VF_COUNT * n * 8, hipMemcpyDeviceToHost));
@@ -1384,7 +1426,7 @@ bool Sim::endLaunch(int nsteps, int* done) {
         rtime[r] = t[r];
         if (done[r] > 0 && launchDt[r] != 0) rprev[r] = launchDt[r];
     }
-    hostStale = true;
+    stateMoved();
     return true;
 }
 

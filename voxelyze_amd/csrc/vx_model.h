@@ -183,6 +183,16 @@ struct Sim {
                       D_MOD = 256 };
     unsigned dirty = D_TOPO | D_MATS | D_EXT;
     bool hostStale = false; /* device holds newer dynamic state */
+    bool tempsAtReset = false; /* of that state, the mirror has the temperatures: a reset's */
+    void stateMoved() { hostStale = true; tempsAtReset = false; }
+    /* the values of a link that only the host keeps current: strain ratios, transverse areas and end
+       forces are those of a reset; rest lengths may have left theirs */
+    bool linksAtReset = false, restMoved = true;
+    void resetTime();
+    bool resetOnDevice();
+    /* moduli are not state, but setting them has always refreshed the temperatures that actuation sets on
+       the device and vxg_voxel_temperature answers from the mirror */
+    void actuatedTempsDown() { if (actOn && !tempsAtReset) syncDown(); }
     bool dtCacheValid = false;
     float dtCache = 0.0f;
     hipStream_t stream = nullptr;
@@ -335,7 +345,10 @@ struct Sim {
     void updateSurface(int vi);
     Ext* external(int vi);
     float recommendedTimeStep();
-    void materialsChanged() { dirty |= D_MATS; dtCacheValid = rdtCacheValid = false; }
+    void materialsChanged() {
+        dirty |= D_MATS;
+        dtCacheValid = rdtCacheValid = linksAtReset = false;
+    }
     /* generation of the topology: bumped by every voxel/link/robot edit, so that checkpoints
        and recorded rollouts can refuse state laid out for another topology even where the
        counts agree (a voxel removed and added again shifts every index) */
@@ -343,7 +356,7 @@ struct Sim {
     void topologyChanged(bool edited = true) {
         if (edited) topoGen++;
         dirty |= D_TOPO;
-        dtCacheValid = rdtCacheValid = false;
+        dtCacheValid = rdtCacheValid = linksAtReset = false;
         nearbyStale = collisionsStale = true;
     }
 
