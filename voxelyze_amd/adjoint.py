@@ -14,6 +14,9 @@ import numpy as np
 import torch
 
 
+PARTS = 64  # of a robot's sums in robot_com
+
+
 class Rollout(torch.autograd.Function):
     @staticmethod
     def forward(ctx, log_modulus, phase, sim, nsteps, every, dt, reset):
@@ -51,6 +54,9 @@ def robot_com(sim, pos):
     span = torch.from_numpy(np.concatenate([np.arange(f, f + c) for f, c in zip(first, count)])
                             if R else np.zeros(0, np.int64)).to(pos.device)
     w = pos[span] * m[span, None]
-    num = torch.zeros((R, 3), dtype=pos.dtype, device=pos.device).index_add_(0, idx, w)
-    den = torch.zeros(R, dtype=pos.dtype, device=pos.device).index_add_(0, idx, m[span])
-    return num / den[:, None]
+    # 64 partial sums per robot, so that the lanes of a wavefront add to different addresses: on
+    # 92,000 voxels of 8 robots the two sums took 3.7 ms with one sum per robot, 0.7 ms so
+    idx = idx * PARTS + torch.arange(len(idx), device=pos.device) % PARTS
+    num = torch.zeros((R * PARTS, 3), dtype=pos.dtype, device=pos.device).index_add_(0, idx, w)
+    den = torch.zeros(R * PARTS, dtype=pos.dtype, device=pos.device).index_add_(0, idx, m[span])
+    return num.view(R, PARTS, 3).sum(1) / den.view(R, PARTS).sum(1)[:, None]
