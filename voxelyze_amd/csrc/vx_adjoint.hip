@@ -34,11 +34,12 @@ __device__ __forceinline__ bool fully_fixed(const AdjPtrs& a, int i) {
     return e >= 0 && (a.exts[e].dof & 0x3F) == 0x3F;
 }
 
-/* 3 waves per SIMD (168 VGPRs, 64 B spilled per lane): 549 us per reverse step on the
-   2.9M-voxel differentiable batch against 558 us at 2 waves (184 VGPRs) and 598 us at 4;
-   the gradient bits do not change */
+/* Bound by the memory path: 0.8 KB of slots, state and adjoint state per voxel, the slots written by other
+   dies.  2 waves per SIMD (184 VGPRs), so that the 54 values of the link ends are in flight together:
+   22.57 ms per 200-step reverse pass of 91,000 voxels and 46.63 ms per 40 steps of 1,099,000, against 22.67
+   and 46.86 with one direction in flight at a time at 3 waves.  The gradient bits do not change. */
 #ifndef VX_ADJV_WAVES
-#define VX_ADJV_WAVES 3
+#define VX_ADJV_WAVES 2
 #endif
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(VX_ADJV_WAVES, 8))) k_adj_voxels(AdjPtrs a) {
     const int i = (int)blockIdx.x * 256 + (int)threadIdx.x;
@@ -59,19 +60,25 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(VX_ADJ
         lAng1 = dv(P[AP_ANG * nv + i], P[(AP_ANG + 1) * nv + i], P[(AP_ANG + 2) * nv + i]);
         lQ1 = dq(P[AP_Q * nv + i], P[(AP_Q + 1) * nv + i], P[(AP_Q + 2) * nv + i], P[(AP_Q + 3) * nv + i]);
         double th = 0.0, lt = a.lamT[i];
-        for (int d = 0; d < 6; d++) { /* the link ends of step k+1, in direction order */
-            const double* S = a.slots;
-            lPos1.x += S[slot_index(d, AS_POS, nv, i)];
-            lPos1.y += S[slot_index(d, AS_POS + 1, nv, i)];
-            lPos1.z += S[slot_index(d, AS_POS + 2, nv, i)];
-            lQ1.w += S[slot_index(d, AS_Q, nv, i)];
-            lQ1.x += S[slot_index(d, AS_Q + 1, nv, i)];
-            lQ1.y += S[slot_index(d, AS_Q + 2, nv, i)];
-            lQ1.z += S[slot_index(d, AS_Q + 3, nv, i)];
-            th += S[slot_index(d, AS_THETA, nv, i)];
-            lt += S[slot_index(d, AS_TEMP, nv, i)];
+        const double gTheta = a.gTheta[i];
+        double in[6][AS_COUNT]; /* the link ends of step k+1, all in flight at once */
+#pragma unroll
+        for (int d = 0; d < 6; d++)
+#pragma unroll
+            for (int c = 0; c < AS_COUNT; c++) in[d][c] = a.slots[slot_index(d, c, nv, i)];
+#pragma unroll
+        for (int d = 0; d < 6; d++) { /* summed in direction order */
+            lPos1.x += in[d][AS_POS];
+            lPos1.y += in[d][AS_POS + 1];
+            lPos1.z += in[d][AS_POS + 2];
+            lQ1.w += in[d][AS_Q];
+            lQ1.x += in[d][AS_Q + 1];
+            lQ1.y += in[d][AS_Q + 2];
+            lQ1.z += in[d][AS_Q + 3];
+            th += in[d][AS_THETA];
+            lt += in[d][AS_TEMP];
         }
-        a.gTheta[i] += th;
+        a.gTheta[i] = gTheta + th;
         if (a.vphase) { /* T = base + amp sin(2 pi f t + phase) at step k+1 */
             const double arg = 6.283185307179586 * (double)a.actFreq * (double)a.rtimeNext[rob] + (double)a.vphase[i];
             a.gPhase[i] += lt * (double)a.actAmp * cos(arg);
@@ -237,8 +244,8 @@ __device__ __forceinline__ void write_slot(const AdjPtrs& a, int d, int v, dvec 
     S[slot_index(d, AS_TEMP, nv, v)] = lt;
 }
 
-template <int axis>
-__device__ __forceinline__ void adj_link(const AdjPtrs& a, int n) {
+template <typename T>
+__device__ __forceinline__ void adj_link(const AdjPtrs& a, int axis, int n) {
     const int nv = a.nv, S = 3 * nv;
     const int slot = axis * nv + n;
     const int p = a.vnbr[(2 * axis) * nv + n]; /* a listed link has both ends */
@@ -251,13 +258,18 @@ __device__ __forceinline__ void adj_link(const AdjPtrs& a, int n) {
     in.qN = dq(vd[VQW * nv + n], vd[VQX * nv + n], vd[VQY * nv + n], vd[VQZ * nv + n]);
     in.posP = dv(vd[VPX * nv + p], vd[VPY * nv + p], vd[VPZ * nv + p]);
     in.qP = dq(vd[VQW * nv + p], vd[VQX * nv + p], vd[VQY * nv + p], vd[VQZ * nv + p]);
+    const double* LS = a.lamSum;
+    const dvec lFN = dv(LS[n], LS[nv + n], LS[2 * nv + n]), lMN = dv(LS[3 * nv + n], LS[4 * nv + n], LS[5 * nv + n]);
+    const dvec lFP = dv(LS[p], LS[nv + p], LS[2 * nv + p]), lMP = dv(LS[3 * nv + p], LS[4 * nv + p], LS[5 * nv + p]);
+    double* LL = a.lamLink;
+    const dvec lNewP2 = dv(LL[0 * S + slot], LL[1 * S + slot], LL[2 * S + slot]);
+    const dvec lNewA1 = dv(LL[3 * S + slot], LL[4 * S + slot], LL[5 * S + slot]);
+    const dvec lNewA2 = dv(LL[6 * S + slot], LL[7 * S + slot], LL[8 * S + slot]);
     const float tn = a.t.vtemp[n], tp = a.t.vtemp[p];
     const double sn = axis == 0 ? mn.sizeX : axis == 1 ? mn.sizeY : mn.sizeZ;
     const double sp = axis == 0 ? mp.sizeX : axis == 1 ? mp.sizeY : mp.sizeZ;
     in.rest = a.vphase ? 0.5 * (base_size(sn, tn, mn.alphaCTE) + base_size(sp, tp, mp.alphaCTE)) : a.lrest[slot];
-    auto old = [&](int c) -> double {
-        return a.lsDouble ? ((const double*)a.t.ls)[c * S + slot] : (double)((const float*)a.t.ls)[c * S + slot];
-    };
+    auto old = [&](int c) -> double { return ((const T*)a.t.ls)[c * S + slot]; };
     in.oldP2 = dv(old(MS_P2X), old(MS_P2Y), old(MS_P2Z));
     in.oldA1 = dv(old(MS_A1X), old(MS_A1Y), old(MS_A1Z));
     in.oldA2 = dv(old(MS_A2X), old(MS_A2Y), old(MS_A2Z));
@@ -275,13 +287,6 @@ __device__ __forceinline__ void adj_link(const AdjPtrs& a, int n) {
     const float prevDt = a.k == 0 ? a.rprev[rob] : a.rdt[rob];
     in.dmN = mn.dampNum / prevDt;
     in.dmP = mp.dampNum / prevDt;
-    const double* LS = a.lamSum;
-    const dvec lFN = dv(LS[n], LS[nv + n], LS[2 * nv + n]), lMN = dv(LS[3 * nv + n], LS[4 * nv + n], LS[5 * nv + n]);
-    const dvec lFP = dv(LS[p], LS[nv + p], LS[2 * nv + p]), lMP = dv(LS[3 * nv + p], LS[4 * nv + p], LS[5 * nv + p]);
-    double* LL = a.lamLink;
-    const dvec lNewP2 = dv(LL[0 * S + slot], LL[1 * S + slot], LL[2 * S + slot]);
-    const dvec lNewA1 = dv(LL[3 * S + slot], LL[4 * S + slot], LL[5 * S + slot]);
-    const dvec lNewA2 = dv(LL[6 * S + slot], LL[7 * S + slot], LL[8 * S + slot]);
     LinkAdjOut o;
     link_vjp(in, lFN, lMN, lFP, lMP, lNewP2, lNewA1, lNewA2, &o);
     LL[0 * S + slot] = o.lOldP2.x; LL[1 * S + slot] = o.lOldP2.y; LL[2 * S + slot] = o.lOldP2.z;
@@ -328,10 +333,13 @@ __global__ void __launch_bounds__(256) k_adj_list(AdjPtrs a) {
    does.  8 bodies of 32 x 32 x 16 sites, 70 % filled (188,000 links of 275,000 voxel-axis pairs):
    52.5 us per reverse step against 71 us for one lane per voxel and axis; building the lists is
    21 us per reverse pass.  Blocks of the three axes over the same voxels run on one die, which
-   then reads their states once. */
+   then reads their states once.  With the type of the recorded state known to the compiler (its nine
+   values in flight at once, not one after the other) and the axis not (one copy of the code, 28 KB of
+   the 64 KB instruction cache that two CUs share, and no spills): 46.5 us. */
 #ifndef VX_ADJ_WAVES
 #define VX_ADJ_WAVES 2
 #endif
+template <typename T> /* of the recorded link state */
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(VX_ADJ_WAVES, 8))) k_adj_links(AdjPtrs a) {
     const int c0 = a.linkCount[0], c1 = a.linkCount[1], c2 = a.linkCount[2];
     const int b0 = (c0 + 255) / 256, b1 = (c1 + 255) / 256, b2 = (c2 + 255) / 256, total = b0 + b1 + b2;
@@ -351,11 +359,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(VX_ADJ
         else { axis = 2; b += m - b1; }
     }
     const int at = b * 256 + (int)threadIdx.x;
-    switch (axis) {
-        case 0: if (at < c0) adj_link<0>(a, a.links[at]); break;
-        case 1: if (at < c1) adj_link<1>(a, a.links[(size_t)a.nv + at]); break;
-        default: if (at < c2) adj_link<2>(a, a.links[2 * (size_t)a.nv + at]); break;
-    }
+    if (at < (axis == 0 ? c0 : axis == 1 ? c1 : c2)) adj_link<T>(a, axis, a.links[(size_t)axis * a.nv + at]);
 }
 
 void launch_adj_voxels(const AdjPtrs& a, hipStream_t st) {
@@ -365,8 +369,10 @@ void launch_adj_list(const AdjPtrs& a, hipStream_t st) {
     if (a.nv > 0) hipLaunchKernelGGL(k_adj_list, dim3((unsigned)((a.nv + 255) / 256), 3), dim3(256), 0, st, a);
 }
 void launch_adj_links(const AdjPtrs& a, hipStream_t st) { /* blocks past the last listed link return at once */
-    if (a.nv > 0)
-        hipLaunchKernelGGL(k_adj_links, dim3(((unsigned)((a.nv + 255) / 256) * 3 + 7) / 8 * 8), dim3(256), 0, st, a);
+    if (a.nv <= 0) return;
+    const dim3 grid(((unsigned)((a.nv + 255) / 256) * 3 + 7) / 8 * 8), block(256);
+    if (a.lsDouble) hipLaunchKernelGGL(k_adj_links<double>, grid, block, 0, st, a);
+    else hipLaunchKernelGGL(k_adj_links<float>, grid, block, 0, st, a);
 }
 void launch_adj_contacts(const AdjPtrs& a, hipStream_t st) {
     if (a.nv > 0 && a.colCnt) hipLaunchKernelGGL(k_adj_contacts, dim3((unsigned)((a.nv + 255) / 256)), dim3(256), 0, st, a);
