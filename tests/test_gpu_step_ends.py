@@ -200,3 +200,36 @@ def test_mixed_diverging_and_idle_robots(side, precision):
         done = [sim.robotStep(n, dt) for n in (7, 60, 1)]
         return np.array(done + [[sim.robotTime(r) for r in range(4)], [sim.voxel(i).temperature() for i in (0, 30, 40, 60)]])
     same_bits_pinned(build, precision, run, "robots")
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("nv", [262144, 262145, 524288])
+def test_mixed_sizes_where_the_cached_kernel_starts_and_ends(nv):
+    test_mixed_sizes_at_the_edges(MIXED, nv)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("moduli", [False, True])
+def test_mixed_step_past_the_caches(moduli):
+    """one voxel more than the cached kernel takes: a body stepped among them as it is alone"""
+    small, big = 300, 524289 - 300
+    both, alone = lattice(0, big), lattice(0, small)
+    both.addRobot()
+    n = 7
+    s = np.arange(small)
+    ijk = np.stack([s % n, (s // n) % n, s // n ** 2], 1)
+    mat = (s % 3 == 0).astype(np.int32)
+    both.setVoxels(mat, ijk)
+    alone.addRobot()
+    alone.setVoxels(mat, ijk)
+    states = []
+    for sim in (both, alone):
+        sim.setPrecision(MIXED)
+        if moduli:
+            E = np.full(sim.voxelCount(), 1e6, np.float32)
+            E[-small:] = 1e6 * (0.5 + W.uniform(7, np.arange(small, dtype=np.uint64)))
+            sim.setModuli(E)
+        sim.robotStep(9, np.full(2, 1e-5, np.float32))
+        states.append(sim.state(sim.voxelCount() - small, small))
+    for k, v in states[0].items():
+        assert v.tobytes() == states[1][k].tobytes(), k

@@ -203,6 +203,9 @@ __device__ __forceinline__ void put(T* p, T v) {
     else st_nt(p, v);
 }
 
+/* largest model whose mixed step stores through the caches */
+constexpr int kMixedCachedMax = 524288;
+
 /* the step kernels that split a voxel's link directions over waves take tiles of 64 voxels; their
    widest form has one wave for each of the six, and one such workgroup finds room on a CU */
 constexpr int kEndsTile = 64;

@@ -596,8 +596,12 @@ __device__ __forceinline__ void plain(MixPtrs& s) {
 /* Batch: instances for contact-batch steps whose successor is in the batch, which test the
    watch list on the positions they write; the others carry no part of that test.
    Plain: no actuation, per-voxel moduli, contacts or tape, nor their registers (1M-site lattice:
-   193 us a step without this instance, 180 with it). */
-template <typename T, bool Batch, bool Plain>
+   193 us a step without this instance, 180 with it).
+   Cached: the new state goes through the caches, not past them, where both copies of it (550 bytes a voxel)
+   stay in the 256 MB Infinity Cache until the next step.  us per step past / through: plain 378,112
+   voxels 68.5 / 56.6, 467,338: 92.5 / 84.2, 593,979: 119 / 126, 943,896: 181 / 192; actuated populations
+   323,960: 105.5 / 98.5, 485,940: 158.5 / 155.2, 566,930: 177.5 / 183.2. */
+template <typename T, bool Batch, bool Plain, bool Cached>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(VX_FUSED_WAVES, 8))) k_step_mixed(MixPtrs s) {
     if (Plain) plain(s);
     const int i = lane_index(s.xcd);
@@ -630,7 +634,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(VX_FUS
         const int o = s.vnbr[dir * nv + i];
         if (o < 0) continue;
         dvec f, mm;
-        mix_end<T, 0, false>(s, i, o, mi, dir, rob, prevDt, tempI, pos0, q0, &f, &mm);
+        mix_end<T, 0, Cached>(s, i, o, mi, dir, rob, prevDt, tempI, pos0, q0, &f, &mm);
         lf.x += f.x; lf.y += f.y; lf.z += f.z;
         lm.x += mm.x; lm.y += mm.y; lm.z += mm.z;
     }
@@ -664,12 +668,12 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(VX_FUS
         mix_fix_translation(s, v.m, ex, i, pos, lin);
         mix_fix_rotation(ex, ang, q);
     }
-    st_nt(&out[VPX * nv + i], pos.x); st_nt(&out[VPY * nv + i], pos.y); st_nt(&out[VPZ * nv + i], pos.z);
-    st_nt(&out[VLX * nv + i], lin.x); st_nt(&out[VLY * nv + i], lin.y); st_nt(&out[VLZ * nv + i], lin.z);
-    st_nt(&out[VAX * nv + i], ang.x); st_nt(&out[VAY * nv + i], ang.y); st_nt(&out[VAZ * nv + i], ang.z);
-    st_nt(&out[VQW * nv + i], q.w); st_nt(&out[VQX * nv + i], q.x); st_nt(&out[VQY * nv + i], q.y);
-    st_nt(&out[VQZ * nv + i], q.z);
-    st_nt(&s.vflOut[i], flags);
+    put<Cached>(&out[VPX * nv + i], pos.x); put<Cached>(&out[VPY * nv + i], pos.y); put<Cached>(&out[VPZ * nv + i], pos.z);
+    put<Cached>(&out[VLX * nv + i], lin.x); put<Cached>(&out[VLY * nv + i], lin.y); put<Cached>(&out[VLZ * nv + i], lin.z);
+    put<Cached>(&out[VAX * nv + i], ang.x); put<Cached>(&out[VAY * nv + i], ang.y); put<Cached>(&out[VAZ * nv + i], ang.z);
+    put<Cached>(&out[VQW * nv + i], q.w); put<Cached>(&out[VQX * nv + i], q.x); put<Cached>(&out[VQY * nv + i], q.y);
+    put<Cached>(&out[VQZ * nv + i], q.z);
+    put<Cached>(&s.vflOut[i], flags);
     if (Batch && s.haltTest) halt_if_stale(s.halt, s.k + 1, s.colLast, s.recalcSq, s.vflIn, nv, i, pos.x, pos.y, pos.z);
 }
 
@@ -678,8 +682,8 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(VX_FUS
    LDS; wave 0 integrates the translations, wave 1 the rotations, wave 2 sets the next
    temperatures.  The same bits as k_step_mixed.  us per step of a two-material lattice,
    k_step_mixed at its best launch shape -> here, in float: 290 voxels 16.2 -> 6.1, 14,048 voxels
-   17.5 -> 6.2 (PerWave 1), 17,676 voxels 18.0 -> 10.4, 112,451 voxels 29.0 -> 23.8, 332,769 voxels
-   67.7 -> 59.8 (PerWave 2); in double: 290 voxels 19.2 -> 6.8, 45,352 voxels 28.0 -> 18.9. */
+   17.5 -> 6.2 (PerWave 1), 17,676 voxels 18.0 -> 10.4, 107,926 voxels 25.3 -> 23.2, 241,914 voxels
+   45.9 -> 45.7 (PerWave 2); in double: 290 voxels 19.2 -> 6.8, 45,352 voxels 28.0 -> 18.9. */
 template <typename T, int PerWave, bool Batch, bool Plain>
 __global__ void __launch_bounds__(6 / PerWave * kEndsTile) __attribute__((amdgpu_waves_per_eu(PerWave == 1 ? 2 : 3, 8))) k_step_mixed_ends(MixPtrs s) {
     if (Plain) plain(s);
@@ -798,13 +802,16 @@ void launch_step_mixed(const MixPtrs& s, bool fp64, int block, hipStream_t st) {
     if (s.nv <= 0) return;
     const dim3 grid((unsigned)((s.nv + block - 1) / block));
     const bool plain = !s.vE && !s.vphase && !s.tapeSums && !s.colCnt;
+    const bool cached = s.nv <= kMixedCachedMax;
     if (fp64) {
-        if (s.haltTest) hipLaunchKernelGGL((k_step_mixed<double, true, false>), grid, dim3(block), 0, st, s);
-        else hipLaunchKernelGGL((k_step_mixed<double, false, false>), grid, dim3(block), 0, st, s);
+        if (s.haltTest) hipLaunchKernelGGL((k_step_mixed<double, true, false, false>), grid, dim3(block), 0, st, s);
+        else hipLaunchKernelGGL((k_step_mixed<double, false, false, false>), grid, dim3(block), 0, st, s);
     } else {
-        if (s.haltTest) hipLaunchKernelGGL((k_step_mixed<float, true, false>), grid, dim3(block), 0, st, s);
-        else if (plain) hipLaunchKernelGGL((k_step_mixed<float, false, true>), grid, dim3(block), 0, st, s);
-        else hipLaunchKernelGGL((k_step_mixed<float, false, false>), grid, dim3(block), 0, st, s);
+        if (s.haltTest) hipLaunchKernelGGL((k_step_mixed<float, true, false, false>), grid, dim3(block), 0, st, s);
+        else if (plain && cached) hipLaunchKernelGGL((k_step_mixed<float, false, true, true>), grid, dim3(block), 0, st, s);
+        else if (plain) hipLaunchKernelGGL((k_step_mixed<float, false, true, false>), grid, dim3(block), 0, st, s);
+        else if (cached) hipLaunchKernelGGL((k_step_mixed<float, false, false, true>), grid, dim3(block), 0, st, s);
+        else hipLaunchKernelGGL((k_step_mixed<float, false, false, false>), grid, dim3(block), 0, st, s);
     }
 }
 

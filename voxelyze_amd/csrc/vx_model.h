@@ -268,10 +268,12 @@ struct Sim {
        282,309 voxels 68.2 / 63.4, 332,769 voxels 77.5 / 82.2, 943,896 voxels 226 / 251). */
     bool endsPath(int t, int maxVoxels);
     static constexpr int kEndsMaxFp64 = 294912;
-    /* the mixed step's state is smaller (368,744 voxels: k_step_mixed 69.7, k_step_mixed_ends 69.1;
-       387,158: 73.0 / 75.4), the FP64 fused step's form with three waves runs short of registers
-       (112,451 voxels 41.5 / 38.1, 235,932: 84.8 / 91.1) */
-    static constexpr int kEndsMaxMixed = 368640, kEndsMaxFused64 = 131072;
+    /* the mixed step up to where its kernel with a voxel per lane fills the chip (us per step of
+       k_step_mixed / k_step_mixed_ends: 107,926 voxels 25.3 / 23.2, 241,914: 45.9 / 45.7, 324,084:
+       55.5 / 59.0, 364,607: 59.9 / 71.5; actuated populations 242,970: 82.0 / 80.9, 323,960: 98.5 /
+       103.9); the FP64 fused step's form with three waves runs short of registers (112,451 voxels
+       41.5 / 38.1, 235,932: 84.8 / 91.1) */
+    static constexpr int kEndsMaxMixed = 262144, kEndsMaxFused64 = 131072;
     /* kernel timing */
     bool profiling = false;
     std::vector<hipEvent_t> events;
