@@ -523,7 +523,7 @@ bool Sim::resetOnDevice() {
         dirty = keep;
         restMoved = false;
     }
-    hostStale = tempsAtReset = true;
+    hostStale = tempsAtReset = resetFresh = true;
     return true;
 }
 
@@ -1163,6 +1163,7 @@ bool Sim::syncUp() {
     }
     HIPCHK(hipStreamSynchronize(stream));
     dirty = 0;
+    resetFresh = false;
     return true;
 }
 
@@ -1647,7 +1648,7 @@ bool Sim::robotComNoAlloc(double* com) {
         err = "vxg_robot_com_noalloc handles at most 65536 robots (its staging array's size)";
         return false;
     }
-    if (!stream || !scratchPtr || dirty != 0 || !brfirst.p || !dp.vd) {
+    if (!stream || !scratchPtr || dirty != 0 || resetFresh || !brfirst.p || !dp.vd) {
         err = "vxg_robot_com_noalloc needs the state resident on the device with no pending edits: "
               "step, or call vxg_robot_com, once first";
         return false;

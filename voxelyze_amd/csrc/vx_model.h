@@ -188,6 +188,7 @@ struct Sim {
     /* the values of a link that only the host keeps current: strain ratios, transverse areas and end
        forces are those of a reset; rest lengths may have left theirs */
     bool linksAtReset = false, restMoved = true;
+    bool resetFresh = false; /* a reset waits for its first step, as one through the mirror does */
     void resetTime();
     bool resetOnDevice();
     /* moduli are not state, but setting them has always refreshed the temperatures that actuation sets on
