@@ -543,8 +543,8 @@ def bench_adjoint(n_robots, steps):
     sim.adjointBackward(dl)
     sim.resetTime()
     sim.robotStep(steps)  # records the forward's step graph outside the timing
-    # resetTime rewrites the state on the host; robotCom uploads it (outside the timing) so that
-    # both timed forwards start from a resident state, as the backward does
+    # robotCom uploads what a reset through the host mirror leaves pending (outside the timing), so
+    # that both timed forwards start from a resident state, as the backward does
     sim.resetTime()
     sim.robotCom()
     torch.cuda.synchronize()
