@@ -664,6 +664,7 @@ struct AdjPtrs {
     double* lamLink;         /* 9 * 3nv: dL/d(stored link pose p2, a1v, a2v) */
     int* links;              /* 3 * nv: the negative voxels of the links, listed per axis */
     int* linkCount;          /* 3 */
+    int* linkShare;          /* 3 * (workgroups of 256 voxels) */
     double* gTheta;          /* nv */
     double* gPhase;          /* nv */
     /* self-collision: the partner lists step k used, and dL/d(each voxel's summed force) */

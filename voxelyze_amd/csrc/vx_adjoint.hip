@@ -34,15 +34,19 @@ __device__ __forceinline__ bool fully_fixed(const AdjPtrs& a, int i) {
     return e >= 0 && (a.exts[e].dof & 0x3F) == 0x3F;
 }
 
-/* Bound by the memory path: 0.8 KB of slots, state and adjoint state per voxel, the slots written by other
-   dies.  2 waves per SIMD (184 VGPRs), so that the 54 values of the link ends are in flight together:
-   22.57 ms per 200-step reverse pass of 91,000 voxels and 46.63 ms per 40 steps of 1,099,000, against 22.67
-   and 46.86 with one direction in flight at a time at 3 waves.  The gradient bits do not change. */
+/* Bound by the memory path: 0.8 KB of slots, state and adjoint state per voxel.  The dies take the
+   voxels whose links they evaluated, from the last to the first, as the link kernel leaves the last
+   slots it wrote in the caches: us per reverse pass step of both kernels, first to last / last to
+   first, 412 / 395 at 733,061 voxels, 1,668 / 1,659 at 2,932,965; 92,000 voxels 22.1 / 21.9 ms per
+   200-step pass.  2 waves per SIMD (184 VGPRs) hold the 54 values of the link ends in flight together;
+   one direction at a time at 3 waves was within 1 %.  The gradient bits do not change. */
 #ifndef VX_ADJV_WAVES
 #define VX_ADJV_WAVES 2
 #endif
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(VX_ADJV_WAVES, 8))) k_adj_voxels(AdjPtrs a) {
-    const int i = (int)blockIdx.x * 256 + (int)threadIdx.x;
+    /* each die from the last workgroup of its share of the voxels to the first */
+    const int x = (int)blockIdx.x & 7, q = (int)gridDim.x >> 3, r = (int)gridDim.x & 7;
+    const int i = (x * q + min(x, r) + q + (x < r) - 1 - ((int)blockIdx.x >> 3)) * 256 + (int)threadIdx.x;
     const int nv = a.nv;
     if (i >= nv) return;
     const int rob = a.vrobot[i];
@@ -300,42 +304,57 @@ __device__ __forceinline__ void adj_link(const AdjPtrs& a, int axis, int n) {
     write_slot(a, 2 * axis + 1, p, o.lposP, o.lqP, o.lthetaLink * wp, ltp);
 }
 
-/* The links of every axis, listed by their negative voxel, once per reverse pass: links[axis * nv ..]
-   and linkCount[axis].  The slots of the directions a voxel has no link in are zeroed here and
-   stay so: no reverse step writes them.  The order of the blocks' shares is open, but every link
-   writes its own slots only, so gradients do not depend on it.  linkCount starts at zero. */
-__global__ void __launch_bounds__(256) k_adj_list(AdjPtrs a) {
-    __shared__ int waveCount[4], base;
-    const int i = (int)blockIdx.x * 256 + (int)threadIdx.x, wave = (int)threadIdx.x >> 6, lane = (int)threadIdx.x & 63;
-    const int axis = (int)blockIdx.y, nv = a.nv;
+/* The links of every axis, listed by their negative voxel in voxel order, once per reverse pass:
+   links[axis * nv ..] and linkCount[axis].  The slots of the directions a voxel has no link in are
+   zeroed here and stay so: no reverse step writes them.  k_adj_count leaves each workgroup's share of
+   an axis, k_adj_list adds up the shares before its own. */
+__global__ void __launch_bounds__(256) k_adj_count(AdjPtrs a) {
+    const int i = (int)blockIdx.x * 256 + (int)threadIdx.x, axis = (int)blockIdx.y, nv = a.nv;
     bool has = false;
     if (i < nv) {
         has = a.vnbr[(2 * axis) * nv + i] >= 0;
         if (!has) write_slot(a, 2 * axis, i, dv(0, 0, 0), qzero(), 0.0, 0.0);
         if (a.vnbr[(2 * axis + 1) * nv + i] < 0) write_slot(a, 2 * axis + 1, i, dv(0, 0, 0), qzero(), 0.0, 0.0);
     }
+    const int n = __syncthreads_count(has);
+    if (threadIdx.x == 0) a.linkShare[axis * gridDim.x + blockIdx.x] = n;
+}
+__global__ void __launch_bounds__(256) k_adj_list(AdjPtrs a) {
+    __shared__ int before[4], waveCount[4];
+    const int i = (int)blockIdx.x * 256 + (int)threadIdx.x, wave = (int)threadIdx.x >> 6, lane = (int)threadIdx.x & 63;
+    const int axis = (int)blockIdx.y, nv = a.nv;
+    int sum = 0;
+    for (int b = (int)threadIdx.x; b < (int)blockIdx.x; b += 256) sum += a.linkShare[axis * gridDim.x + b];
+    for (int o = 32; o > 0; o >>= 1) sum += __shfl_xor(sum, o);
+    const bool has = i < nv && a.vnbr[(2 * axis) * nv + i] >= 0;
     const unsigned long long mask = __ballot(has);
-    if (lane == 0) waveCount[wave] = __popcll(mask);
+    if (lane == 0) {
+        before[wave] = sum;
+        waveCount[wave] = __popcll(mask);
+    }
     __syncthreads();
-    if (threadIdx.x == 0) base = atomicAdd(&a.linkCount[axis], waveCount[0] + waveCount[1] + waveCount[2] + waveCount[3]);
-    __syncthreads();
-    int at = base + __popcll(mask & ((1ull << lane) - 1));
+    int at = before[0] + before[1] + before[2] + before[3];
+    if (blockIdx.x == gridDim.x - 1 && threadIdx.x == 0)
+        a.linkCount[axis] = at + waveCount[0] + waveCount[1] + waveCount[2] + waveCount[3];
     for (int w = 0; w < wave; w++) at += waveCount[w];
-    if (has) a.links[(size_t)axis * nv + at] = i;
+    if (has) a.links[(size_t)axis * nv + at + __popcll(mask & ((1ull << lane) - 1))] = i;
 }
 
-/* One lane per link at 2 waves per SIMD (256 VGPRs, a few spilled): on the 2.9M-voxel
+/* One lane per link at 2 waves per SIMD (256 VGPRs): on the 2.9M-voxel
    differentiable batch over 2,000 steps, 1.72 ms per reverse step against 1.91 ms for one lane
    doing a voxel's three links, 2.76 ms at 1 wave and 3.27 ms at 3 waves; the gradient bits do
    not change (every link writes its own slots).
    The lanes hold listed links and no absent ones: FP64 issue (4,044 instructions a wave) and
    register-bound residency set the time, so a lane without a link costs what one with a link
    does.  8 bodies of 32 x 32 x 16 sites, 70 % filled (188,000 links of 275,000 voxel-axis pairs):
-   52.5 us per reverse step against 71 us for one lane per voxel and axis; building the lists is
-   21 us per reverse pass.  Blocks of the three axes over the same voxels run on one die, which
-   then reads their states once.  With the type of the recorded state known to the compiler (its nine
-   values in flight at once, not one after the other) and the axis not (one copy of the code, 28 KB of
-   the 64 KB instruction cache that two CUs share, and no spills): 46.5 us. */
+   52.5 us per reverse step against 71 us for one lane per voxel and axis.  Blocks of the three axes
+   over the same voxels run on one die, which then reads their states once.  With the type of the
+   recorded state known to the compiler (its nine values in flight at once, not one after the other)
+   and the axis not (one copy of the code, 28 KB of the 64 KB instruction cache that two CUs share, and
+   no spills): 46.5 us, 43.7 with the lists in voxel order.  They are in that order because
+   neighbouring waves share the cache lines at their ends: 2,932,965 voxels 1,337 us with the
+   workgroups' shares in any order, 1,091 in order (one lane per voxel and axis: 1,289).  Building
+   them is 18 us per reverse pass. */
 #ifndef VX_ADJ_WAVES
 #define VX_ADJ_WAVES 2
 #endif
@@ -366,7 +385,10 @@ void launch_adj_voxels(const AdjPtrs& a, hipStream_t st) {
     if (a.nv > 0) hipLaunchKernelGGL(k_adj_voxels, dim3((unsigned)((a.nv + 255) / 256)), dim3(256), 0, st, a);
 }
 void launch_adj_list(const AdjPtrs& a, hipStream_t st) {
-    if (a.nv > 0) hipLaunchKernelGGL(k_adj_list, dim3((unsigned)((a.nv + 255) / 256), 3), dim3(256), 0, st, a);
+    if (a.nv <= 0) return;
+    const dim3 grid((unsigned)((a.nv + 255) / 256), 3);
+    hipLaunchKernelGGL(k_adj_count, grid, dim3(256), 0, st, a);
+    hipLaunchKernelGGL(k_adj_list, grid, dim3(256), 0, st, a);
 }
 void launch_adj_links(const AdjPtrs& a, hipStream_t st) { /* blocks past the last listed link return at once */
     if (a.nv <= 0) return;

@@ -224,7 +224,7 @@ bool Sim::adjointBackward(const double* dLdpos, double* gThetaOut, double* gPhas
     if (!a->lamFinal.ensure(3 * n * 8) || !a->part.ensure(13 * n * 8) || !a->lamSum.ensure(6 * n * 8) ||
         !a->lamT.ensure(n * 8) || !a->slots.ensure(6 * 9 * n * 8) || !a->lamLink.ensure(9 * S * 8) ||
         !a->gTheta.ensure(n * 8) || !a->gPhase.ensure(n * 8) || !a->times_d.ensure(a->times.size() * 4) ||
-        !a->links.ensure((3 * n + 3) * 4) || (collisions && !a->lamF.ensure(3 * n * 8)) ||
+        !a->links.ensure((3 * n + 3 + 3 * ((n + 255) / 256)) * 4) || (collisions && !a->lamF.ensure(3 * n * 8)) ||
         !a->dt_d.ensure((size_t)R * 4) || !a->rprev_d.ensure((size_t)R * 4)) {
         err = "device allocation failed (adjoint)";
         return false;
@@ -258,7 +258,6 @@ bool Sim::adjointBackward(const double* dLdpos, double* gThetaOut, double* gPhas
     HIPCHK(hipMemsetAsync(a->lamT.p, 0, n * 8, stream));
     HIPCHK(hipMemsetAsync(a->gTheta.p, 0, n * 8, stream));
     HIPCHK(hipMemsetAsync(a->gPhase.p, 0, n * 8, stream));
-    HIPCHK(hipMemsetAsync((int*)a->links.p + 3 * n, 0, 3 * 4, stream));
 
     AdjPtrs ap{};
     ap.nv = (int)n;
@@ -289,6 +288,7 @@ bool Sim::adjointBackward(const double* dLdpos, double* gThetaOut, double* gPhas
     ap.gPhase = (double*)a->gPhase.p;
     ap.links = (int*)a->links.p;
     ap.linkCount = (int*)a->links.p + 3 * n;
+    ap.linkShare = ap.linkCount + 3;
     ap.lamF = collisions ? (double*)a->lamF.p : nullptr;
     if (collisions) tape.colSnaps = &a->colSnaps;
     launch_adj_list(ap, stream);
