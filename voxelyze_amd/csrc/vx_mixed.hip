@@ -600,7 +600,8 @@ __device__ __forceinline__ void plain(MixPtrs& s) {
    Cached: the new state goes through the caches, not past them, where both copies of it (550 bytes a voxel)
    stay in the 256 MB Infinity Cache until the next step.  us per step past / through: plain 378,112
    voxels 68.5 / 56.6, 467,338: 92.5 / 84.2, 593,979: 119 / 126, 943,896: 181 / 192; actuated populations
-   323,960: 105.5 / 98.5, 485,940: 158.5 / 155.2, 566,930: 177.5 / 183.2. */
+   323,960: 105.5 / 98.5, 485,940: 158.5 / 155.2, 566,930: 177.5 / 183.2; 150 steps of a porous block
+   with contacts, 298,579 voxels: 13.7 / 12.2 ms. */
 template <typename T, bool Batch, bool Plain, bool Cached>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(VX_FUSED_WAVES, 8))) k_step_mixed(MixPtrs s) {
     if (Plain) plain(s);
@@ -807,7 +808,8 @@ void launch_step_mixed(const MixPtrs& s, bool fp64, int block, hipStream_t st) {
         if (s.haltTest) hipLaunchKernelGGL((k_step_mixed<double, true, false, false>), grid, dim3(block), 0, st, s);
         else hipLaunchKernelGGL((k_step_mixed<double, false, false, false>), grid, dim3(block), 0, st, s);
     } else {
-        if (s.haltTest) hipLaunchKernelGGL((k_step_mixed<float, true, false, false>), grid, dim3(block), 0, st, s);
+        if (s.haltTest && cached) hipLaunchKernelGGL((k_step_mixed<float, true, false, true>), grid, dim3(block), 0, st, s);
+        else if (s.haltTest) hipLaunchKernelGGL((k_step_mixed<float, true, false, false>), grid, dim3(block), 0, st, s);
         else if (plain && cached) hipLaunchKernelGGL((k_step_mixed<float, false, true, true>), grid, dim3(block), 0, st, s);
         else if (plain) hipLaunchKernelGGL((k_step_mixed<float, false, true, false>), grid, dim3(block), 0, st, s);
         else if (cached) hipLaunchKernelGGL((k_step_mixed<float, false, false, true>), grid, dim3(block), 0, st, s);
