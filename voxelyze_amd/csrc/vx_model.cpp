@@ -936,20 +936,16 @@ bool Sim::syncUp() {
     if (!ensureDevice()) return false;
     const int n = nv(), L = nl();
     if (dirty & D_TOPO) {
-        if (n > nvCap || L > nlCap || !bvd.p) {
-            int vc = std::max(n, 1), lc = std::max(L, 1);
-            const size_t sc = (size_t)3 * vc; /* link slots */
-            if (!bvd.ensure((size_t)VD_COUNT * vc * 8) || !bvf.ensure((size_t)VF_COUNT * vc * 8) ||
-                !bvflags.ensure((size_t)vc * 4) || !bvmat.ensure((size_t)vc * 4) || !bvext.ensure((size_t)vc * 4) ||
-                !bvprevdt.ensure((size_t)vc * 4) || !bvtemp.ensure((size_t)vc * 4) || !bvijk.ensure((size_t)3 * vc * 4) ||
-                !blpos.ensure(sc * 4) || !blmeta.ensure(sc * 4) || !bld.ensure((size_t)LDEV_COUNT * sc * 8) ||
-                !blf.ensure((size_t)LF_COUNT * sc * 4) || !blflags.ensure(sc * 4) || !bvps.ensure((size_t)3 * vc * 4) ||
-                !blratio.ensure(sc * 4)) {
-                err = "device allocation failed";
-                return false;
-            }
-            nvCap = vc;
-            nlCap = lc;
+        /* every array by its own size: the fused steps leave the halves of the state swapped, and a second
+           half is as large as the model was when it was first needed */
+        const size_t vc = (size_t)std::max(n, 1), sc = 3 * vc; /* voxels, link slots */
+        if (!bvd.ensure((size_t)VD_COUNT * vc * 8) || !bvf.ensure((size_t)VF_COUNT * vc * 8) || !bvflags.ensure(vc * 4) ||
+            !bvmat.ensure(vc * 4) || !bvext.ensure(vc * 4) || !bvprevdt.ensure(vc * 4) || !bvtemp.ensure(vc * 4) ||
+            !bvijk.ensure(3 * vc * 4) || !blpos.ensure(sc * 4) || !blmeta.ensure(sc * 4) ||
+            !bld.ensure((size_t)LDEV_COUNT * sc * 8) || !blf.ensure((size_t)LF_COUNT * sc * 4) || !blflags.ensure(sc * 4) ||
+            !bvps.ensure(3 * vc * 4) || !blratio.ensure(sc * 4)) {
+            err = "device allocation failed";
+            return false;
         }
         dp.nv = n;
         dp.nl = 3 * n;

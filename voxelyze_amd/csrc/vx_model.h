@@ -205,7 +205,6 @@ struct Sim {
     void launchRamps(); /* the ramps' translations at each robot's current time (dp.rtime) */
     /* the ramp table's address and length, which a captured step graph bakes in */
     int rampKey() const { return (int)(((uintptr_t)bramps.p >> 8) * 31u + (unsigned)nRamps) << 8; }
-    int nvCap = 0, nlCap = 0;
     std::vector<int> extIndex; /* compact external index per voxel, -1 none */
     std::vector<int> slotOf;   /* linksList position -> device link slot */
     bool forcesStale = false;  /* host end-force view older than the device slots */
