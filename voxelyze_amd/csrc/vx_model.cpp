@@ -1173,7 +1173,8 @@ bool Sim::syncDown() {
     if (n) HIPCHK(hipMemcpyAsync(vprevdt.data(), dp.vprevdt, (size_t)n * 4, hipMemcpyDeviceToHost, stream));
     for (int c = 0; c < 3; c++)
         if (n) HIPCHK(hipMemcpyAsync(vps[c].data(), dp.vps + (size_t)c * n, (size_t)n * 4, hipMemcpyDeviceToHost, stream));
-    if (n && actOn) HIPCHK(hipMemcpyAsync(vtemp.data(), dp.vtemp, (size_t)n * 4, hipMemcpyDeviceToHost, stream));
+    const bool temps = actOn && !tempsAtReset; /* set by the device since; after a reset the host may have set them */
+    if (n && temps) HIPCHK(hipMemcpyAsync(vtemp.data(), dp.vtemp, (size_t)n * 4, hipMemcpyDeviceToHost, stream));
     const size_t S = (size_t)3 * n;
     std::vector<double> bufD((size_t)LREST * S);
     std::vector<float> bufF((size_t)LF_COUNT * S);
@@ -1191,7 +1192,7 @@ bool Sim::syncDown() {
         for (int c = 0; c < (poisson ? LF_COUNT : LTAREA); c++) lf[c][l] = bufF[c * S + d];
         lflags[l] = bufU[d];
     }
-    if (actOn) { /* the temperatures the device set; rest lengths follow them */
+    if (temps) { /* the temperatures the device set; rest lengths follow them */
         const unsigned keep = dirty;
         for (int l = 0; l < L; l++) updateRestLength(l);
         dirty = keep;
