@@ -572,12 +572,12 @@ API void vxg_voxel_get_state(vxg_sim* h, int first, int count, double* pos, doub
                              uint32_t* flags) {
     Sim* s = S(h);
     if (first < 0 || count <= 0 || first + count > s->nv()) return;
-    /* after steps, a read moves just the voxel arrays it asks for and leaves the host mirror stale;
-       under actuation a whole-population read of everything refreshes the mirror, from which
-       vxg_voxel_temperature answers */
+    /* after steps, a read moves just the voxel arrays it asks for and leaves the host mirror stale (a
+       whole one is held for the reads after it); under actuation a whole-population read of everything
+       refreshes the mirror, from which vxg_voxel_temperature answers */
     const bool whole = (size_t)count * 4 >= (size_t)s->nv() && pos && orient && lin && ang;
     if (s->hostStale && !(s->actOn && whole)) {
-        s->readVoxelRange(first, count, pos, orient, lin, ang, flags);
+        s->readVoxelRange(first, count, pos, orient, lin, ang, flags, whole);
         if (flags)
             for (int k = 0; k < count; k++) flags[k] &= 0xFFu;
         return;

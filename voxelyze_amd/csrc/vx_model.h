@@ -184,7 +184,7 @@ struct Sim {
     unsigned dirty = D_TOPO | D_MATS | D_EXT;
     bool hostStale = false; /* device holds newer dynamic state */
     bool tempsAtReset = false; /* of that state, the mirror has the temperatures: a reset's */
-    void stateMoved() { hostStale = true; tempsAtReset = false; }
+    void stateMoved() { hostStale = true; tempsAtReset = rowsHeld = false; }
     /* the values of a link that only the host keeps current: strain ratios, transverse areas and end
        forces are those of a reset; rest lengths may have left theirs */
     bool linksAtReset = false, restMoved = true;
@@ -214,6 +214,11 @@ struct Sim {
     char* pin = nullptr;
     size_t pinBytes = 0;
     bool pinned(size_t bytes);
+    char* rows = nullptr; /* pinned: the state of voxels rowsFirst on as a read left it (readVoxelRange) */
+    size_t rowsBytes = 0;
+    int rowsFirst = 0, rowsCount = 0;
+    bool rowsHeld = false; /* the device's, which has not moved since */
+    bool holdRows(size_t bytes);
     bool pinFresh = false; /* pin holds this launch's final divergence record and clocks */
     DevBuf bvrobot, bvphase, brfirst, brdt, brprev, brtime, brtimeAlt, brdiv, bcom;
     /* self-collision (src/Voxelyze.cpp:670-750) */
@@ -367,7 +372,8 @@ struct Sim {
     bool syncUp();
     bool syncDown();
     bool syncForces();
-    bool readVoxelRange(int first, int count, double* pos, double* orient, double* lin, double* ang, uint32_t* flags);
+    bool readVoxelRange(int first, int count, double* pos, double* orient, double* lin, double* ang, uint32_t* flags,
+                        bool whole);
     int step(float dt, int nsteps, int* divergedAt);
     bool fail(const char* what, hipError_t e);
 };
