@@ -32,6 +32,7 @@ struct StateCheckpoint {
 void launch_copy_list(const CopyList& c, hipStream_t st);
 
 bool Sim::checkpointSave(int slot) {
+    OnDevice here(device);
     if (slot < 0 || slot >= kCheckpointSlots) {
         err = "checkpoint slot out of range";
         return false;
@@ -97,6 +98,7 @@ bool Sim::checkpointSave(int slot) {
 }
 
 bool Sim::checkpointRestore(int slot) {
+    OnDevice here(device);
     if (slot < 0 || slot >= kCheckpointSlots || !checkpoints[slot]) {
         err = "no checkpoint in that slot";
         return false;

@@ -491,6 +491,7 @@ void Sim::resetLink(int li) {
 
 /* CVoxelyze::resetTime (src/Voxelyze.cpp:313-321) */
 void Sim::resetTime() {
+    OnDevice here(device);
     const bool there = resetOnDevice();
     if (!there) syncDown();
     for (auto& t : rtime) t = 0.0f;
@@ -900,7 +901,9 @@ float Sim::recommendedTimeStep() {
 /* ============================================================ host <-> device */
 bool Sim::ensureDevice() {
     if (stream) return true;
-    hipError_t e = hipStreamCreate(&stream);
+    hipError_t e = hipGetDevice(&device);
+    if (e != hipSuccess) return fail("hipGetDevice", e);
+    e = hipStreamCreate(&stream);
     if (e != hipSuccess) return fail("hipStreamCreate", e);
     e = hipHostMalloc((void**)&ctlHost, 8 * sizeof(int), hipHostMallocDefault);
     if (e != hipSuccess) return fail("hipHostMalloc", e);
@@ -1280,6 +1283,7 @@ bool Sim::readVoxelRange(int first, int count, double* pos, double* orient, doub
     const Fields every{true, true, true, true, true};
     Fields ask{pos != nullptr, orient != nullptr, lin != nullptr, ang != nullptr, flags != nullptr};
     if (!ask.row() || count <= 0) return true;
+    OnDevice here(device);
     const bool held = rowsHeld && first >= rowsFirst && first + count <= rowsFirst + rowsCount;
     const bool hold = !held && whole && holdRows((size_t)count * every.row());
     if (hold) rowsFirst = first, rowsCount = count;

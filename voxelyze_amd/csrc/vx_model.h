@@ -98,6 +98,18 @@ struct MixTape {
     std::vector<int> colVer;
 };
 
+/* the calling thread's current device is d's for the scope: calls that launch kernels where a copy, which
+   works from any device, would also do */
+struct OnDevice {
+    int before = -1;
+    explicit OnDevice(int d) {
+        int now = -1;
+        if (d >= 0 && hipGetDevice(&now) == hipSuccess && now != d && hipSetDevice(d) == hipSuccess) before = now;
+    }
+    ~OnDevice() { if (before >= 0) (void)hipSetDevice(before); }
+    OnDevice(const OnDevice&) = delete;
+};
+
 struct StateCheckpoint;
 
 struct Sim {
@@ -197,6 +209,7 @@ struct Sim {
     bool dtCacheValid = false;
     float dtCache = 0.0f;
     hipStream_t stream = nullptr;
+    int device = -1; /* of the stream */
     DevPtrs dp{};
     DevBuf bvd, bvf, bvflags, bvmat, bvext, bvprevdt, bvtemp, bvijk, bvps, blratio;
     DevBuf blpos, blmeta, bld, blf, blflags;
