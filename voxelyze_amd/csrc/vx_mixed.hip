@@ -378,8 +378,9 @@ __device__ __forceinline__ void mix_end(const MixPtrs& s, int i, int o, int mi, 
         }
         rest = neg ? 0.5 * (bi + bo) : 0.5 * (bo + bi);
     }
+    const int mo = Early ? in.mo : -1;
     /* one call site: the negative end first */
-    link_fused<T, Early, Cached>(s, in, slot, neg ? i : o, neg ? o : i, neg ? mi : in.mo, neg ? in.mo : mi, axis, !neg, neg, rest, prevDt,
+    link_fused<T, Early, Cached>(s, in, slot, neg ? i : o, neg ? o : i, neg ? mi : mo, neg ? mo : mi, axis, !neg, neg, rest, prevDt,
                   neg ? pos0 : in.po, neg ? q0 : in.qo, neg ? in.po : pos0, neg ? in.qo : q0, f, mm);
 }
 
