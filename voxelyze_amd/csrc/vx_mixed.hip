@@ -170,24 +170,27 @@ template <typename T> struct MixIn {
     dvec po;
     dquat qo;
 };
-template <typename T, int Early>
-__device__ __forceinline__ void mix_load(const MixPtrs& s, int slot, int o, MixIn<T>& in) {
-    const int nv = s.nv, S = 3 * nv;
-    const T* ls = (const T*)s.lsIn;
+template <typename T>
+__device__ __forceinline__ void mix_pose(const MixPtrs& s, int o, MixIn<T>& in) {
+    const int nv = s.nv;
     const double* __restrict__ vd = s.vdIn;
-    if (Early) {
-        in.meta = s.lmeta[slot];
-        in.fl = s.lflIn[slot];
-        if (Early == 2)
-            for (int c = 0; c < 9; c++) in.pose[c] = ls[c * S + slot];
-        in.maxStrain = ls[MS_MAX * S + slot];
-        in.strainOffset = ls[MS_OFF * S + slot];
-        in.mo = s.vmat[o];
-        if (s.vphase) in.to = s.vtempIn[o];
-    }
-    if (!s.vphase) in.rest = s.lrest[slot];
     in.po = dv(vd[VPX * nv + o], vd[VPY * nv + o], vd[VPZ * nv + o]);
     in.qo = dq(vd[VQW * nv + o], vd[VQX * nv + o], vd[VQY * nv + o], vd[VQZ * nv + o]);
+}
+template <typename T, int Early>
+__device__ __forceinline__ void mix_load(const MixPtrs& s, int slot, int o, MixIn<T>& in) {
+    const int S = 3 * s.nv;
+    const T* ls = (const T*)s.lsIn;
+    in.meta = s.lmeta[slot];
+    in.fl = s.lflIn[slot];
+    if (Early == 2)
+        for (int c = 0; c < 9; c++) in.pose[c] = ls[c * S + slot];
+    in.maxStrain = ls[MS_MAX * S + slot];
+    in.strainOffset = ls[MS_OFF * S + slot];
+    in.mo = s.vmat[o];
+    if (s.vphase) in.to = s.vtempIn[o];
+    if (!s.vphase) in.rest = s.lrest[slot];
+    mix_pose(s, o, in);
 }
 
 /* One link (CVX_Link::updateForces, VX_Link.cpp:149-217): pose extraction in FP64, beam
@@ -349,7 +352,7 @@ __device__ void frozen_copy(const MixPtrs& s, int i, int rob, int d) {
 }
 
 /* voxel i's end of its link in direction dir to neighbour o: end force f and moment mm */
-template <typename T, int Early, bool Cached>
+template <typename T, int Early, bool Cached, bool PoseLast>
 __device__ __forceinline__ void mix_end(const MixPtrs& s, int i, int o, int mi, int dir, int rob, float prevDt, float tempI,
                                         const dvec& pos0, const dquat& q0, dvec* f, dvec* mm) {
     const int nv = s.nv;
@@ -357,8 +360,10 @@ __device__ __forceinline__ void mix_end(const MixPtrs& s, int i, int o, int mi, 
     const bool neg = (dir & 1) == 0; /* this voxel is the link's negative end */
     const int slot = neg ? axis * nv + i : axis * nv + o;
     MixIn<T> in;
-    mix_load<T, Early>(s, slot, o, in);
-    double rest = in.rest;
+    double rest = 0.0;
+    if (Early) mix_load<T, Early>(s, slot, o, in);
+    if (!s.vphase && (Early || !PoseLast)) rest = Early ? in.rest : s.lrest[slot];
+    if (!Early && !PoseLast) mix_pose(s, o, in);
     if (s.vphase) { /* actuated: rest length from the two temperatures (VX_Link.cpp:137-140) */
         const VoxMat& mt = s.vmats[mi];
         const VoxMat& mo = s.vmats[Early ? in.mo : s.vmat[o]];
@@ -377,7 +382,10 @@ __device__ __forceinline__ void mix_end(const MixPtrs& s, int i, int o, int mi, 
             bo = base_size(so, Early ? in.to : s.vtempIn[o], mo.alphaCTE);
         }
         rest = neg ? 0.5 * (bi + bo) : 0.5 * (bo + bi);
+    } else if (!Early && PoseLast) {
+        rest = s.lrest[slot];
     }
+    if (!Early && PoseLast) mix_pose(s, o, in);
     const int mo = Early ? in.mo : -1;
     /* one call site: the negative end first */
     link_fused<T, Early, Cached>(s, in, slot, neg ? i : o, neg ? o : i, neg ? mi : mo, neg ? mo : mi, axis, !neg, neg, rest, prevDt,
@@ -602,8 +610,12 @@ __device__ __forceinline__ void plain(MixPtrs& s) {
    stay in the 256 MB Infinity Cache until the next step.  us per step past / through: plain 378,112
    voxels 68.5 / 56.6, 467,338: 92.5 / 84.2, 593,979: 119 / 126, 943,896: 181 / 192; actuated populations
    323,960: 105.5 / 98.5, 485,940: 158.5 / 155.2, 566,930: 177.5 / 183.2; 150 steps of a porous block
-   with contacts, 298,579 voxels: 13.7 / 12.2 ms. */
-template <typename T, bool Batch, bool Plain, bool Cached>
+   with contacts, 298,579 voxels: 13.7 / 12.2 ms.
+   PoseLast: the neighbour's pose is asked for after the link's rest length, not before.  The order decides
+   which scalar registers the compiler spills: the Batch instances move 209 scalars between lanes so, 505 with
+   the pose first (48 steps of 700,000 voxels with contacts: 7.46 / 7.64 ms), and in double a step without
+   actuation is faster so (270,000 voxels with moduli 5.16 / 5.21 ms), one with it slower (7.94 / 7.54). */
+template <typename T, bool Batch, bool Plain, bool Cached, bool PoseLast>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(VX_FUSED_WAVES, 8))) k_step_mixed(MixPtrs s) {
     if (Plain) plain(s);
     const int i = lane_index(s.xcd);
@@ -636,7 +648,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(VX_FUS
         const int o = s.vnbr[dir * nv + i];
         if (o < 0) continue;
         dvec f, mm;
-        mix_end<T, 0, Cached>(s, i, o, mi, dir, rob, prevDt, tempI, pos0, q0, &f, &mm);
+        mix_end<T, 0, Cached, PoseLast>(s, i, o, mi, dir, rob, prevDt, tempI, pos0, q0, &f, &mm);
         lf.x += f.x; lf.y += f.y; lf.z += f.z;
         lm.x += mm.x; lm.y += mm.y; lm.z += mm.z;
     }
@@ -717,7 +729,7 @@ __global__ void __launch_bounds__(6 / PerWave * kEndsTile) __attribute__((amdgpu
         for (int dir = PerWave * wave; dir < PerWave * (wave + 1); dir++) {
             if (PerWave > 1 && dir > PerWave * wave) o = s.vnbr[dir * nv + i];
             dvec f = dv(0.0, 0.0, 0.0), mm = dv(0.0, 0.0, 0.0);
-            if (o >= 0) mix_end<T, PerWave == 1 ? 2 : sizeof(T) == 4 ? 1 : 0, true>(s, i, o, mi, dir, rob, prevDt, tempI, pos0, q0, &f, &mm);
+            if (o >= 0) mix_end<T, PerWave == 1 ? 2 : sizeof(T) == 4 ? 1 : 0, true, Batch>(s, i, o, mi, dir, rob, prevDt, tempI, pos0, q0, &f, &mm);
             ends[dir][0][lane] = (T)f.x; ends[dir][1][lane] = (T)f.y; ends[dir][2][lane] = (T)f.z;
             ends[dir][3][lane] = (T)mm.x; ends[dir][4][lane] = (T)mm.y; ends[dir][5][lane] = (T)mm.z;
         }
@@ -806,15 +818,16 @@ void launch_step_mixed(const MixPtrs& s, bool fp64, int block, hipStream_t st) {
     const bool plain = !s.vE && !s.vphase && !s.tapeSums && !s.colCnt;
     const bool cached = s.nv <= kMixedCachedMax;
     if (fp64) {
-        if (s.haltTest) hipLaunchKernelGGL((k_step_mixed<double, true, false, false>), grid, dim3(block), 0, st, s);
-        else hipLaunchKernelGGL((k_step_mixed<double, false, false, false>), grid, dim3(block), 0, st, s);
+        if (s.haltTest) hipLaunchKernelGGL((k_step_mixed<double, true, false, false, true>), grid, dim3(block), 0, st, s);
+        else if (s.vphase) hipLaunchKernelGGL((k_step_mixed<double, false, false, false, false>), grid, dim3(block), 0, st, s);
+        else hipLaunchKernelGGL((k_step_mixed<double, false, false, false, true>), grid, dim3(block), 0, st, s);
     } else {
-        if (s.haltTest && cached) hipLaunchKernelGGL((k_step_mixed<float, true, false, true>), grid, dim3(block), 0, st, s);
-        else if (s.haltTest) hipLaunchKernelGGL((k_step_mixed<float, true, false, false>), grid, dim3(block), 0, st, s);
-        else if (plain && cached) hipLaunchKernelGGL((k_step_mixed<float, false, true, true>), grid, dim3(block), 0, st, s);
-        else if (plain) hipLaunchKernelGGL((k_step_mixed<float, false, true, false>), grid, dim3(block), 0, st, s);
-        else if (cached) hipLaunchKernelGGL((k_step_mixed<float, false, false, true>), grid, dim3(block), 0, st, s);
-        else hipLaunchKernelGGL((k_step_mixed<float, false, false, false>), grid, dim3(block), 0, st, s);
+        if (s.haltTest && cached) hipLaunchKernelGGL((k_step_mixed<float, true, false, true, true>), grid, dim3(block), 0, st, s);
+        else if (s.haltTest) hipLaunchKernelGGL((k_step_mixed<float, true, false, false, true>), grid, dim3(block), 0, st, s);
+        else if (plain && cached) hipLaunchKernelGGL((k_step_mixed<float, false, true, true, false>), grid, dim3(block), 0, st, s);
+        else if (plain) hipLaunchKernelGGL((k_step_mixed<float, false, true, false, false>), grid, dim3(block), 0, st, s);
+        else if (cached) hipLaunchKernelGGL((k_step_mixed<float, false, false, true, false>), grid, dim3(block), 0, st, s);
+        else hipLaunchKernelGGL((k_step_mixed<float, false, false, false, false>), grid, dim3(block), 0, st, s);
     }
 }
 
