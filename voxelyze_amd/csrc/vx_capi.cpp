@@ -235,7 +235,7 @@ API int vxg_launch_config(vxg_sim* h, int kernel, int* block, int* xcd, int* set
     const Sim::Tuner& t = s->tuner[kernel];
     if (block) *block = t.chosen.block;
     if (xcd) *xcd = t.chosen.xcd;
-    if (settled) *settled = t.settled ? 1 : 0;
+    if (settled) *settled = t.settled || s->endsSize(kernel) ? 1 : 0;
     return 1;
 }
 API int vxg_set_launch_config(vxg_sim* h, int kernel, int block, int xcd) {

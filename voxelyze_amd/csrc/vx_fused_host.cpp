@@ -84,7 +84,7 @@ bool Sim::stepFp64Fused(int nsteps) {
         nearbyStale = true;
     }
     if (!fusedFp64Buffers()) return false;
-    const bool ends = endsPath(3, kEndsMaxFp64);
+    const bool ends = endsPath(3);
     psInStep = ends && poisson;
     FusedPtrs fp{};
     fp.nv = nv();

@@ -170,7 +170,7 @@ bool Sim::stepMixed(int nsteps, MixTape* tape) {
     mp.actFreq = actFreq;
     mp.vE = modOn ? (const float*)bvE.p : nullptr;
     /* a launch without contacts, tape or timing is recorded as a graph and replayed */
-    const bool ends = endsPath(0, precision == 2 ? kEndsMaxFused64 : kEndsMaxMixed);
+    const bool ends = endsPath(0);
     const bool tune = !ends && tuning(0);
     const bool timed = profiling || tune;
     const bool graph = useGraphs && !collisions && !tape && !timed && nsteps > 1 && nsteps <= 2048;

@@ -1535,11 +1535,10 @@ bool Sim::tuning(int t) {
     return !tuner[t].settled;
 }
 
-bool Sim::endsPath(int t, int maxVoxels) {
+bool Sim::endsSize(int t) const { return tuner[t].nv == nv() && !tuner[t].pinned && nv() <= endsMax(t); }
+bool Sim::endsPath(int t) {
     if (tuner[t].nv != nv()) tuner[t].reset(nv());
-    if (tuner[t].pinned || nv() > maxVoxels) return false;
-    tuner[t].settled = true; /* nothing to choose */
-    return true;
+    return endsSize(t);
 }
 
 /* ------------------------------------------------------------ step graphs */

@@ -280,11 +280,13 @@ struct Sim {
     bool autotune = true;
     bool tuning(int t);
     /* step kernel t with its link directions split over waves (vx_fused.hip): models of at most
-       maxVoxels, unless a launch configuration was pinned.  The FP64 step up to 294,912 voxels,
+       endsMax voxels, unless a launch configuration was pinned.  The FP64 step up to 294,912 voxels,
        where the two copies of the state outgrow the 256 MB Infinity Cache and the kernel with the
        fewest bytes in flight per voxel wins (us per step, k_step_fp64 against k_step_fp64_ends:
        282,309 voxels 68.2 / 63.4, 332,769 voxels 77.5 / 82.2, 943,896 voxels 226 / 251). */
-    bool endsPath(int t, int maxVoxels);
+    bool endsPath(int t);
+    bool endsSize(int t) const; /* the last step of kernel t was in that form, with no launch shape to choose */
+    int endsMax(int t) const { return t == 3 ? kEndsMaxFp64 : t == 0 ? (precision == 2 ? kEndsMaxFused64 : kEndsMaxMixed) : -1; }
     static constexpr int kEndsMaxFp64 = 294912;
     /* the mixed step up to where its kernel with a voxel per lane fills the chip (us per step of
        k_step_mixed / k_step_mixed_ends: 107,926 voxels 25.3 / 23.2, 241,914: 45.9 / 45.7, 324,084:
