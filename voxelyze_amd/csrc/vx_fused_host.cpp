@@ -31,6 +31,7 @@ uint64_t graph_key(const void* args, size_t n, int path, int nsteps, int flags);
 /* the "out" half of the voxel and link state, and the saved link state of diverged robots */
 bool Sim::fusedFp64Buffers() {
     const size_t vc = (size_t)std::max(nv(), 1), sc = 3 * vc;
+    const bool fresh = !blfAlt.p || blfAlt.bytes < (size_t)LF_COUNT * sc * 4;
     if (!bvdAlt.ensure((size_t)VD_COUNT * vc * 8) || !bvflAlt.ensure(vc * 4) || !bvtempAlt.ensure(vc * 4) ||
         (poisson && !bvpsAlt.ensure(3 * vc * 4)) || !bldAlt.ensure((size_t)LDEV_COUNT * sc * 8) ||
         !blfAlt.ensure((size_t)LF_COUNT * sc * 4) || !blflAlt.ensure(sc * 4) || !bldSide.ensure((size_t)LDEV_COUNT * sc * 8) ||
@@ -38,6 +39,15 @@ bool Sim::fusedFp64Buffers() {
         err = "device allocation failed";
         return false;
     }
+    return !fresh || mirrorTransverse();
+}
+
+/* The transverse info in both halves of the link state: the steps write it only under a Poisson's ratio, and a
+   checkpoint saved before one was set is restored after */
+bool Sim::mirrorTransverse() {
+    const size_t S = (size_t)3 * nv();
+    if (blfAlt.p && blfAlt.bytes >= (size_t)LF_COUNT * S * 4)
+        HIPCHK(hipMemcpyAsync((float*)blfAlt.p + LTAREA * S, dp.lf + LTAREA * S, 2 * S * 4, hipMemcpyDeviceToDevice, stream));
     return true;
 }
 

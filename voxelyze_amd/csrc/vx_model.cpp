@@ -1152,6 +1152,7 @@ bool Sim::syncUp() {
             stageF.push_back(to_slots(lf[c], slotOf, S, 0.0f));
             if (S) HIPCHK(hipMemcpyAsync(dp.lf + c * S, stageF.back().data(), S * 4, hipMemcpyHostToDevice, stream));
         }
+        if (!mirrorTransverse()) return false;
         std::vector<uint32_t> fl = to_slots(lflags, slotOf, S, 0u);
         HIPCHK(up(dp.lflags, fl, stream));
         stageF.push_back(to_slots(lratio, slotOf, S, 1.0f));

@@ -320,6 +320,7 @@ struct Sim {
     bool fp64Split = false;
     DevBuf bldAlt, blfAlt, blflAlt, bldSide, blfSide, blflSide;
     bool fusedFp64Buffers();
+    bool mirrorTransverse();
     void swapFp64Buffers();
     void swapTemps();   /* the halves of the temperatures (actuated FP64 steps) */
     void swapPoisson(); /* the halves of the Poisson strains (steps that form the next one's) */
